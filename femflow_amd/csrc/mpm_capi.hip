@@ -65,23 +65,50 @@ int32_t mpm_device_count(void) {
   return n;
 }
 
-int32_t mpm_p2g(void* stream, const mpm_params* prm, const mpm_particles* p, int32_t kind_override,
-                double hardening, const mpm_material* materials, int32_t nmat, void* grid_v,
-                void* grid_m, int64_t* oob_count) {
+static int p2g_call(void* stream, const mpm_params* prm, const mpm_particles* p, int32_t kind_override,
+                    double hardening, const mpm_material* materials, int32_t nmat, void* grid_v, void* grid_m,
+                    int64_t* oob_count, void* work, int64_t work_bytes, const char* fn) {
   int rc;
-  if ((rc = check_params(prm, "mpm_p2g")) || (rc = check_particles(p, "mpm_p2g", true))) return rc;
+  if ((rc = check_params(prm, fn)) || (rc = check_particles(p, fn, true))) return rc;
   if (!grid_v || !grid_m) {
-    set_error("mpm_p2g: null grid");
+    set_error(std::string(fn) + ": null grid");
     return MPM_ERR_ARG;
   }
   if (kind_override < 0 && (nmat <= 0 || nmat > MPM_PHASE_MAX_MATERIALS || !materials)) {
-    set_error("mpm_p2g: per-particle materials need 1 <= nmat <= 16 and a table");
+    set_error(std::string(fn) + ": per-particle materials need 1 <= nmat <= 16 and a table");
     return MPM_ERR_ARG;
   }
+  const size_t need = mpm::phase_p2g_workspace_bytes(prm, p->n);
+  if (need == 0 || work_bytes < (int64_t)need) work = nullptr;
   mpm::phase_p2g((hipStream_t)stream, prm, p, kind_override, hardening, materials, nmat, grid_v,
-                 grid_m, (unsigned long long*)oob_count);
+                 grid_m, (unsigned long long*)oob_count, work);
   CHECK_HIP(hipGetLastError());
   return MPM_OK;
+}
+
+int32_t mpm_p2g(void* stream, const mpm_params* prm, const mpm_particles* p, int32_t kind_override,
+                double hardening, const mpm_material* materials, int32_t nmat, void* grid_v,
+                void* grid_m, int64_t* oob_count) {
+  return p2g_call(stream, prm, p, kind_override, hardening, materials, nmat, grid_v, grid_m, oob_count, nullptr, 0,
+                  "mpm_p2g");
+}
+
+int32_t mpm_p2g_workspace_bytes(const mpm_params* prm, int64_t n, int64_t* bytes) {
+  int rc;
+  if ((rc = check_params(prm, "mpm_p2g_workspace_bytes"))) return rc;
+  if (!bytes || n < 0) {
+    set_error("mpm_p2g_workspace_bytes: null output or n < 0");
+    return MPM_ERR_ARG;
+  }
+  *bytes = (int64_t)mpm::phase_p2g_workspace_bytes(prm, n);
+  return MPM_OK;
+}
+
+int32_t mpm_p2g_ws(void* stream, const mpm_params* prm, const mpm_particles* p, int32_t kind_override,
+                   double hardening, const mpm_material* materials, int32_t nmat, void* grid_v, void* grid_m,
+                   int64_t* oob_count, void* work, int64_t work_bytes) {
+  return p2g_call(stream, prm, p, kind_override, hardening, materials, nmat, grid_v, grid_m, oob_count, work,
+                  work_bytes, "mpm_p2g_ws");
 }
 
 static int check_dense(const mpm_params* prm, const mpm_particles* p, const void* work, const char* fn) {

@@ -1,0 +1,186 @@
+// Particle-to-node sums without one atomic per particle and node.
+//
+// A workgroup takes CELLSUM_THREADS consecutive particles of a cell-ordered
+// list.  Each thread writes its particle's B-spline weights and linear terms
+// to an LDS table; each wave then walks the runs of equal stencil bases among
+// its 64 particles with one lane per (node, channel) output, so a run of m
+// particles ends in one add per output instead of m.  The adds go to an LDS
+// arena over the workgroup's stencil bounding box, which is added to memory
+// once, one device atomic per nonzero value.  Device-scope float atomics run
+// at about 1e10 per second over the whole chip here (one L2 per XCD, so they
+// are served behind it), which is what a per-particle scatter is bound by.
+//
+// Value of channel c at stencil node (i, j[, k]) of a particle:
+//   w_i w_j [w_k] (q[c] + A[c][0] i + A[c][1] j [+ A[c][2] k]).
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <climits>
+
+#include "mpm_math.h"
+
+namespace mpm {
+
+constexpr int CELLSUM_THREADS = 256;
+
+template <typename T, int DIM, int NCH> struct CellSum {
+  static constexpr int NODES = DIM == 3 ? 27 : 9;
+  static constexpr int ROW = DIM == 3 ? 4 : 3;  // q, A[0..DIM-1] of a channel
+  // per-particle table entry: NCH rows, then DIM x 3 weights, padded to 16
+  // bytes, so that a 3D row is read 16 bytes at a time
+  static constexpr int PAD = 16 / (int)sizeof(T);
+  static constexpr int ENTRY = (NCH * ROW + 3 * DIM + PAD - 1) / PAD * PAD;
+  typedef T Row3 __attribute__((ext_vector_type(4), aligned(16)));
+  // outputs per lane: 3D uses 54 lanes with up to two channels each, 2D two
+  // groups of 27 lanes that take alternate particles of a run
+  static constexpr int GROUP = DIM == 3 ? 1 : 2;
+  static constexpr int ARENA = sizeof(T) == 8 ? 576 : 1024;  // nodes
+
+  struct alignas(16) Shared {
+    T table[CELLSUM_THREADS * ENTRY];
+    T arena[ARENA * NCH];
+    int box_w[CELLSUM_THREADS / 64][2 * DIM];
+    int box[2 * DIM];  // low corner, extent (0: the box does not fit the arena)
+  };
+
+  // Bounding box of the workgroup's stencils (valid particles) and the
+  // cleared arena.  Every thread of the workgroup calls it; ends in a
+  // barrier, so the table may be written before it and read after it.
+  static __device__ __forceinline__ void prepare(Shared& sh, const int (&base)[DIM], bool valid) {
+    const int t = threadIdx.x;
+    int lo[DIM], hi[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+      lo[d] = valid ? base[d] : INT_MAX;
+      hi[d] = valid ? base[d] : INT_MIN;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        lo[d] = min(lo[d], __shfl_xor(lo[d], o));
+        hi[d] = max(hi[d], __shfl_xor(hi[d], o));
+      }
+      if ((t & 63) == 0) {
+        sh.box_w[t >> 6][d] = lo[d];
+        sh.box_w[t >> 6][DIM + d] = hi[d];
+      }
+    }
+    __syncthreads();
+    if (t == 0) {
+      int64_t vol = 1;
+      int l[DIM], e[DIM];
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) {
+        int a = INT_MAX, b = INT_MIN;
+        for (int w = 0; w < CELLSUM_THREADS / 64; ++w) {
+          a = min(a, sh.box_w[w][d]);
+          b = max(b, sh.box_w[w][DIM + d]);
+        }
+        l[d] = a;
+        e[d] = a <= b ? b - a + 3 : 0;
+        vol *= e[d];
+      }
+      const bool fits = vol > 0 && vol <= ARENA;
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) {
+        sh.box[d] = l[d];
+        sh.box[DIM + d] = fits ? e[d] : 0;
+      }
+    }
+    __syncthreads();
+    const int n = volume(sh) * NCH;
+    for (int e = t; e < n; e += CELLSUM_THREADS) sh.arena[e] = T(0);
+    __syncthreads();
+  }
+
+  static __device__ __forceinline__ int volume(const Shared& sh) {
+    int v = 1;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) v *= sh.box[DIM + d];
+    return v;
+  }
+
+  // Sums every run of this wave's particles.  direct(node offsets from the
+  // run's base, channel, value, base) adds to memory where the box does not
+  // fit the arena.  The table entries of the wave were written by its own
+  // lanes; prepare()'s barriers order them.
+  template <typename Add>
+  static __device__ __forceinline__ void sum_runs(Shared& sh, const int (&base)[DIM], bool valid, Add direct) {
+    const int t = threadIdx.x, lane = t & 63;
+    bool head = lane == 0;
+    {
+      const int pv = __shfl_up(valid ? 1 : 0, 1);
+      head = head || (pv != 0) != valid;
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) head = head || __shfl_up(base[d], 1) != base[d];
+    }
+    unsigned long long heads = __ballot(head);
+    const unsigned long long vmask = __ballot(valid);
+    constexpr int OUT = DIM == 3 ? 27 : NODES * NCH;
+    const int sub = lane / OUT, o = lane - sub * OUT;  // sub 2: idle lanes
+    const int node = DIM == 3 ? o : o % NODES;
+    const int i = DIM == 3 ? node / 9 : node / 3, j = DIM == 3 ? (node / 3) % 3 : node % 3, k = node % 3;
+    const int c0 = DIM == 3 ? 2 * sub : o / NODES;
+    const bool on0 = lane < 2 * OUT && c0 < NCH, on1 = DIM == 3 && lane < OUT * 2 && c0 + 1 < NCH;
+    const T fi = (T)i, fj = (T)j, fk = (T)k;
+    const int r0 = (on0 ? c0 : 0) * ROW, r1 = (on1 ? c0 + 1 : 0) * ROW;
+    const int wi = NCH * ROW + i, wj = NCH * ROW + 3 + j, wk = NCH * ROW + (DIM == 3 ? 6 + k : 0);
+    const bool arena = sh.box[DIM] > 0;
+    while (heads) {
+      const int s = __builtin_ctzll(heads);
+      heads &= heads - 1;
+      const int e = heads ? __builtin_ctzll(heads) : 64;
+      if (!((vmask >> s) & 1ull)) continue;
+      T a0 = T(0), a1 = T(0);
+      const T* tab = sh.table + ((t & ~63) + s + (DIM == 2 ? sub : 0)) * ENTRY;
+#pragma unroll 2
+      for (int p = s + (DIM == 2 ? sub : 0); p < e; p += GROUP, tab += GROUP * ENTRY) {
+        T w = tab[wi] * tab[wj];
+        if constexpr (DIM == 3) {
+          w *= tab[wk];
+          const Row3 q0 = *reinterpret_cast<const Row3*>(tab + r0), q1 = *reinterpret_cast<const Row3*>(tab + r1);
+          a0 += w * (q0.x + q0.y * fi + q0.z * fj + q0.w * fk);
+          a1 += w * (q1.x + q1.y * fi + q1.z * fj + q1.w * fk);
+        } else {
+          a0 += w * (tab[r0] + tab[r0 + 1] * fi + tab[r0 + 2] * fj);
+        }
+      }
+      int b[DIM];
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) b[d] = __shfl(base[d], s);
+      if (arena) {
+        int at = (b[0] + i - sh.box[0]) * sh.box[DIM + 1] + (b[1] + j - sh.box[1]);
+        if constexpr (DIM == 3) at = at * sh.box[DIM + 2] + (b[2] + k - sh.box[2]);
+        if (on0) atomicAdd(&sh.arena[at * NCH + c0], a0);
+        if (on1) atomicAdd(&sh.arena[at * NCH + c0 + 1], a1);
+      } else {
+        b[0] += i;
+        b[1] += j;
+        if constexpr (DIM == 3) b[2] += k;
+        if (on0) direct(b, c0, a0);
+        if (on1) direct(b, c0 + 1, a1);
+      }
+    }
+  }
+
+  // After every wave's sum_runs: the arena's nonzero values to memory.
+  template <typename Add> static __device__ __forceinline__ void flush(Shared& sh, Add add) {
+    __syncthreads();
+    const int n = volume(sh) * NCH;
+    for (int e = threadIdx.x; e < n; e += CELLSUM_THREADS) {
+      const T v = sh.arena[e];
+      if (v != T(0)) {
+        const int c = e % NCH;
+        int sl = e / NCH;
+        int b[DIM];
+#pragma unroll
+        for (int d = DIM - 1; d > 0; --d) {
+          b[d] = sh.box[d] + sl % sh.box[DIM + d];
+          sl /= sh.box[DIM + d];
+        }
+        b[0] = sh.box[0] + sl;
+        add(b, c, v);
+      }
+    }
+  }
+};
+
+}  // namespace mpm

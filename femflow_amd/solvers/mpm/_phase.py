@@ -124,8 +124,12 @@ def run_p2g(sp, prm, kind_override, hardening, grid_velocity, grid_mass, materia
     oob = torch.zeros(1, dtype=torch.int64, device=sp.device)
     mats, nmat = materials_array(materials)
     p = sp.struct()
-    _lib.check(L.mpm_p2g(stream_ptr(sp.device), ct.byref(prm), ct.byref(p), int(kind_override),
-                         float(hardening), mats, nmat, gv.ptr, gm.ptr, oob.data_ptr()), "p2g")
+    nbytes = ct.c_int64()
+    _lib.check(L.mpm_p2g_workspace_bytes(ct.byref(prm), sp.n, ct.byref(nbytes)), "p2g")
+    work = torch.empty(nbytes.value, dtype=torch.uint8, device=sp.device) if nbytes.value else None
+    _lib.check(L.mpm_p2g_ws(stream_ptr(sp.device), ct.byref(prm), ct.byref(p), int(kind_override),
+                            float(hardening), mats, nmat, gv.ptr, gm.ptr, oob.data_ptr(),
+                            None if work is None else work.data_ptr(), nbytes.value), "p2g")
     n_oob = int(oob.item())
     gv.commit()
     gm.commit()

@@ -113,6 +113,17 @@ int32_t mpm_p2g(void* stream, const mpm_params* prm, const mpm_particles* p,
                 int32_t kind_override, double hardening, const mpm_material* materials,
                 int32_t nmat, void* grid_v, void* grid_m, int64_t* oob_count);
 
+/* mpm_p2g with scratch memory (device, 8-byte aligned), which lets it sort
+ * the particles by cell and sum each cell's particles before they reach the
+ * grid.  mpm_p2g_workspace_bytes gives the size for n particles; 0 where the
+ * scatter needs none (few particles, key space beyond 32 bits).  With less
+ * (or NULL) the call runs like mpm_p2g.  The scratch memory may be reused
+ * once the call's work on the stream is done. */
+int32_t mpm_p2g_workspace_bytes(const mpm_params* prm, int64_t n, int64_t* bytes);
+int32_t mpm_p2g_ws(void* stream, const mpm_params* prm, const mpm_particles* p, int32_t kind_override,
+                   double hardening, const mpm_material* materials, int32_t nmat, void* grid_v, void* grid_m,
+                   int64_t* oob_count, void* work, int64_t work_bytes);
+
 /* Replaces three_d.grid_op (three_d/grid_op.py:5-47) and two_d.grid_op
  * (two_d/grid_op.py:5-24). In place on grid_v. */
 int32_t mpm_grid_op(void* stream, const mpm_params* prm, int32_t dtype, void* grid_v,
