@@ -31,7 +31,7 @@ EXPORTS = (
     "mpm_adjoint_step_grids",
     "mpm_ctx_set_corrector", "mpm_corrector_sample", "mpm_grid_velocity",
     "mpm_collide_planes", "mpm_ctx_set_planes",
-    "mpm_mlp_sizes", "mpm_mlp_pack", "mpm_mlp_forward", "mpm_mlp_loss", "mpm_mlp_backward", "mpm_mlp_adam",
+    "mpm_mlp_sizes", "mpm_mlp_pack", "mpm_mlp_forward", "mpm_mlp_loss", "mpm_mlp_backward", "mpm_mlp_backward_workspace_bytes", "mpm_mlp_backward_ws", "mpm_mlp_adam",
 )
 
 
@@ -128,6 +128,8 @@ def load():
             "mpm_mlp_forward": ([vp, vp, vp, vp, i64, vp, vp, vp], i32),
             "mpm_mlp_loss": ([vp, vp, vp, vp, i64, ct.c_float, vp, vp], i32),
             "mpm_mlp_backward": ([vp, vp, vp, i64, vp, vp, vp, vp, vp, vp], i32),
+            "mpm_mlp_backward_workspace_bytes": ([i64, ct.POINTER(i64)], i32),
+            "mpm_mlp_backward_ws": ([vp, vp, vp, i64, vp, vp, vp, vp, vp, vp, vp, i64], i32),
             "mpm_mlp_adam": ([vp, vp, vp, vp, vp, i64, ct.c_float, ct.c_float, ct.c_float, ct.c_float, i32], i32),
         }
         for name, (args, res) in sig.items():

@@ -76,6 +76,9 @@ class CorrectorMLP:
             self.dH2 = torch.empty((cap, HIDDEN), dtype=torch.bfloat16, device=d)
             self.Y = torch.empty((cap, OUT_PAD), dtype=torch.float32, device=d)
             self.dY = torch.empty((cap, DY_PAD), dtype=torch.bfloat16, device=d)
+            nbytes = ct.c_int64()
+            _lib.check(self.L.mpm_mlp_backward_workspace_bytes(cap, ct.byref(nbytes)), "mpm_mlp_backward")
+            self.parts = torch.empty(nbytes.value // 4, dtype=torch.float32, device=d)
             self._ws_rows = cap
 
     @staticmethod
@@ -111,9 +114,10 @@ class CorrectorMLP:
                                        rows, 1.0 / max(norm, 1e-30), self.dY.data_ptr(), loss.data_ptr()),
                    "mpm_mlp_loss")
         self.grads.zero_()
-        _lib.check(self.L.mpm_mlp_backward(st, self.packed.data_ptr(), X.data_ptr(), rows, self.H1.data_ptr(),
-                                           self.H2.data_ptr(), self.dY.data_ptr(), self.dH2.data_ptr(),
-                                           self.dH1.data_ptr(), self.grads.data_ptr()), "mpm_mlp_backward")
+        _lib.check(self.L.mpm_mlp_backward_ws(st, self.packed.data_ptr(), X.data_ptr(), rows, self.H1.data_ptr(),
+                                              self.H2.data_ptr(), self.dY.data_ptr(), self.dH2.data_ptr(),
+                                              self.dH1.data_ptr(), self.grads.data_ptr(), self.parts.data_ptr(),
+                                              4 * self.parts.numel()), "mpm_mlp_backward")
         return loss
 
     def adam_step(self, lr: float = 1e-3, beta1: float = 0.9, beta2: float = 0.999, eps: float = 1e-8):

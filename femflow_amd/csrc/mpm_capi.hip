@@ -247,11 +247,27 @@ int32_t mpm_mlp_loss(void* stream, const float* Y, const float* T, const float* 
 int32_t mpm_mlp_backward(void* stream, const uint16_t* packed, const uint16_t* X, int64_t rows,
                          const uint16_t* H1, const uint16_t* H2, const uint16_t* dY, uint16_t* dH2,
                          uint16_t* dH1, float* grads) {
+  return mpm_mlp_backward_ws(stream, packed, X, rows, H1, H2, dY, dH2, dH1, grads, nullptr, 0);
+}
+
+int32_t mpm_mlp_backward_workspace_bytes(int64_t rows, int64_t* bytes) {
+  if (rows < 0 || !bytes) {
+    set_error("mpm_mlp_backward_workspace_bytes: bad argument");
+    return MPM_ERR_ARG;
+  }
+  *bytes = (int64_t)mpm::mlp_backward_workspace_bytes(rows);
+  return MPM_OK;
+}
+
+int32_t mpm_mlp_backward_ws(void* stream, const uint16_t* packed, const uint16_t* X, int64_t rows,
+                            const uint16_t* H1, const uint16_t* H2, const uint16_t* dY, uint16_t* dH2,
+                            uint16_t* dH1, float* grads, void* work, int64_t work_bytes) {
   if (rows < 0 || (rows > 0 && (!packed || !X || !H1 || !H2 || !dY || !dH2 || !dH1 || !grads))) {
     set_error("mpm_mlp_backward: bad argument");
     return MPM_ERR_ARG;
   }
-  mpm::mlp_backward((hipStream_t)stream, packed, X, rows, H1, H2, dY, dH2, dH1, grads);
+  if (work_bytes < (int64_t)mpm::mlp_backward_workspace_bytes(rows)) work = nullptr;
+  mpm::mlp_backward((hipStream_t)stream, packed, X, rows, H1, H2, dY, dH2, dH1, grads, (float*)work);
   CHECK_HIP(hipGetLastError());
   return MPM_OK;
 }

@@ -325,6 +325,14 @@ int32_t mpm_mlp_loss(void* stream, const float* Y, const float* T, const float* 
 int32_t mpm_mlp_backward(void* stream, const uint16_t* packed, const uint16_t* X, int64_t rows,
                          const uint16_t* H1, const uint16_t* H2, const uint16_t* dY, uint16_t* dH2,
                          uint16_t* dH1, float* grads);
+/* mpm_mlp_backward with scratch memory (device, 4-byte aligned) of
+ * mpm_mlp_backward_workspace_bytes: the row splits' gradients are summed in
+ * a fixed order instead of by atomics.  With less (or NULL) the call runs
+ * like mpm_mlp_backward. */
+int32_t mpm_mlp_backward_workspace_bytes(int64_t rows, int64_t* bytes);
+int32_t mpm_mlp_backward_ws(void* stream, const uint16_t* packed, const uint16_t* X, int64_t rows,
+                            const uint16_t* H1, const uint16_t* H2, const uint16_t* dY, uint16_t* dH2,
+                            uint16_t* dH1, float* grads, void* work, int64_t work_bytes);
 /* One Adam step (FP32) on n parameters; step counts from 1. */
 int32_t mpm_mlp_adam(void* stream, float* params, const float* grads, float* m, float* v, int64_t n,
                      float lr, float beta1, float beta2, float eps, int32_t step);

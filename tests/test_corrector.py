@@ -316,3 +316,35 @@ def test_judge_falls_back_to_plain_substeps(gpu):
     assert st2["fallbacks"] == 0 and st2["big_steps_kept"] + 2 * st2["unhealthy"] == n_big, st2
     print("judge stats strict", st, "loose", st2, "loose error", CT.rel_position_error(out2["x"], ref["x"]),
           flush=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 31, 65, 257, 4129, 16_421])
+def test_mlp_gradients_at_row_edges(gpu, rows):
+    """Row counts around the 16-row waves, the 32-row reduction steps and the
+    row splits (16,421: all 64 splits, a short last one), with and without
+    scratch memory, against the NumPy restatement (the bars of the test
+    above) and against each other (FP32 sums in two orders)."""
+    import ctypes as ct
+
+    import torch
+
+    from femflow_amd import _lib
+    from femflow_amd.corrector import CorrectorMLP, to_bf16_features
+
+    X, T, w = _data(rows, rows)
+    p = _params(6)
+    net = CorrectorMLP(device=gpu, params=torch.from_numpy(p))
+    Xg = to_bf16_features(X, gpu)
+    net.loss_grads(Xg, torch.tensor(T, dtype=torch.float32), torch.tensor(w, dtype=torch.float32))
+    g = net.grads.double().cpu().numpy()
+    _, gref, _ = M.loss_and_grads(p.astype(np.float64), X, T, w)
+    assert np.linalg.norm(g - gref) <= 1e-3 * np.linalg.norm(gref)
+    b = ct.c_int64()
+    _lib.check(_lib.load().mpm_mlp_backward_workspace_bytes(rows, ct.byref(b)))
+    assert 4 * p.size <= b.value <= 4 * net.parts.numel()
+    atomic = torch.zeros_like(net.grads)
+    _lib.check(_lib.load().mpm_mlp_backward(
+        torch.cuda.current_stream().cuda_stream, net.packed.data_ptr(), Xg.data_ptr(), rows, net.H1.data_ptr(),
+        net.H2.data_ptr(), net.dY.data_ptr(), net.dH2.data_ptr(), net.dH1.data_ptr(), atomic.data_ptr()))
+    assert float((atomic - net.grads).norm()) <= 1e-5 * float(net.grads.norm())
