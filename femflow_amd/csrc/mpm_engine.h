@@ -17,15 +17,16 @@ void set_error(const std::string& msg);
 // A captured segment fixes the particle count (launch grids, sort sizes),
 // the segment length, whether it rebins first, which state buffer is current,
 // the sums destination, and whether it continues the run's previous segment
-// (cont) and ends the run (fin); any of them changing needs another graph.
+// (cont) and ends the run (fin), and whether it reads uploaded records; any
+// of them changing needs another graph.
 struct GraphKey {
   int64_t n;
   int len, parity, bin;
   uintptr_t sums;
-  int nsteps, cont, fin;
+  int nsteps, cont, fin, records;
   bool operator<(const GraphKey& o) const {
-    return std::tie(n, len, parity, bin, sums, nsteps, cont, fin) <
-           std::tie(o.n, o.len, o.parity, o.bin, o.sums, o.nsteps, o.cont, o.fin);
+    return std::tie(n, len, parity, bin, sums, nsteps, cont, fin, records) <
+           std::tie(o.n, o.len, o.parity, o.bin, o.sums, o.nsteps, o.cont, o.fin, o.records);
   }
 };
 // Captured graphs kept per context; beyond this the cache is emptied first.
@@ -83,6 +84,12 @@ struct Engine {
   std::vector<void*> allocs;
   EngineState st[2] = {};
   int cur = 0;
+  // The uploaded particles are still records (in st[0]'s memory except its x
+  // and attr, which hold them as ever, for the rebin's keys); the first rebin
+  // moves them into st[1].  tiled() does so without one, for calls that read the
+  // state before.
+  bool in_records = false;
+  float4* rec_mem[2] = {};  // the same memory as st[0], st[1] without x and attr
   SceneDev* d_scenes = nullptr;
   MatParams* d_mats = nullptr;
   int* d_block_scene = nullptr;
@@ -125,6 +132,7 @@ struct Engine {
   EngineArgs args(double* sums, int max_steps, int sel) const;
   int upload(const mpm_particles* p, const int32_t* scene_ids);
   int download(mpm_particles* p);
+  void tiled();
   // rebin; also starts the segment of len substeps (counters, sums index)
   void enqueue_bin(hipStream_t s, int len, int with_sums);
   void enqueue_segment(int len, bool bin, hipStream_t s, double* sums, int max_steps, float* frames,

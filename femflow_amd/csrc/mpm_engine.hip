@@ -304,6 +304,35 @@ __device__ __forceinline__ void storek(float* f, int64_t p, const float o[K]) {
   for (int d = 0; d < K; ++d) b[d * PTILE] = o[d];
 }
 
+__device__ __forceinline__ void load_record(const float4* __restrict__ rec, int64_t i, float x[3], float v[3],
+                                            float F[9], float C[9], float& Jp, float& mass, float& mu0, float& lam0,
+                                            uint32_t& attr) {
+  float r[REC_WORDS];
+#pragma unroll
+  for (int q = 0; q < REC_WORDS / 4; ++q) {
+    const float4 w = rec[i * (REC_WORDS / 4) + q];
+    r[4 * q] = w.x;
+    r[4 * q + 1] = w.y;
+    r[4 * q + 2] = w.z;
+    r[4 * q + 3] = w.w;
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    x[d] = r[REC_X + d];
+    v[d] = r[REC_V + d];
+  }
+#pragma unroll
+  for (int d = 0; d < 9; ++d) {
+    F[d] = r[REC_F + d];
+    C[d] = r[REC_C + d];
+  }
+  Jp = r[REC_JP];
+  mass = r[REC_MASS];
+  mu0 = r[REC_MU];
+  lam0 = r[REC_LAM];
+  attr = __float_as_uint(r[REC_ATTR]);
+}
+
 // --------------------------------------------------------- transfer kernel ----
 // One work item = one chunk of at most CHUNK binned particles of one 4x4x4-cell
 // block.  MODE 0: P2G only (right after binning).  MODE 1: fused G2P of this
@@ -537,16 +566,22 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
         // they are read before that (FP64-deferred particles, per-substep
         // state output) or kept (particles that left the grid).
         const int64_t pm = a.perm[p];
-        loadk<3>(a.src.x, pm, x);
-        loadk<9>(a.src.F, pm, F);
-        loadk<3>(a.src.v, pm, v);
-        loadk<9>(a.src.C, pm, C);
-        Jp = a.src.Jp[pm];
-        attr = a.src.attr[pm];
-        pmass = a.src.mass[pm];
-        pmu0 = a.src.mu0[pm];
-        plam0 = a.src.lam0[pm];
-        const uint32_t ord = a.src.order[pm];
+        uint32_t ord;
+        if (a.rec) {
+          load_record(a.rec, pm, x, v, F, C, Jp, pmass, pmu0, plam0, attr);
+          ord = (uint32_t)pm;
+        } else {
+          loadk<3>(a.src.x, pm, x);
+          loadk<9>(a.src.F, pm, F);
+          loadk<3>(a.src.v, pm, v);
+          loadk<9>(a.src.C, pm, C);
+          Jp = a.src.Jp[pm];
+          attr = a.src.attr[pm];
+          pmass = a.src.mass[pm];
+          pmu0 = a.src.mu0[pm];
+          plam0 = a.src.lam0[pm];
+          ord = a.src.order[pm];
+        }
         storek<3>(a.s.x, p, x);
         storek<9>(a.s.F, p, F);
         if (a.store_vc) {
@@ -1294,54 +1329,224 @@ __global__ void fill_f64_kernel(double* p, int64_t n, double v) {
 }
 
 // ----------------------------------------------------------- upload/download ----
-__global__ void upload_kernel(EngineState s, int64_t n, const float* __restrict__ x,
-                              const float* __restrict__ v, const float* __restrict__ F,
-                              const float* __restrict__ C, const float* __restrict__ Jp,
-                              const float* __restrict__ mass, const float* __restrict__ mu0,
-                              const float* __restrict__ lam0, int mat_scalar,
-                              const int32_t* __restrict__ material, const int32_t* __restrict__ scene,
-                              int nscenes) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Both sides of these copies are cut into 64-particle pieces, one per wave,
+// and pass through LDS, so that a wave's loads and stores cover whole runs:
+// the caller's arrays hold a particle's K components side by side, the
+// engine's tiles hold 64 particles of one component side by side.  (A lane
+// per particle writes 64 places per instruction when the order is arbitrary;
+// a lane per value writes one run of up to 36 bytes per particle: 2^20
+// particles in arbitrary order 135 -> 116 us per download.)
+constexpr int UP_STRIDE = REC_WORDS + 4;  // 16-byte aligned rows, spread over the banks
+constexpr int DOWN_STRIDE = 25;
+
+// LDS rows[p][at + d] = src[K (first + p) + d], p < count.  FULL (count 64):
+// no bounds tests, which would put every load behind a lane mask and in
+// series with the one before.
+template <int K, bool FULL>
+__device__ __forceinline__ void rows_in(float* rows, int stride, int at, const float* __restrict__ src, int64_t first,
+                                        int count, int lane) {
+  float val[K];
+#pragma unroll
+  for (int it = 0; it < K; ++it) {
+    const int e = it * 64 + lane;
+    if (FULL || e < count * K) val[it] = src[first * K + e];
+  }
+#pragma unroll
+  for (int it = 0; it < K; ++it) {
+    const int e = it * 64 + lane;
+    if (FULL || e < count * K) rows[(e / K) * stride + at + e % K] = val[it];
+  }
+}
+
+struct UploadArgs {
+  const float *x, *v, *F, *C, *Jp, *mass, *mu0, *lam0;
+  const int32_t *material, *scene;
+  int mat_scalar, nscenes;
+};
+
+template <bool FULL>
+__device__ __forceinline__ void upload_piece(const EngineState& s, float4* __restrict__ rec, const UploadArgs& u,
+                                             float* rows, int64_t first, int count, int lane) {
+  rows_in<3, FULL>(rows, UP_STRIDE, REC_X, u.x, first, count, lane);
+  rows_in<3, FULL>(rows, UP_STRIDE, REC_V, u.v, first, count, lane);
+  rows_in<9, FULL>(rows, UP_STRIDE, REC_F, u.F, first, count, lane);
+  rows_in<9, FULL>(rows, UP_STRIDE, REC_C, u.C, first, count, lane);
+  if (FULL || lane < count) {
+    const int64_t i = first + lane, mi = u.mat_scalar ? 0 : i;
+    float* row = rows + lane * UP_STRIDE;
+    const uint32_t mat = u.material ? (uint32_t)(u.material[i] & 255) : 0u;
+    int sc = u.scene ? u.scene[i] : 0;
+    const float jp = u.Jp[i], m = u.mass[mi], mu = u.mu0[mi], la = u.lam0[mi];
+    sc = sc < 0 ? 0 : (sc >= u.nscenes ? u.nscenes - 1 : sc);
+    const uint32_t attr = mat | ((uint32_t)sc << 8);
+    row[REC_JP] = jp;
+    row[REC_MASS] = m;
+    row[REC_MU] = mu;
+    row[REC_LAM] = la;
+    row[REC_ATTR] = __uint_as_float(attr);
+#pragma unroll
+    for (int d = REC_ATTR + 1; d < REC_WORDS; ++d) row[d] = 0.f;
+    s.attr[i] = attr;
+  }
+  // the piece's rows belong to this wave, whose LDS accesses are in order
+  __builtin_amdgcn_wave_barrier();
+  if (FULL || lane < count) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) s.x[tix(first + lane, 3, d)] = rows[lane * UP_STRIDE + REC_X + d];
+  }
+#pragma unroll
+  for (int it = 0; it < REC_WORDS / 4; ++it) {
+    const int e = it * 64 + lane, p = e / (REC_WORDS / 4), q = e % (REC_WORDS / 4);
+    if (FULL || p < count)
+      rec[first * (REC_WORDS / 4) + e] = *reinterpret_cast<const float4*>(rows + p * UP_STRIDE + 4 * q);
+  }
+}
+
+__global__ __launch_bounds__(256) void upload_kernel(EngineState s, float4* __restrict__ rec, int64_t n, UploadArgs u) {
+  __shared__ __align__(16) float rows_s[4][64 * UP_STRIDE];
+  const int lane = threadIdx.x & 63;
+  float* rows = rows_s[threadIdx.x >> 6];
+  const int64_t first = (int64_t)blockIdx.x * 256 + (threadIdx.x & ~63);
+  if (first + 64 <= n) upload_piece<true>(s, rec, u, rows, first, 64, lane);
+  else if (first < n) upload_piece<false>(s, rec, u, rows, first, (int)(n - first), lane);
+}
+
+// Records to tiles, in the caller's order.
+__global__ __launch_bounds__(256) void unpack_kernel(EngineState s, const float4* __restrict__ rec, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    s.x[tix(i, 3, d)] = x[3 * i + d];
-    s.v[tix(i, 3, d)] = v[3 * i + d];
-  }
-#pragma unroll
-  for (int d = 0; d < 9; ++d) {
-    s.F[tix(i, 9, d)] = F[9 * i + d];
-    s.C[tix(i, 9, d)] = C[9 * i + d];
-  }
-  s.Jp[i] = Jp[i];
-  const int64_t mi = mat_scalar ? 0 : i;
-  s.mass[i] = mass[mi];
-  s.mu0[i] = mu0[mi];
-  s.lam0[i] = lam0[mi];
-  const uint32_t mat = material ? (uint32_t)(material[i] & 255) : 0u;
-  int sc_i = scene ? scene[i] : 0;
-  sc_i = sc_i < 0 ? 0 : (sc_i >= nscenes ? nscenes - 1 : sc_i);
-  const uint32_t sc = (uint32_t)sc_i;
-  s.attr[i] = mat | (sc << 8);
+  float x[3], v[3], F[9], C[9];
+  load_record(rec, i, x, v, F, C, s.Jp[i], s.mass[i], s.mu0[i], s.lam0[i], s.attr[i]);
+  storek<3>(s.x, i, x);
+  storek<3>(s.v, i, v);
+  storek<9>(s.F, i, F);
+  storek<9>(s.C, i, C);
   s.order[i] = (uint32_t)i;
 }
 
-__global__ void download_kernel(EngineState s, int64_t n, float* __restrict__ x, float* __restrict__ v,
-                                float* __restrict__ F, float* __restrict__ C, float* __restrict__ Jp) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int64_t o = s.order[i];
+// dst[K order[p] + d] = rows[p][at + d]
+template <int K>
+__device__ __forceinline__ void rows_out(const float* rows, int stride, int at, const uint32_t* order,
+                                         float* __restrict__ dst, int count, int lane) {
 #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    x[3 * o + d] = s.x[tix(i, 3, d)];
-    v[3 * o + d] = s.v[tix(i, 3, d)];
+  for (int it = 0; it < K; ++it) {
+    const int e = it * 64 + lane, p = e / K;
+    if (p < count) dst[(int64_t)order[p] * K + e % K] = rows[p * stride + at + e % K];
+  }
+}
+
+__global__ __launch_bounds__(256) void download_kernel(EngineState s, int64_t n, float* __restrict__ x,
+                                                       float* __restrict__ v, float* __restrict__ F,
+                                                       float* __restrict__ C, float* __restrict__ Jp) {
+  __shared__ float rows_s[4][64 * DOWN_STRIDE];
+  __shared__ uint32_t order_s[4][64];
+  const int lane = threadIdx.x & 63;
+  float* rows = rows_s[threadIdx.x >> 6];
+  uint32_t* order = order_s[threadIdx.x >> 6];
+  const int64_t first = (int64_t)blockIdx.x * 256 + (threadIdx.x & ~63);
+  const int count = first >= n ? 0 : (n - first < 64 ? (int)(n - first) : 64);
+  if (lane < count) {
+    const int64_t i = first + lane;
+    float* row = rows + lane * DOWN_STRIDE;
+    float c[25];
+    loadk<3>(s.x, i, c);
+    loadk<3>(s.v, i, c + 3);
+    loadk<9>(s.F, i, c + 6);
+    loadk<9>(s.C, i, c + 15);
+    c[24] = s.Jp[i];
+    const uint32_t o = s.order[i];
+#pragma unroll
+    for (int d = 0; d < 24; ++d) row[d] = c[d];
+    order[lane] = o;
+    Jp[o] = c[24];
+  }
+  __builtin_amdgcn_wave_barrier();
+  rows_out<3>(rows, DOWN_STRIDE, 0, order, x, count, lane);
+  rows_out<3>(rows, DOWN_STRIDE, 3, order, v, count, lane);
+  rows_out<9>(rows, DOWN_STRIDE, 6, order, F, count, lane);
+  rows_out<9>(rows, DOWN_STRIDE, 15, order, C, count, lane);
+}
+
+// The same in two passes, for states larger than the caches: the particles
+// go to 128-byte records at their caller indices first (whole lines, where
+// download_kernel's runs of 12 and 36 bytes would each be a partial line on
+// its way to memory), and the records are then split into the caller's
+// arrays in sequence.
+__global__ __launch_bounds__(256) void pack_kernel(EngineState s, int64_t n, float4* __restrict__ rec) {
+  __shared__ __align__(16) float rows_s[4][64 * UP_STRIDE];
+  __shared__ uint32_t order_s[4][64];
+  const int lane = threadIdx.x & 63;
+  float* rows = rows_s[threadIdx.x >> 6];
+  uint32_t* order = order_s[threadIdx.x >> 6];
+  const int64_t first = (int64_t)blockIdx.x * 256 + (threadIdx.x & ~63);
+  const int count = first >= n ? 0 : (n - first < 64 ? (int)(n - first) : 64);
+  if (lane < count) {
+    const int64_t i = first + lane;
+    float* row = rows + lane * UP_STRIDE;
+    float c[25];
+    loadk<3>(s.x, i, c);
+    loadk<3>(s.v, i, c + 3);
+    loadk<9>(s.F, i, c + 6);
+    loadk<9>(s.C, i, c + 15);
+    c[24] = s.Jp[i];
+    order[lane] = s.order[i];
+#pragma unroll
+    for (int d = 0; d < 25; ++d) row[d] = c[d];
+#pragma unroll
+    for (int d = 25; d < REC_WORDS; ++d) row[d] = 0.f;
+  }
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int it = 0; it < REC_WORDS / 4; ++it) {
+    const int e = it * 64 + lane, p = e / (REC_WORDS / 4), q = e % (REC_WORDS / 4);
+    if (p < count)
+      rec[(int64_t)order[p] * (REC_WORDS / 4) + q] = *reinterpret_cast<const float4*>(rows + p * UP_STRIDE + 4 * q);
+  }
+}
+
+template <int K, bool FULL>
+__device__ __forceinline__ void rows_split(const float* rows, int at, float* __restrict__ dst, int64_t first, int count,
+                                           int lane) {
+#pragma unroll
+  for (int it = 0; it < K; ++it) {
+    const int e = it * 64 + lane;
+    if (FULL || e < count * K) dst[first * K + e] = rows[(e / K) * UP_STRIDE + at + e % K];
+  }
+}
+
+__global__ __launch_bounds__(256) void split_kernel(const float4* __restrict__ rec, int64_t n, float* __restrict__ x,
+                                                    float* __restrict__ v, float* __restrict__ F,
+                                                    float* __restrict__ C, float* __restrict__ Jp) {
+  __shared__ __align__(16) float rows_s[4][64 * UP_STRIDE];
+  const int lane = threadIdx.x & 63;
+  float* rows = rows_s[threadIdx.x >> 6];
+  const int64_t first = (int64_t)blockIdx.x * 256 + (threadIdx.x & ~63);
+  const int count = first >= n ? 0 : (n - first < 64 ? (int)(n - first) : 64);
+  if (count == 0) return;
+  float4 w[REC_WORDS / 4];
+#pragma unroll
+  for (int it = 0; it < REC_WORDS / 4; ++it) {
+    const int e = it * 64 + lane, p = e / (REC_WORDS / 4);
+    w[it] = rec[first * (REC_WORDS / 4) + (p < count ? e : 0)];
   }
 #pragma unroll
-  for (int d = 0; d < 9; ++d) {
-    F[9 * o + d] = s.F[tix(i, 9, d)];
-    C[9 * o + d] = s.C[tix(i, 9, d)];
+  for (int it = 0; it < REC_WORDS / 4; ++it) {
+    const int e = it * 64 + lane, p = e / (REC_WORDS / 4), q = e % (REC_WORDS / 4);
+    *reinterpret_cast<float4*>(rows + p * UP_STRIDE + 4 * q) = w[it];
   }
-  Jp[o] = s.Jp[i];
+  __builtin_amdgcn_wave_barrier();
+  if (count == 64) {
+    rows_split<3, true>(rows, REC_X, x, first, count, lane);
+    rows_split<3, true>(rows, REC_V, v, first, count, lane);
+    rows_split<9, true>(rows, REC_F, F, first, count, lane);
+    rows_split<9, true>(rows, REC_C, C, first, count, lane);
+  } else {
+    rows_split<3, false>(rows, REC_X, x, first, count, lane);
+    rows_split<3, false>(rows, REC_V, v, first, count, lane);
+    rows_split<9, false>(rows, REC_F, F, first, count, lane);
+    rows_split<9, false>(rows, REC_C, C, first, count, lane);
+  }
+  if (lane < count) Jp[first + lane] = rows[lane * UP_STRIDE + REC_JP];
 }
 
 // Positions in the caller's order (one frame of the rollout output).
@@ -1380,6 +1585,11 @@ __global__ void particle_sums_kernel(EngineState s, int64_t n, double* out) {
 }
 
 // ================================================================ host ====
+// From this many particles a download takes two passes through records.
+// Arbitrary order, one / two passes in us: 131,072 39 / 38 (launches), 2^20
+// 110 / 98, 2^21 213 / 200, 5,000,000 899 / 462.
+constexpr int64_t TWO_PASS_DOWNLOAD = 1 << 20;
+
 static inline unsigned nblk(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
 #define HIPCHK(expr)                                                                 \
@@ -1488,12 +1698,21 @@ int Engine::init(int64_t n_max_, int nscenes, const mpm_scene* sc, int nmat_, co
   // particle state (two copies for reordering)
   for (int b = 0; b < 2; ++b) {
     EngineState& s = st[b];
-    if ((rc = alloc((void**)&s.x, 12 * n)) || (rc = alloc((void**)&s.v, 12 * n)) ||
-        (rc = alloc((void**)&s.F, 36 * n)) || (rc = alloc((void**)&s.C, 36 * n)) ||
-        (rc = alloc((void**)&s.Jp, 4 * n)) || (rc = alloc((void**)&s.mass, 4 * n)) ||
-        (rc = alloc((void**)&s.mu0, 4 * n)) || (rc = alloc((void**)&s.lam0, 4 * n)) ||
-        (rc = alloc((void**)&s.attr, 4 * n)) || (rc = alloc((void**)&s.order, 4 * n)))
+    // 104 bytes per particle beside x and attr, which a rebin's keys read;
+    // the same memory holds 128-byte records of an upload or a download
+    float* rest = nullptr;
+    if ((rc = alloc((void**)&s.x, 12 * n)) || (rc = alloc((void**)&s.attr, 4 * n)) ||
+        (rc = alloc((void**)&rest, 4 * REC_WORDS * n)))
       return rc;
+    rec_mem[b] = reinterpret_cast<float4*>(rest);
+    s.v = rest;
+    s.F = rest + 3 * n;
+    s.C = rest + 12 * n;
+    s.Jp = rest + 21 * n;
+    s.mass = rest + 22 * n;
+    s.mu0 = rest + 23 * n;
+    s.lam0 = rest + 24 * n;
+    s.order = reinterpret_cast<uint32_t*>(rest + 25 * n);
   }
   // grids
   if ((rc = alloc((void**)&d_acc, sizeof(float4) * 64 * blocks))) return rc;
@@ -1546,6 +1765,7 @@ EngineArgs Engine::args(double* sums, int max_steps, int sel) const {
   a.s = st[cur];
   a.src = st[cur ^ 1];
   a.perm = nullptr;
+  a.rec = nullptr;
   a.scenes = d_scenes;
   a.mats = d_mats;
   a.nmat = nmat;
@@ -1602,14 +1822,23 @@ int Engine::upload(const mpm_particles* p, const int32_t* scene_ids) {
   n = p->n;
   cur = 0;
   since_bin = -1;
-  if (n > 0)
-    hipLaunchKernelGGL(upload_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[0], n,
-                       (const float*)p->x, (const float*)p->v, (const float*)p->F, (const float*)p->C,
-                       (const float*)p->Jp, (const float*)p->mass, (const float*)p->mu0,
-                       (const float*)p->lambda0, p->mat_scalar, p->material, scene_ids,
-                       (int)scenes_host.size());
+  in_records = n > 0;
+  if (n > 0) {
+    const UploadArgs u{(const float*)p->x,       (const float*)p->v,    (const float*)p->F,
+                       (const float*)p->C,       (const float*)p->Jp,   (const float*)p->mass,
+                       (const float*)p->mu0,     (const float*)p->lambda0, p->material, scene_ids,
+                       p->mat_scalar,            (int)scenes_host.size()};
+    hipLaunchKernelGGL(upload_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[0], rec_mem[0], n, u);
+  }
   HIPCHK(hipGetLastError());
   return MPM_OK;
+}
+
+void Engine::tiled() {
+  if (!in_records) return;
+  hipLaunchKernelGGL(unpack_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[1], rec_mem[0], n);
+  cur = 1;
+  in_records = false;
 }
 
 int Engine::download(mpm_particles* p) {
@@ -1617,9 +1846,16 @@ int Engine::download(mpm_particles* p) {
     set_error("mpm_state_download: needs FP32 arrays x, v, F, C, Jp with the uploaded n");
     return MPM_ERR_ARG;
   }
-  if (n > 0)
+  tiled();
+  if (n > 0 && n < TWO_PASS_DOWNLOAD) {
     hipLaunchKernelGGL(download_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[cur], n,
                        (float*)p->x, (float*)p->v, (float*)p->F, (float*)p->C, (float*)p->Jp);
+  } else if (n > 0) {  // through the other state copy, which holds nothing between runs
+    float4* rec = rec_mem[cur ^ 1];
+    hipLaunchKernelGGL(pack_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[cur], n, rec);
+    hipLaunchKernelGGL(split_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, rec, n, (float*)p->x,
+                       (float*)p->v, (float*)p->F, (float*)p->C, (float*)p->Jp);
+  }
   HIPCHK(hipGetLastError());
   return MPM_OK;
 }
@@ -1775,6 +2011,7 @@ void Engine::enqueue_segment(int len, bool bin, hipStream_t s, double* sums, int
   {
     EngineArgs a0 = args(sums, max_steps, 0);
     a0.perm = bin ? pending_perm : nullptr;
+    a0.rec = in_records ? rec_mem[0] : nullptr;  // a segment after an upload rebins
     pending_perm = nullptr;
     launch_transfer(cont ? 3 : 0, s, a0, sep);
   }
@@ -1844,7 +2081,7 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
     if (graphed) {
       const int parity = cur;
       const GraphKey key{n, len, parity, bin ? 1 : 0, (uintptr_t)sums, sums ? nsteps : 0, cont ? 1 : 0,
-                         fin ? 1 : 0};
+                         fin ? 1 : 0, in_records ? 1 : 0};
       auto it = graphs.find(key);
       hipGraphExec_t exec = nullptr;
       if (it == graphs.end()) {
@@ -1866,6 +2103,7 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
       enqueue_segment(len, bin, own_stream, sums, nsteps, frames, done, sink, cont, fin);
     }
     HIPCHK(hipGetLastError());
+    in_records = false;
     since_bin = bin ? len : since_bin + len;
     last_list = (len - 1) & 1;
     done += len;
@@ -1898,6 +2136,7 @@ int Engine::positions(float* x) {
     set_error("mpm_state_positions: null output");
     return MPM_ERR_ARG;
   }
+  tiled();
   enqueue_frame(own_stream, x, 0);
   HIPCHK(hipGetLastError());
   return MPM_OK;
@@ -1923,6 +2162,7 @@ int Engine::particle_sums(double* out) {
   // cleared on the engine's own stream (a null-stream memset would not be
   // ordered with it)
   hipLaunchKernelGGL(fill_f64_kernel, dim3(1), dim3(64), 0, own_stream, d, (int64_t)8, 0.0);
+  tiled();
   if (n > 0)
     hipLaunchKernelGGL(particle_sums_kernel, dim3(256), dim3(ENG_THREADS), 0, own_stream, st[cur], n, d);
   HIPCHK(hipStreamSynchronize(own_stream));
