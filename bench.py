@@ -181,8 +181,8 @@ def batched_bench(steps, dev):
     run = BatchedRun(work, device=dev)
     tuned = run.autotune(steps=32, reps=2, cache_path=None)
     run.upload()
-    for _ in range(2):  # captures the timed shape's graphs (both buffer parities)
-        run.engine.request_rebin()
+    for _ in range(2):  # captures the timed shape's graphs
+        run.upload()
         run.run(steps, check_oob=False)
     # the timed substeps are substeps 0 .. steps of the configuration (the
     # upload makes the first of them rebin)
@@ -450,10 +450,10 @@ def main():
 
     restart()
     eng.run(args.warmup, check_oob=False)
-    # the timed window's shape from a rebin, once per state-buffer parity, so
-    # that its graphs are captured before the clock starts
+    # the timed window's shape from an upload, so that its graphs are captured
+    # before the clock starts
     for _ in range(2):
-        eng.request_rebin()
+        restart()
         eng.run(args.steps, check_oob=False)
     torch.cuda.synchronize()
     print(f"[bench] warmup {args.warmup} (+ graph capture of the timed shape) done", file=sys.stderr, flush=True)
@@ -484,7 +484,7 @@ def main():
         # whole rebin periods from t = 0 (their graphs captured first)
         ks = args.steady_periods * args.sort_every
         for _ in range(2):
-            eng.request_rebin()
+            restart()
             eng.run(ks, check_oob=False)
         sms, _ = timed(ks)
         steady = {"steps": ks, "rebins": args.steady_periods, "ms_per_step": sms / ks,

@@ -17,20 +17,23 @@ void set_error(const std::string& msg);
 // A captured segment fixes the particle count (launch grids, sort sizes),
 // the segment length, whether it rebins first, which state buffer is current,
 // the sums destination, and whether it continues the run's previous segment
-// (cont) and ends the run (fin), and whether it reads uploaded records; any
+// (cont) and ends the run (fin), whether it reads uploaded records, the
+// substep of the segment it starts at, and which speed counts it sends; any
 // of them changing needs another graph.
 struct GraphKey {
   int64_t n;
   int len, parity, bin;
   uintptr_t sums;
-  int nsteps, cont, fin, records;
+  int nsteps, cont, fin, records, k0, speeds;
   bool operator<(const GraphKey& o) const {
-    return std::tie(n, len, parity, bin, sums, nsteps, cont, fin, records) <
-           std::tie(o.n, o.len, o.parity, o.bin, o.sums, o.nsteps, o.cont, o.fin, o.records);
+    return std::tie(n, len, parity, bin, sums, nsteps, cont, fin, records, k0, speeds) <
+           std::tie(o.n, o.len, o.parity, o.bin, o.sums, o.nsteps, o.cont, o.fin, o.records, o.k0, o.speeds);
   }
 };
 // Captured graphs kept per context; beyond this the cache is emptied first.
-constexpr size_t MAX_GRAPHS = 16;
+constexpr size_t MAX_GRAPHS = 32;
+// Shortest rebin cadence the engine takes by itself.
+constexpr int MIN_CADENCE = 8;
 
 struct CorrExtract {
   uint16_t* X;      // rows x 352 BF16 features
@@ -64,6 +67,12 @@ struct Engine {
   // fused passes take chunks from per-XCD ticket queues (set for engines of
   // 8 or more scenes, whose many uneven chunks the queue balances)
   bool dyn_sched = false;
+  // substeps between rebins for the speeds last seen (cadence_of; 0: none
+  // seen, sort_every applies, which also bounds it)
+  int cadence = 0;
+  bool speeds_uploaded = false;  // an upload's counts wait for the next run
+  bool speeds_waited = false;    // the last run's do, and the host has waited for that run
+  const uint32_t* speeds_from = nullptr;  // see EngineArgs; set while a probing segment is enqueued
   // set while a segment with per-substep state output is enqueued: the fused
   // pass then writes v and C every substep
   bool store_vc = false;
@@ -98,6 +107,8 @@ struct Engine {
   uint32_t *d_flags = nullptr, *d_list = nullptr, *d_bstart = nullptr, *d_bend = nullptr;
   uint32_t* d_counters = nullptr;
   unsigned long long *d_oob = nullptr, *d_fallback = nullptr;
+  uint32_t* d_speeds = nullptr;
+  uint32_t* h_speeds = nullptr;  // pinned: totals per class, then the sent flag
   int4* d_chunks = nullptr;
   uint32_t *d_nchunks = nullptr, *d_keys = nullptr, *d_vals = nullptr,
            *d_bocc = nullptr, *d_part = nullptr;
@@ -135,7 +146,7 @@ struct Engine {
   void tiled();
   // rebin; also starts the segment of len substeps (counters, sums index)
   void enqueue_bin(hipStream_t s, int len, int with_sums);
-  void enqueue_segment(int len, bool bin, hipStream_t s, double* sums, int max_steps, float* frames,
+  void enqueue_segment(int k0, int len, bool bin, hipStream_t s, double* sums, int max_steps, float* frames,
                        int64_t step0, const StateSink* sink, bool cont, bool fin);
   // destroy every captured graph (after anything they baked in changes)
   void drop_graphs();
@@ -158,6 +169,7 @@ struct Engine {
   int grid_velocity(const uint32_t* nodes, int64_t count, float* out);
   int set_planes(int scene, int count, const double* points, const double* normals, int quirks);
   hipEvent_t tevent();
+  int cadence_of(const uint32_t* counts) const;
   int run(int nsteps, double* sums, float* frames = nullptr, const StateSink* sink = nullptr);
   int take_counter(int which, int64_t* out);
   int particle_sums(double* out);

@@ -5,6 +5,7 @@
 #include <hip/hip_ext.h>
 #include <string.h>
 
+#include <chrono>
 #include <string>
 #include <vector>
 
@@ -644,6 +645,7 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
           storek<3>(a.s.v, p, v);
           storek<9>(a.s.C, p, C);
         }
+        if constexpr (MODE == 2) count_speed(a.speeds, v, sc.dt * sc.inv_dx);
         if (!ok) {
           defer(a, p, MODE == 2 ? 3u : 1u);
           continue;
@@ -942,7 +944,7 @@ __global__ __launch_bounds__(ENG_THREADS) void deferred_kernel(EngineArgs a) {
   if (done_here) atomicAdd(a.fallback, (unsigned long long)done_here);
 }
 
-// Start of a segment: clear both marked-block list counters, both deferred
+// Start of a segment (its kernel also clears the speed counts): clear both marked-block list counters, both deferred
 // counts, the grid update's start ticket and the chunk queues, advance the
 // per-substep sums index by the segment length, and, when the segment
 // rebins, start a new candidate list (count 0, next generation).
@@ -960,8 +962,27 @@ __device__ __forceinline__ void segment_begin(uint32_t* counters, int len, int w
   }
 }
 
-__global__ void segment_begin_kernel(uint32_t* counters, int len, int with_sums, int bin) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) segment_begin(counters, len, with_sums, bin);
+// The segment start's part of the speed counts, by one workgroup: totals to
+// the host where it asked for them, then both sets cleared.
+__device__ __forceinline__ void segment_speeds(const EngineArgs& a) {
+  const int t = threadIdx.x;
+  if (a.speeds_from) {
+    if (t < SPEED_CLASSES) {
+      uint32_t sum = 0;
+#pragma unroll 16
+      for (int c = 0; c < SPEED_COPIES; ++c) sum += a.speeds_from[c * SPEED_WORDS + t];
+      __hip_atomic_store(a.speeds_to + t, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __threadfence_system();
+    }
+    __syncthreads();
+    if (t == 0) __hip_atomic_store(a.speeds_to + SPEED_CLASSES, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  for (int i = t; i < 2 * SPEED_SET; i += blockDim.x) a.speeds[i] = 0u;
+}
+
+__global__ void segment_begin_kernel(EngineArgs a, int len, int with_sums, int bin) {
+  if (threadIdx.x == 0) segment_begin(a.counters, len, with_sums, bin);
+  segment_speeds(a);
 }
 
 // ------------------------------------------------------------ grid update ----
@@ -1228,6 +1249,7 @@ __global__ __launch_bounds__(RS_THREADS) void engine_keys_kernel(EngineArgs a, i
   __shared__ uint32_t h[RS_BINS];
   const int64_t gid = (int64_t)blockIdx.x * RS_THREADS + threadIdx.x;
   if (gid == 0) segment_begin(a.counters, len, with_sums, 1);
+  if (blockIdx.x == 0) segment_speeds(a);
   for (int64_t j = gid; j < nblocks; j += (int64_t)gridDim.x * RS_THREADS) bocc[j] = 0u;
   const bool one_scene = a.nscenes == 1;
   const SceneDev sc0 = a.scenes[0];
@@ -1359,6 +1381,8 @@ __device__ __forceinline__ void rows_in(float* rows, int stride, int at, const f
 }
 
 struct UploadArgs {
+  const SceneDev* scenes;
+  uint32_t* speeds;
   const float *x, *v, *F, *C, *Jp, *mass, *mu0, *lam0;
   const int32_t *material, *scene;
   int mat_scalar, nscenes;
@@ -1391,8 +1415,11 @@ __device__ __forceinline__ void upload_piece(const EngineState& s, float4* __res
   // the piece's rows belong to this wave, whose LDS accesses are in order
   __builtin_amdgcn_wave_barrier();
   if (FULL || lane < count) {
+    const float* row = rows + lane * UP_STRIDE;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) s.x[tix(first + lane, 3, d)] = rows[lane * UP_STRIDE + REC_X + d];
+    for (int d = 0; d < 3; ++d) s.x[tix(first + lane, 3, d)] = row[REC_X + d];
+    const SceneDev& sc = u.scenes[__float_as_uint(row[REC_ATTR]) >> 8];
+    count_speed(u.speeds, row + REC_V, sc.dt * sc.inv_dx);
   }
 #pragma unroll
   for (int it = 0; it < REC_WORDS / 4; ++it) {
@@ -1610,6 +1637,8 @@ void Engine::release() {
   graphs.clear();
   for (void* p : allocs) hipFree(p);
   allocs.clear();
+  if (h_speeds) hipHostFree(h_speeds);
+  h_speeds = nullptr;
   if (ev_in) hipEventDestroy(ev_in);
   if (ev_out) hipEventDestroy(ev_out);
   for (auto& e : tevents) hipEventDestroy(e);
@@ -1724,6 +1753,8 @@ int Engine::init(int64_t n_max_, int nscenes, const mpm_scene* sc, int nmat_, co
   if ((rc = alloc((void**)&d_counters, sizeof(uint32_t) * 16))) return rc;
   if ((rc = alloc((void**)&d_oob, sizeof(unsigned long long) * 2))) return rc;
   d_fallback = d_oob + 1;
+  if ((rc = alloc((void**)&d_speeds, sizeof(uint32_t) * 2 * SPEED_SET))) return rc;
+  HIPCHK(hipHostMalloc((void**)&h_speeds, sizeof(uint32_t) * SPEED_WORDS, hipHostMallocDefault));
   // binning workspace
   const int64_t max_chunks = n / 256 + blocks + 1;
   if ((rc = alloc((void**)&d_chunks, sizeof(int4) * (max_chunks < n + 1 ? max_chunks : n + 1)))) return rc;
@@ -1753,6 +1784,7 @@ int Engine::init(int64_t n_max_, int nscenes, const mpm_scene* sc, int nmat_, co
   HIPCHK(hipMemset(d_flags, 0, sizeof(uint32_t) * blocks));
   HIPCHK(hipMemset(d_counters, 0, sizeof(uint32_t) * 16));
   HIPCHK(hipMemset(d_oob, 0, sizeof(unsigned long long) * 2));
+  HIPCHK(hipMemset(d_speeds, 0, sizeof(uint32_t) * 2 * SPEED_SET));
   HIPCHK(hipMemset(d_nchunks, 0, sizeof(uint32_t) * 4));
   // the memsets above run on the null stream; the engine's stream does not
   // synchronise with it, so wait for them here
@@ -1781,6 +1813,9 @@ EngineArgs Engine::args(double* sums, int max_steps, int sel) const {
   a.list_count = d_counters + sel;
   a.other_count = d_counters + (sel ^ 1);
   a.counters = d_counters;
+  a.speeds = d_speeds;
+  a.speeds_from = speeds_from;
+  a.speeds_to = h_speeds;
   a.chunks = d_chunks;
   a.keys = d_sorted_keys;
   a.nchunks = d_nchunks;
@@ -1824,10 +1859,17 @@ int Engine::upload(const mpm_particles* p, const int32_t* scene_ids) {
   since_bin = -1;
   in_records = n > 0;
   if (n > 0) {
-    const UploadArgs u{(const float*)p->x,       (const float*)p->v,    (const float*)p->F,
-                       (const float*)p->C,       (const float*)p->Jp,   (const float*)p->mass,
-                       (const float*)p->mu0,     (const float*)p->lambda0, p->material, scene_ids,
-                       p->mat_scalar,            (int)scenes_host.size()};
+    uint32_t* speeds = d_speeds + SPEED_SET;
+    if (speeds_uploaded) fill_u32(own_stream, speeds, SPEED_SET, 0u);  // a second upload without a run
+    const UploadArgs u{d_scenes,           speeds,
+                       (const float*)p->x, (const float*)p->v,
+                       (const float*)p->F, (const float*)p->C,
+                       (const float*)p->Jp, (const float*)p->mass,
+                       (const float*)p->mu0, (const float*)p->lambda0,
+                       p->material,        scene_ids,
+                       p->mat_scalar,      (int)scenes_host.size()};
+    speeds_uploaded = true;
+    cadence = 0;
     hipLaunchKernelGGL(upload_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[0], rec_mem[0], n, u);
   }
   HIPCHK(hipGetLastError());
@@ -1865,7 +1907,8 @@ int Engine::download(mpm_particles* p) {
 // order in the segment's first P2G (through pending_perm).
 void Engine::enqueue_bin(hipStream_t s, int len, int with_sums) {
   if (n <= 0) {
-    hipLaunchKernelGGL(segment_begin_kernel, dim3(1), dim3(64), 0, s, d_counters, len, with_sums, 1);
+    hipLaunchKernelGGL(segment_begin_kernel, dim3(1), dim3(256), 0, s, args(nullptr, 0, 0), len,
+                       with_sums, 1);
     hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, d_nchunks, (int64_t)1, 0u);
     return;
   }
@@ -1989,18 +2032,21 @@ void Engine::enqueue_state(hipStream_t s, const StateSink* sink, int64_t step) {
 // substep plus this segment's first P2G, moving the particles into the new
 // order (MODE 3) instead of a G2P, the rebin and a moving P2G.  fin: the
 // run's last segment, which ends with the G2P.
-void Engine::enqueue_segment(int len, bool bin, hipStream_t s, double* sums, int max_steps, float* frames,
+//
+// k0 > 0: substeps k0 .. k0 + len - 1 of a segment whose first k0 were
+// enqueued before (no sums).
+void Engine::enqueue_segment(int k0, int len, bool bin, hipStream_t s, double* sums, int max_steps, float* frames,
                              int64_t step0, const StateSink* sink, bool cont, bool fin) {
   const int ws = sums ? 1 : 0;
   if (bin)
     enqueue_bin(s, len, ws);
-  else
-    hipLaunchKernelGGL(segment_begin_kernel, dim3(1), dim3(64), 0, s, d_counters, len, ws, 0);
+  else if (k0 == 0)
+    hipLaunchKernelGGL(segment_begin_kernel, dim3(1), dim3(256), 0, s, args(nullptr, 0, 0), len, ws, 0);
   // substep k appends to active list k % 2; its grid update clears the other
   const size_t rec_nn = (size_t)(scenes_host[0].res + 1) * (scenes_host[0].res + 1) * (scenes_host[0].res + 1);
   auto grid_args = [&](int k) {
     EngineArgs a = args(sums, max_steps, k & 1);
-    if (sink && sink->grids) a.grid_rec = sink->grids + (size_t)(step0 + k) * 7 * rec_nn;
+    if (sink && sink->grids) a.grid_rec = sink->grids + (size_t)(step0 + k - k0) * 7 * rec_nn;
     return a;
   };
   // the deferred FP64 particles are finished by the grid update unless the
@@ -2008,34 +2054,68 @@ void Engine::enqueue_segment(int len, bool bin, hipStream_t s, double* sums, int
   // per-substep state output also needs each substep's v and C in memory
   const bool sep = corr_on || sink != nullptr;
   store_vc = sink != nullptr;
-  {
+  // step0: the run's index of this call's first substep
+  if (k0 == 0) {
     EngineArgs a0 = args(sums, max_steps, 0);
     a0.perm = bin ? pending_perm : nullptr;
     a0.rec = in_records ? rec_mem[0] : nullptr;  // a segment after an upload rebins
     pending_perm = nullptr;
     launch_transfer(cont ? 3 : 0, s, a0, sep);
+    if (cont) {  // the previous segment's last substep finished its G2P
+      enqueue_frame(s, frames, step0 - 1);
+      enqueue_state(s, sink, step0 - 1);
+    }
+    if (corr_on) launch_cellf(s, args(sums, max_steps, 0));
+    launch_grid(s, grid_args(0), ws, len, 0, sep ? 0 : 1);
+    if (corr_on) launch_corrector(s, args(sums, max_steps, 0), nullptr);
   }
-  if (cont) {  // the previous segment's last substep finished its G2P
-    enqueue_frame(s, frames, step0 - 1);
-    enqueue_state(s, sink, step0 - 1);
-  }
-  if (corr_on) launch_cellf(s, args(sums, max_steps, 0));
-  launch_grid(s, grid_args(0), ws, len, 0, sep ? 0 : 1);
-  if (corr_on) launch_corrector(s, args(sums, max_steps, 0), nullptr);
-  for (int k = 1; k < len; ++k) {
+  for (int k = k0 > 0 ? k0 : 1; k < k0 + len; ++k) {
     launch_transfer(1, s, args(sums, max_steps, k & 1), sep);
-    enqueue_frame(s, frames, step0 + k - 1);  // substep k-1 finished its G2P
-    enqueue_state(s, sink, step0 + k - 1);
+    enqueue_frame(s, frames, step0 + k - k0 - 1);  // substep k-1 finished its G2P
+    enqueue_state(s, sink, step0 + k - k0 - 1);
     if (corr_on) launch_cellf(s, args(sums, max_steps, k & 1));
     launch_grid(s, grid_args(k), ws, len, k, sep ? 0 : 1);
     if (corr_on) launch_corrector(s, args(sums, max_steps, k & 1), nullptr);
   }
   if (fin) {
-    launch_transfer(2, s, args(sums, max_steps, len & 1));
+    launch_transfer(2, s, args(sums, max_steps, (k0 + len) & 1));
     enqueue_frame(s, frames, step0 + len - 1);
     enqueue_state(s, sink, step0 + len - 1);
   }
   store_vc = false;
+}
+
+// Rebin cadence from the particles per speed class: the
+// candidate K <= sort_every with the least cost per substep,
+//   rebin / K + outside / particle-substep sum_p f(s_p, K).
+// A particle of speed s (cells per substep) leaves the arena of its chunk,
+// which reaches one cell past a 4-cell block, with probability (s t - 1) / 4
+// t substeps after a rebin, so f = (s K - 1)^2 / (8 s K) on average for
+// s K > 1; outside it costs 108 device atomics, about 10 ns of the chip's
+// atomic rate.  A rebin measured 75 us at 2^17 particles, 130 us at 2^20 and
+// 500 us at 5 million.  Three cubes of 2^20 particles at up to 8.8 m/s on a
+// 128^3 grid, 64 substeps: 10.0 ms rebinning every 48 substeps, 7.5 ms every
+// 24 (chosen) or 16, 7.7 every 12; at the 0.5 m/s of the headline scene no
+// speed reaches the first class and sort_every stays.
+int Engine::cadence_of(const uint32_t* cnt) const {
+  const double rebin = 70e-6 + 80e-12 * (double)n, outside = 10e-9;
+  int best = sort_every;
+  double best_cost = 1e30;
+  for (const int k : {sort_every, 32, 24, 16, 12, MIN_CADENCE}) {
+    if (k > sort_every) continue;
+    double cost = rebin / k;
+    for (int b = 0; b < SPEED_CLASSES; ++b) {
+      const double next = b + 1 < SPEED_CLASSES ? SPEED_EDGE[b + 1] : 2 * SPEED_EDGE[b];
+      const double sk = 0.5 * (SPEED_EDGE[b] + next) * k;
+      const double f = sk > 1 ? (sk - 1) * (sk - 1) / (8 * sk) : 0.0;
+      cost += outside * cnt[b] * (f < 1 ? f : 1.0);
+    }
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = k;
+    }
+  }
+  return best;
 }
 
 int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) {
@@ -2044,6 +2124,22 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
     return MPM_ERR_ARG;
   }
   if (nsteps == 0) return MPM_OK;
+  // Probe (adaptive cadence): the run's first kernel sends the counts of the upload, or of the
+  // run before if the host has waited for that, and the first MIN_CADENCE
+  // substeps are enqueued by themselves; the host waits for the counts while
+  // the GPU works on those, and the cadence then holds for the rest of the
+  // run (and until new counts).  The counts follow program order, so a
+  // sequence of calls always takes the same rebins.
+  bool probe = (speeds_uploaded || speeds_waited) && n > 0 && nsteps > MIN_CADENCE && sort_every > MIN_CADENCE && !sums;
+  if (probe) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(user_stream, &cap));
+    probe = cap == hipStreamCaptureStatusNone;
+  }
+  if (probe) __atomic_store_n(h_speeds + SPEED_CLASSES, 0u, __ATOMIC_RELEASE);
+  speeds_from = probe ? d_speeds + (speeds_uploaded ? SPEED_SET : 0) : nullptr;
+  const bool from_upload = speeds_uploaded;
+  speeds_uploaded = speeds_waited = false;
   HIPCHK(hipEventRecord(ev_in, user_stream));
   HIPCHK(hipStreamWaitEvent(own_stream, ev_in, 0));
   if (sums) {
@@ -2058,7 +2154,7 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
                        reinterpret_cast<uint32_t*>(sink->grids), cnt, 0u);
   }
   // Segments: the particles are rebinned when they never were since the
-  // upload (or a rebin request) or after sort_every substeps; the schedule
+  // upload (or a rebin request) or after `every` substeps; the schedule
   // carries over from one call to the next, so callers that advance a few
   // substeps per call do not pay a rebin per call.  Every call ends with
   // complete particle state (G2P), so a call costs one split P2G / G2P pair
@@ -2066,29 +2162,28 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
   // grid update and the next one (which always rebins: segments are cut at
   // the schedule's rebins) starts with the fused G2P of that substep, which
   // also moves the particles into the new order.
-  int done = 0;
+  int done = 0, k0 = 0;  // k0: substeps of the current segment already enqueued
   while (done < nsteps) {
-    const bool bin = since_bin < 0 || since_bin >= sort_every || n <= 0;
-    const int room = bin ? sort_every : sort_every - since_bin;
-    const int len = (nsteps - done) < room ? (nsteps - done) : room;
+    const int every = cadence > 0 && cadence < sort_every ? cadence : sort_every;
+    const bool bin = n <= 0 || since_bin < 0 || since_bin >= every;
+    if (bin) k0 = 0;
+    int len = bin ? every : every - since_bin;
+    if (probe && len > MIN_CADENCE) len = MIN_CADENCE;
+    if (len > nsteps - done) len = nsteps - done;
     const bool cont = n > 0 && done > 0;
     const bool fin = n <= 0 || done + len == nsteps;
-    if (cont && !bin) {
-      set_error("mpm_run: internal error: a continued segment must rebin");
-      return MPM_ERR_HIP;
-    }
     const bool graphed = use_graph && !timing && n > 0 && !frames && !sink;
     if (graphed) {
       const int parity = cur;
       const GraphKey key{n, len, parity, bin ? 1 : 0, (uintptr_t)sums, sums ? nsteps : 0, cont ? 1 : 0,
-                         fin ? 1 : 0, in_records ? 1 : 0};
+                         fin ? 1 : 0, in_records ? 1 : 0, k0, speeds_from ? (from_upload ? 2 : 1) : 0};
       auto it = graphs.find(key);
       hipGraphExec_t exec = nullptr;
       if (it == graphs.end()) {
         if (graphs.size() >= MAX_GRAPHS) drop_graphs();
         hipGraph_t graph;
         HIPCHK(hipStreamBeginCapture(own_stream, hipStreamCaptureModeThreadLocal));
-        enqueue_segment(len, bin, own_stream, sums, nsteps, nullptr, 0, nullptr, cont, fin);
+        enqueue_segment(k0, len, bin, own_stream, sums, nsteps, nullptr, 0, nullptr, cont, fin);
         HIPCHK(hipStreamEndCapture(own_stream, &graph));
         HIPCHK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
         HIPCHK(hipGraphDestroy(graph));
@@ -2100,13 +2195,26 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
       HIPCHK(hipGraphLaunch(exec, own_stream));
       cur = bin ? parity ^ 1 : parity;
     } else {
-      enqueue_segment(len, bin, own_stream, sums, nsteps, frames, done, sink, cont, fin);
+      enqueue_segment(k0, len, bin, own_stream, sums, nsteps, frames, done, sink, cont, fin);
     }
     HIPCHK(hipGetLastError());
     in_records = false;
     since_bin = bin ? len : since_bin + len;
-    last_list = (len - 1) & 1;
+    k0 += len;
+    last_list = (k0 - 1) & 1;
     done += len;
+    if (probe) {
+      probe = false;
+      speeds_from = nullptr;
+      uint32_t* const sent = h_speeds + SPEED_CLASSES;
+      // bounded: work that the caller's stream waits for may come from this
+      // very thread, after the call
+      const auto start = std::chrono::steady_clock::now();
+      while (!__atomic_load_n(sent, __ATOMIC_ACQUIRE) &&
+             std::chrono::steady_clock::now() - start < std::chrono::seconds(1))
+        __builtin_ia32_pause();
+      if (__atomic_load_n(sent, __ATOMIC_ACQUIRE)) cadence = cadence_of(h_speeds);
+    }
   }
   HIPCHK(hipEventRecord(ev_out, own_stream));
   HIPCHK(hipStreamWaitEvent(user_stream, ev_out, 0));
@@ -2147,6 +2255,7 @@ int Engine::take_counter(int which, int64_t* out) {
   unsigned long long v = 0;
   unsigned long long* p = which == 0 ? d_oob : d_fallback;
   HIPCHK(hipMemcpy(&v, p, sizeof(v), hipMemcpyDeviceToHost));
+  speeds_waited = !speeds_uploaded;  // the last run is over: its speeds can be had at once
   // cleared on the engine's own stream, ahead of its later work
   hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, own_stream, reinterpret_cast<uint32_t*>(p),
                      (int64_t)2, 0u);

@@ -92,6 +92,15 @@ struct EngineState {
 constexpr int REC_X = 0, REC_V = 3, REC_F = 6, REC_C = 15, REC_JP = 24, REC_MASS = 25, REC_MU = 26, REC_LAM = 27,
               REC_ATTR = 28, REC_WORDS = 32;
 
+// Speeds of the particles in cells per substep (largest axis), counted after
+// an upload and at the end of a run: class b holds the speeds from
+// SPEED_EDGE[b] to the next edge (below the first: not counted).  The
+// workgroups spread their counts over SPEED_COPIES rows, since same-address
+// device atomics run one after the other.
+constexpr int SPEED_CLASSES = 9, SPEED_COPIES = 64, SPEED_WORDS = 16, SPEED_SET = SPEED_COPIES * SPEED_WORDS;
+constexpr float SPEED_EDGE[SPEED_CLASSES] = {1.f / 48, 1.f / 32, 1.f / 24, 1.f / 16, 1.f / 12,
+                                             1.f / 8,  1.f / 6,  1.f / 4,  1.f / 2};
+
 struct EngineArgs {
   EngineState s;
   // The first P2G after a rebin also moves the particles into binned order:
@@ -129,6 +138,13 @@ struct EngineArgs {
   uint32_t* hard_count;  // this substep's deferred count (counters[3] or [6] by parity)
   uint32_t* other_hard;  // the other parity's count (cleared by the grid update)
   uint32_t* defer_ticket;  // counters[7]: start order of the grid update's workgroups
+  // class counts, SPEED_COPIES rows of SPEED_WORDS each: of the run's last
+  // G2P, then of the upload; a segment's start clears both
+  uint32_t* speeds;
+  // the set whose totals a run's first kernel sends to the host (null: none)
+  // and where to (pinned; word SPEED_CLASSES is set last)
+  const uint32_t* speeds_from;
+  uint32_t* speeds_to;
   const int4* chunks;  // start, count, global block, scene (one per occupied block)
   const uint32_t* keys;  // binned (sorted) cell keys of the current order
   const uint32_t* nchunks;
@@ -209,6 +225,22 @@ __device__ __forceinline__ void mark_active(const EngineArgs& a, uint32_t g) {
       const uint32_t idx = atomicAdd(a.list_count, 1u);
       a.list[idx] = g;
     }
+  }
+}
+
+// Adds the particles of this wave's active lanes to the speed counts.
+__device__ __forceinline__ void count_speed(uint32_t* speeds, const float v[3], float cells_per_v) {
+  const float s = fmaxf(fabsf(v[0]), fmaxf(fabsf(v[1]), fabsf(v[2]))) * cells_per_v;
+  int cls = -1;
+#pragma unroll
+  for (int b = 0; b < SPEED_CLASSES; ++b) cls += s >= SPEED_EDGE[b] ? 1 : 0;
+  if (__ballot(cls >= 0) == 0ull) return;
+  const int leader = __builtin_ctzll(__ballot(true));
+  uint32_t* row = speeds + (blockIdx.x % SPEED_COPIES) * SPEED_WORDS;
+#pragma unroll
+  for (int b = 0; b < SPEED_CLASSES; ++b) {
+    const unsigned long long m = __ballot(cls == b);
+    if (m && (int)(threadIdx.x & 63) == leader) atomicAdd(row + b, (uint32_t)__popcll(m));
   }
 }
 
