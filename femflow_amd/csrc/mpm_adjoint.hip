@@ -18,9 +18,8 @@
 // fixed and a clamped or masked component passes no gradient.
 #include <hip/hip_runtime.h>
 
-#include <climits>
-
 #include "mpm355.h"
+#include "mpm_cellsum.h"
 #include "mpm_math.h"
 #include "mpm_phase.h"
 
@@ -72,35 +71,18 @@ __device__ __forceinline__ void bspline_d(float fx, float w[3], float dw[3]) {
 }
 
 // ---------------------------------------------------------------- G2P^T ----
-// The node-velocity adjoint is scattered in two levels: a wave sums the lanes
-// of each run of particles in one cell (seg_reduce), and the workgroup sums
-// those into an LDS arena over the bounding box of its particles' stencils,
-// which it then adds to the grid with one device atomic per nonzero node
-// component.  Particles in cell order give a box of a few cells, so most of
-// the adds stay on the chip; device-scope atomics, which serialise across
-// the XCDs, were the kernel's cost.  A box larger than the arena falls back
-// to one device atomic per segment.
-constexpr int AG_THREADS = 256;
-constexpr int AG_CAP = 1024;  // arena nodes (x 3 components)
-
-__device__ __forceinline__ int wave_min(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
-  return v;
-}
-__device__ __forceinline__ int wave_max(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
-  return v;
-}
-
-__global__ __launch_bounds__(AG_THREADS) void adj_g2p_kernel(AdjArgs a) {
-  __shared__ float arena[AG_CAP * 3];
-  __shared__ int box_w[AG_THREADS / 64][6];
-  __shared__ int box[6];  // low corner (3), extent (3) of the stencil box
-  // lanes past the end or out of the grid stay in the wave (its segmented
-  // atomics need every lane) and write nothing
-  const int64_t p0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// The node-velocity adjoint vt + c4 Ct (n - fx), weighted, is summed per cell
+// and workgroup before memory (mpm_cellsum.h); the rollout keeps the
+// particles in cell order.  A thread loads its 27 nodes' velocities once, all
+// in flight together, and keeps them for both uses (v', C' and the weight
+// derivatives): at 2^17 particles there are two waves per SIMD, so a chain
+// of nine dependent rows, twice, was latency, and 243 lane-shuffle sums per
+// particle were most of the rest (68 us per substep -> 28).
+__global__ __launch_bounds__(CELLSUM_THREADS) __attribute__((amdgpu_waves_per_eu(2))) void adj_g2p_kernel(AdjArgs a) {
+  using Sum = CellSum<float, 3, 3>;
+  __shared__ __align__(16) Sum::Shared sh;
+  // lanes past the end or out of the grid stay in the wave and write nothing
+  const int64_t p0 = (int64_t)blockIdx.x * CELLSUM_THREADS + threadIdx.x;
   const bool inrange = p0 < a.n;
   const int64_t p = inrange ? p0 : a.n - 1;
   int base[3];
@@ -120,26 +102,16 @@ __global__ __launch_bounds__(AG_THREADS) void adj_g2p_kernel(AdjArgs a) {
   for (int d = 0; d < 3; ++d) bspline_d(fx[d], w[d], dw[d]);
   const int64_t r1 = a.res + 1;
   const float c4 = 4.f * a.inv_dx;
-  // forward gather (v', C') of this particle
-  float vn[3] = {0.f, 0.f, 0.f}, Cn[9];
+  float g[27][3];
+  {
+    const float* g0 = a.gv + 3 * (((int64_t)base[0] * r1 + base[1]) * r1 + base[2]);
 #pragma unroll
-  for (int e = 0; e < 9; ++e) Cn[e] = 0.f;
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j)
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const float wt = w[0][i] * w[1][j] * w[2][k];
-        const int64_t node = ((int64_t)(base[0] + i) * r1 + (base[1] + j)) * r1 + (base[2] + k);
-        const float* g = a.gv + 3 * node;
-        const float dp[3] = {(float)i - fx[0], (float)j - fx[1], (float)k - fx[2]};
+      for (int j = 0; j < 3; ++j)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          const float wg = wt * g[d];
-          vn[d] += wg;
-#pragma unroll
-          for (int e = 0; e < 3; ++e) Cn[3 * d + e] += c4 * wg * dp[e];
-        }
-      }
+        for (int e = 0; e < 9; ++e) g[9 * i + 3 * j + e / 3][e % 3] = g0[3 * (i * r1 + j) * r1 + e];
+  }
   // adjoints of the outputs x', v', C', F'
   float xo[3], vo[3], Co[9], Fo[9], F[9];
 #pragma unroll
@@ -153,6 +125,26 @@ __global__ __launch_bounds__(AG_THREADS) void adj_g2p_kernel(AdjArgs a) {
     Fo[e] = a.Fb[9 * p + e];
     F[e] = a.F[9 * p + e];
   }
+  // forward gather (v', C') of this particle
+  float vn[3] = {0.f, 0.f, 0.f}, Cn[9];
+#pragma unroll
+  for (int e = 0; e < 9; ++e) Cn[e] = 0.f;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const float wt = w[0][i] * w[1][j] * w[2][k];
+        const float dp[3] = {(float)i - fx[0], (float)j - fx[1], (float)k - fx[2]};
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const float wg = wt * g[9 * i + 3 * j + k][d];
+          vn[d] += wg;
+#pragma unroll
+          for (int e = 0; e < 3; ++e) Cn[3 * d + e] += c4 * wg * dp[e];
+        }
+      }
   // F' = (I + dt C') F:  Fbar = (I + dt C')^T Fo,  Cbar += dt Fo F^T
   float Fbar[9], Ct[9], vt[3];
 #pragma unroll
@@ -172,97 +164,56 @@ __global__ __launch_bounds__(AG_THREADS) void adj_g2p_kernel(AdjArgs a) {
   // x' = x + dt v'
 #pragma unroll
   for (int d = 0; d < 3; ++d) vt[d] = vo[d] + a.dt * xo[d];
-  // C' depends on fx through (n - fx):  dC'_ab/dfx_c = -c4 v'_a delta_bc
-  float gx[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) gx[c] = -c4 * (Ct[c] * vn[0] + Ct[3 + c] * vn[1] + Ct[6 + c] * vn[2]);
-  const WaveSeg sg = wave_segments(valid, (int)((base[0] * r1 + base[1]) * r1 + base[2]));
-  {
-    const int t = threadIdx.x, wv = t >> 6;
-    int lo[3], hi[3];
+  // the table entry of the scatter: row d is (q, A) with q + A (i, j, k) =
+  // vt[d] + c4 Ct[d] (n - fx)
+  if (valid) {
+    float* e = sh.table + threadIdx.x * Sum::ENTRY;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      lo[d] = wave_min(valid ? base[d] : INT_MAX);
-      hi[d] = wave_max(valid ? base[d] : INT_MIN);
-    }
-    if ((t & 63) == 0) {
+      float off = 0.f;
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        box_w[wv][d] = lo[d];
-        box_w[wv][3 + d] = hi[d];
+      for (int c = 0; c < 3; ++c) {
+        e[d * Sum::ROW + 1 + c] = c4 * Ct[3 * d + c];
+        off += c4 * Ct[3 * d + c] * fx[c];
       }
+      e[d * Sum::ROW] = vt[d] - off;
     }
-    __syncthreads();
-    if (t == 0) {
-      int l[3] = {INT_MAX, INT_MAX, INT_MAX}, h[3] = {INT_MIN, INT_MIN, INT_MIN};
-      for (int w2 = 0; w2 < AG_THREADS / 64; ++w2)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          l[d] = min(l[d], box_w[w2][d]);
-          h[d] = max(h[d], box_w[w2][3 + d]);
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) e[3 * Sum::ROW + 3 * d + c] = w[d][c];
+    // C' depends on fx through (n - fx):  dC'_ab/dfx_c = -c4 v'_a delta_bc
+    float gx[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) gx[c] = -c4 * (Ct[c] * vn[0] + Ct[3 + c] * vn[1] + Ct[6 + c] * vn[2]);
+    // weight derivatives
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const float dp[3] = {(float)i - fx[0], (float)j - fx[1], (float)k - fx[2]};
+          float s = 0.f;
+#pragma unroll
+          for (int d = 0; d < 3; ++d)
+            s += g[9 * i + 3 * j + k][d] *
+                 (vt[d] + c4 * (Ct[3 * d] * dp[0] + Ct[3 * d + 1] * dp[1] + Ct[3 * d + 2] * dp[2]));
+          gx[0] += dw[0][i] * w[1][j] * w[2][k] * s;
+          gx[1] += w[0][i] * dw[1][j] * w[2][k] * s;
+          gx[2] += w[0][i] * w[1][j] * dw[2][k] * s;
         }
-      const bool any = l[0] <= h[0];
-      const int64_t e0 = any ? h[0] - l[0] + 3 : 0, e1 = any ? h[1] - l[1] + 3 : 0, e2 = any ? h[2] - l[2] + 3 : 0;
-      const bool fits = any && e0 * e1 * e2 <= AG_CAP;
-#pragma unroll
-      for (int d = 0; d < 3; ++d) box[d] = l[d];
-      box[3] = fits ? (int)e0 : 0;
-      box[4] = fits ? (int)e1 : 0;
-      box[5] = fits ? (int)e2 : 0;
-    }
-    __syncthreads();
-    const int vol = box[3] * box[4] * box[5];
-    for (int e = t; e < 3 * vol; e += AG_THREADS) arena[e] = 0.f;
-    __syncthreads();
-  }
-  const int bl0 = box[0], bl1 = box[1], bl2 = box[2], be1 = box[4], be2 = box[5];
-  const bool use_arena = box[3] > 0;
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const float wt = w[0][i] * w[1][j] * w[2][k];
-        const int64_t node = ((int64_t)(base[0] + i) * r1 + (base[1] + j)) * r1 + (base[2] + k);
-        const float* g = a.gv + 3 * node;
-        const float dp[3] = {(float)i - fx[0], (float)j - fx[1], (float)k - fx[2]};
-        // node velocity adjoint: vt + c4 Ct (n - fx), weighted
-        float gb[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d)
-          gb[d] = vt[d] + c4 * (Ct[3 * d] * dp[0] + Ct[3 * d + 1] * dp[1] + Ct[3 * d + 2] * dp[2]);
-        float* dst = a.gbar + 4 * node;
-        const int slot = ((base[0] + i - bl0) * be1 + (base[1] + j - bl1)) * be2 + (base[2] + k - bl2);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          const float r = seg_reduce(wt * gb[d], sg);
-          if (sg.tail) {
-            if (use_arena) atomicAdd(&arena[3 * slot + d], r);
-            else atomicAdd(dst + d, r);
-          }
-        }
-        // weight derivative
-        const float s = g[0] * gb[0] + g[1] * gb[1] + g[2] * gb[2];
-        gx[0] += dw[0][i] * w[1][j] * w[2][k] * s;
-        gx[1] += w[0][i] * dw[1][j] * w[2][k] * s;
-        gx[2] += w[0][i] * w[1][j] * dw[2][k] * s;
-      }
-  if (valid) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) a.xb[3 * p + d] = xo[d] + a.inv_dx * gx[d];
 #pragma unroll
-    for (int e = 0; e < 9; ++e) a.Fb[9 * p + e] = Fbar[e];
+    for (int e9 = 0; e9 < 9; ++e9) a.Fb[9 * p + e9] = Fbar[e9];
   }
-  if (!use_arena) return;  // workgroup-uniform
-  __syncthreads();
-  const int e1 = box[4], e2 = box[5], vol = box[3] * e1 * e2;
-  for (int e = threadIdx.x; e < 3 * vol; e += AG_THREADS) {
-    const float val = arena[e];
-    if (val != 0.f) {
-      const int sl = e / 3, d = e - 3 * sl;
-      const int64_t I = bl0 + sl / (e1 * e2), J = bl1 + (sl / e2) % e1, K = bl2 + sl % e2;
-      atomicAdd(a.gbar + 4 * ((I * r1 + J) * r1 + K) + d, val);
-    }
-  }
+  auto add = [&](const int* b, int c, float v) {
+    atomicAdd(a.gbar + 4 * (((int64_t)b[0] * r1 + b[1]) * r1 + b[2]) + c, v);
+  };
+  Sum::prepare(sh, base, valid);
+  Sum::sum_groups(sh, base, valid, add);
+  Sum::flush(sh, add);
 }
 
 // --------------------------------------------------------------- grid^T ----
@@ -540,7 +491,8 @@ static void adjoint_from_grids(hipStream_t st, const mpm_params* prm, const mpm_
   a.lamb = lamb;
   a.oob = oob;
   hipLaunchKernelGGL(adj_fill_kernel, dim3(nblk(4 * nn, 256)), dim3(256), 0, st, a.gbar, 4 * nn, 0.f);
-  if (a.n > 0) hipLaunchKernelGGL(adj_g2p_kernel, dim3(nblk(a.n, AG_THREADS)), dim3(AG_THREADS), 0, st, a);
+  if (a.n > 0) hipLaunchKernelGGL(adj_g2p_kernel, dim3(nblk(a.n, CELLSUM_THREADS)), dim3(CELLSUM_THREADS), 0, st,
+                                  a);
   hipLaunchKernelGGL(adj_grid_kernel, dim3(nblk(nn, 256)), dim3(256), 0, st, a);
   if (a.n > 0) hipLaunchKernelGGL(adj_p2g_kernel, dim3(nblk(a.n, 128)), dim3(128), 0, st, a);
 }

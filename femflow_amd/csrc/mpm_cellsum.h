@@ -2,9 +2,11 @@
 //
 // A workgroup takes CELLSUM_THREADS consecutive particles of a cell-ordered
 // list.  Each thread writes its particle's B-spline weights and linear terms
-// to an LDS table; each wave then walks the runs of equal stencil bases among
-// its 64 particles with one lane per (node, channel) output, so a run of m
-// particles ends in one add per output instead of m.  The adds go to an LDS
+// to an LDS table; each wave then walks the groups of equal stencil bases
+// among its 64 particles with one lane per (node, channel) output (3D: 54
+// lanes with up to two channels each; 2D: two sets of 27 lanes that take
+// alternate particles), so a group of m particles ends in one add per output
+// instead of m.  The adds go to an LDS
 // arena over the workgroup's stencil bounding box, which is added to memory
 // once, one device atomic per nonzero value.  Device-scope float atomics run
 // at about 1e10 per second over the whole chip here (one L2 per XCD, so they
@@ -31,9 +33,6 @@ template <typename T, int DIM, int NCH> struct CellSum {
   static constexpr int PAD = 16 / (int)sizeof(T);
   static constexpr int ENTRY = (NCH * ROW + 3 * DIM + PAD - 1) / PAD * PAD;
   typedef T Row3 __attribute__((ext_vector_type(4), aligned(16)));
-  // outputs per lane: 3D uses 54 lanes with up to two channels each, 2D two
-  // groups of 27 lanes that take alternate particles of a run
-  static constexpr int GROUP = DIM == 3 ? 1 : 2;
   static constexpr int ARENA = sizeof(T) == 8 ? 576 : 1024;  // nodes
 
   struct alignas(16) Shared {
@@ -98,22 +97,15 @@ template <typename T, int DIM, int NCH> struct CellSum {
     return v;
   }
 
-  // Sums every run of this wave's particles.  direct(node offsets from the
-  // run's base, channel, value, base) adds to memory where the box does not
-  // fit the arena.  The table entries of the wave were written by its own
-  // lanes; prepare()'s barriers order them.
+  // Sums every group of this wave's particles that share a base (the lanes
+  // of a group need not be neighbours: an order that was by cell some
+  // substeps ago serves as well).  direct(node, channel, value) adds to
+  // memory where the box does not fit the arena.  The table entries of the
+  // wave were written by its own lanes; prepare()'s barriers order them.
   template <typename Add>
-  static __device__ __forceinline__ void sum_runs(Shared& sh, const int (&base)[DIM], bool valid, Add direct) {
+  static __device__ __forceinline__ void sum_groups(Shared& sh, const int (&base)[DIM], bool valid, Add direct) {
     const int t = threadIdx.x, lane = t & 63;
-    bool head = lane == 0;
-    {
-      const int pv = __shfl_up(valid ? 1 : 0, 1);
-      head = head || (pv != 0) != valid;
-#pragma unroll
-      for (int d = 0; d < DIM; ++d) head = head || __shfl_up(base[d], 1) != base[d];
-    }
-    unsigned long long heads = __ballot(head);
-    const unsigned long long vmask = __ballot(valid);
+    unsigned long long left = __ballot(valid);
     constexpr int OUT = DIM == 3 ? 27 : NODES * NCH;
     const int sub = lane / OUT, o = lane - sub * OUT;  // sub 2: idle lanes
     const int node = DIM == 3 ? o : o % NODES;
@@ -124,28 +116,41 @@ template <typename T, int DIM, int NCH> struct CellSum {
     const int r0 = (on0 ? c0 : 0) * ROW, r1 = (on1 ? c0 + 1 : 0) * ROW;
     const int wi = NCH * ROW + i, wj = NCH * ROW + 3 + j, wk = NCH * ROW + (DIM == 3 ? 6 + k : 0);
     const bool arena = sh.box[DIM] > 0;
-    while (heads) {
-      const int s = __builtin_ctzll(heads);
-      heads &= heads - 1;
-      const int e = heads ? __builtin_ctzll(heads) : 64;
-      if (!((vmask >> s) & 1ull)) continue;
+    while (left) {
+      const int s = __builtin_ctzll(left);
+      int b[DIM];
+      bool same = valid;
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) {
+        b[d] = __builtin_amdgcn_readlane(base[d], s);
+        same = same && base[d] == b[d];
+      }
+      unsigned long long m = __ballot(same);
+      left &= ~m;
       T a0 = T(0), a1 = T(0);
-      const T* tab = sh.table + ((t & ~63) + s + (DIM == 2 ? sub : 0)) * ENTRY;
+      const T* wave = sh.table + (t & ~63) * ENTRY;
+      if constexpr (DIM == 3) {
 #pragma unroll 2
-      for (int p = s + (DIM == 2 ? sub : 0); p < e; p += GROUP, tab += GROUP * ENTRY) {
-        T w = tab[wi] * tab[wj];
-        if constexpr (DIM == 3) {
-          w *= tab[wk];
+        while (m) {
+          const T* tab = wave + __builtin_ctzll(m) * ENTRY;
+          m &= m - 1;
+          const T w = tab[wi] * tab[wj] * tab[wk];
           const Row3 q0 = *reinterpret_cast<const Row3*>(tab + r0), q1 = *reinterpret_cast<const Row3*>(tab + r1);
           a0 += w * (q0.x + q0.y * fi + q0.z * fj + q0.w * fk);
           a1 += w * (q1.x + q1.y * fi + q1.z * fj + q1.w * fk);
-        } else {
-          a0 += w * (tab[r0] + tab[r0 + 1] * fi + tab[r0 + 2] * fj);
+        }
+      } else {
+        while (m) {  // two particles at a time, one per group of lanes
+          const int p0 = __builtin_ctzll(m);
+          m &= m - 1;
+          const int p1 = m ? __builtin_ctzll(m) : -1;
+          m &= m - 1;
+          const int p = sub == 0 ? p0 : p1;
+          const T* tab = wave + (p < 0 ? p0 : p) * ENTRY;
+          const T v = tab[wi] * tab[wj] * (tab[r0] + tab[r0 + 1] * fi + tab[r0 + 2] * fj);
+          a0 += p < 0 ? T(0) : v;
         }
       }
-      int b[DIM];
-#pragma unroll
-      for (int d = 0; d < DIM; ++d) b[d] = __shfl(base[d], s);
       if (arena) {
         int at = (b[0] + i - sh.box[0]) * sh.box[DIM + 1] + (b[1] + j - sh.box[1]);
         if constexpr (DIM == 3) at = at * sh.box[DIM + 2] + (b[2] + k - sh.box[2]);
@@ -161,7 +166,7 @@ template <typename T, int DIM, int NCH> struct CellSum {
     }
   }
 
-  // After every wave's sum_runs: the arena's nonzero values to memory.
+  // After every wave's sum_groups: the arena's nonzero values to memory.
   template <typename Add> static __device__ __forceinline__ void flush(Shared& sh, Add add) {
     __syncthreads();
     const int n = volume(sh) * NCH;

@@ -173,7 +173,7 @@ __global__ __launch_bounds__(256) void phase_keys_kernel(const T* __restrict__ x
   keys[p] = (blk << 6) | cell;
 }
 
-// P2G of particles in cell order (perm), summed per cell run and workgroup
+// P2G of particles in cell order (perm), summed per cell and workgroup
 // before memory (mpm_cellsum.h).  At 131,072 FP64 particles in arbitrary
 // order on a 64^3 grid the per-particle scatter of phase_p2g_kernel issues
 // 14 million device atomics and takes 1,426 us; sort and sums together take
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(CELLSUM_THREADS) void phase_p2g_sorted_kernel(Phase
     else atomicAdd(a.grid_m + node, v);
   };
   Sum::prepare(sh, base, valid);
-  Sum::sum_runs(sh, base, valid, add);
+  Sum::sum_groups(sh, base, valid, add);
   Sum::flush(sh, add);
 }
 
