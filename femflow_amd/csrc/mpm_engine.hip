@@ -207,7 +207,7 @@ struct P2GTerms {
 // FP32 terms; false when the FP32 polar factor is not trustworthy (F near
 // singular or the iteration did not settle): the caller defers the particle.
 // P F^T = 2 mu (F - R) F^T + lam (J - 1) J (utils.py:120-135): the first
-// term from the series of stretch_series while F is within 3% of a
+// term from the series of stretch_series while F is within 15% of a
 // rotation (every snow particle after its clamp, and elastic ones under
 // moderate strain), else from the FP32 polar iteration.
 __device__ __forceinline__ bool p2g_terms(const SceneDev& sc, const MatParams& mp, float mass,
@@ -308,10 +308,15 @@ __device__ __forceinline__ void storek(float* f, int64_t p, const float o[K]) {
 __device__ __forceinline__ void load_record(const float4* __restrict__ rec, int64_t i, float x[3], float v[3],
                                             float F[9], float C[9], float& Jp, float& mass, float& mu0, float& lam0,
                                             uint32_t& attr) {
+  // vector loads as such: as float4 members the compiler may merge them with
+  // the tiled branch's loads of the same fields, one word at a time (the
+  // move of 2^20 particles 84 -> 108 us)
+  typedef float vec4 __attribute__((ext_vector_type(4)));
+  const vec4* r4 = reinterpret_cast<const vec4*>(rec) + i * (REC_WORDS / 4);
   float r[REC_WORDS];
 #pragma unroll
   for (int q = 0; q < REC_WORDS / 4; ++q) {
-    const float4 w = rec[i * (REC_WORDS / 4) + q];
+    const vec4 w = r4[q];
     r[4 * q] = w.x;
     r[4 * q + 1] = w.y;
     r[4 * q + 2] = w.z;
@@ -452,6 +457,14 @@ __device__ __forceinline__ int round_fixed(float w, float q) {
 // the particles into the new binned order), 1 = fused G2P + P2G, 2 = G2P
 // (the last substep of a run), 3 = the fused pass that also moves the
 // particles (the first substep after a rebin inside a run).
+// A value the compiler cannot see through: what is computed from it stays
+// where it is used, instead of being hoisted out of the chunk loop or kept
+// between its phases, where it would take registers from the particle phase.
+__device__ __forceinline__ int here(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
 // DYN: workgroups take their chunks from a per-XCD ticket queue instead of
 // a fixed interleave.  With tens of thousands of uneven chunks (many scenes
 // of different densities) the queue balances the tail; with a few thousand
@@ -518,7 +531,7 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
     const int bi = local / (nb * nb), bj = (local / nb) % nb, bk = local % nb;
     const int O0 = bi * 4 - 1, O1 = bj * 4 - 1, O2 = bk * 4 - 1;
     if constexpr (MODE != 0) {
-      for (int e = t; e < ARENA_NODES; e += ENG_THREADS) {
+      for (int e = here(t); e < ARENA_NODES; e += ENG_THREADS) {
         const int gi = O0 + (e >> 6), gj = O1 + ((e >> 3) & 7), gk = O2 + (e & 7);
         const bool in = gi >= 0 && gj >= 0 && gk >= 0 && gi <= sc.res && gj <= sc.res && gk <= sc.res;
         vel_s[(e >> 6) * VEL_S0 + ((e >> 3) & 7) * VEL_S1 + (e & 7)] =
@@ -707,7 +720,7 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
         if (lane == 0) red_s[wv][d] = m;
       }
       __syncthreads();
-      for (int e = t; e < 2 * ACC_NODES; e += ENG_THREADS) acc2[0][e] = 0ull;
+      for (int e = here(t); e < 2 * ACC_NODES; e += ENG_THREADS) acc2[0][e] = 0ull;
       if (t < 4) {
         float m = 0.f;
 #pragma unroll
@@ -811,7 +824,7 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
       const bool staged = c < a.stage_cap;
       float4* stage = a.stage + (size_t)c * STAGE_REC;
 #pragma unroll 1
-      for (int e = t; e < ARENA_NODES; e += ENG_THREADS) {
+      for (int e = here(t); e < ARENA_NODES; e += ENG_THREADS) {
         const int e0 = e >> 6, e1 = (e >> 3) & 7, e2 = e & 7;
         const int ph = e0 * ACC_S0 + e1 * ACC_S1 + e2;
         int q0, q1, q2, q3;
@@ -1925,7 +1938,7 @@ void Engine::enqueue_bin(hipStream_t s, int len, int with_sums) {
   pending_perm = vs;
   hipLaunchKernelGGL(block_bounds_kernel, dim3(nblk(n, 256)), dim3(256), 0, s, ks, n, d_bstart, d_bend, d_bocc);
   chunk_list(d_bocc, d_bstart, d_bend, d_block_scene, (int64_t)total_blocks, chunk, d_part, d_chunks, d_bfirst,
-             d_bcount, d_nchunks, s);
+             d_bcount, d_nchunks, dyn_sched, s);
   d_sorted_keys = ks;
   hipLaunchKernelGGL(cand_build_kernel, dim3(num_cus * 2), dim3(256), 0, s, args(nullptr, 0, 0), d_cand_list,
                      d_counters + 4, d_cand_flag);

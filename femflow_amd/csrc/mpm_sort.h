@@ -11,15 +11,15 @@ namespace mpm {
 size_t radix_workspace_bytes(int64_t n);
 int radix_passes(uint32_t max_key);
 // Chunk list of a binning: occupied block b (bocc[b] != 0, particles
-// bstart[b] .. bend[b]) gets ceil(count / chunk) chunks of nearly equal size
-// (start, count, b, block_scene[b]), numbered after those of the blocks
+// bstart[b] .. bend[b]) gets chunks of at most `chunk` particles (a multiple
+// of 256; start, count, b, block_scene[b]), numbered after those of the blocks
 // before it; bfirst[b]
 // and bcount[b] are its first chunk and chunk count (0 for empty blocks);
-// *nchunks = the total.  part: chunk_list_part_words(nblocks) words.
+// *nchunks = the total.  plain: equal chunks (see FEW_ROWS).  part: chunk_list_part_words(nblocks) words.
 size_t chunk_list_part_words(int64_t nblocks);
 void chunk_list(const uint32_t* bocc, const uint32_t* bstart, const uint32_t* bend, const int* block_scene,
                 int64_t nblocks, int chunk, uint32_t* part, int4* chunks, uint32_t* bfirst, uint32_t* bcount,
-                uint32_t* nchunks, hipStream_t st);
+                uint32_t* nchunks, bool plain, hipStream_t st);
 // Tiles of the sort (one workgroup each) and the first pass's tile
 // histogram inside the workspace, for a key kernel that also counts the
 // first digit (rs_tile_histogram, mpm_sort_dev.h) and passes

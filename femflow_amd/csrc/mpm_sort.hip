@@ -190,55 +190,109 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
 }
 
 // ------------------------------------------------------- chunk list ----
-// Chunk list of the new binning, numbered over blocks: block b holds
-// ceil(count_b / chunk) chunks of nearly equal size, numbered after those
-// of the blocks before it.  Two launches over tiles of SCAN_THREADS blocks, one block per thread
-// (coalesced reads, a few hundred tiles for a 128^3 grid): per-tile chunk
-// counts, then each tile adds the counts of the tiles before it, scans its
-// own blocks and writes their chunks, first chunk and chunk count.
-__device__ __forceinline__ uint32_t block_chunks(const uint32_t* __restrict__ bocc,
-                                                 const uint32_t* __restrict__ bstart,
-                                                 const uint32_t* __restrict__ bend, int64_t b, int chunk) {
-  return bocc[b] ? (bend[b] - bstart[b] + (uint32_t)chunk - 1u) / (uint32_t)chunk : 0u;
+// Chunk list of the new binning, numbered over blocks.  A transfer workgroup
+// works through a chunk in rows of CHUNK_ROW particles, one per thread, so a
+// block's particles are cut into R = ceil(count / CHUNK_ROW) rows of nearly
+// equal size first (chunks of 333 would take two rows each for the work of
+// 1.3).  Either every row is a chunk, or the rows of a block are grouped into
+// chunks of up to `chunk` particles: a row by itself finishes sooner and
+// leaves a shorter tail; a pair loads and stages one arena for both and
+// spreads a wave's lanes over twice as many cells, which is what counts where
+// a cell holds dozens of particles (the lanes that share one add to the same
+// words).  One choice for the whole list: chunks of one and of two rows side
+// by side were the slowest (2^20 particles 5,464 us, see below).  Two launches
+// over tiles of SCAN_THREADS blocks, one block per thread (coalesced reads,
+// a few hundred tiles for a 128^3 grid): per-tile counts, then each tile adds
+// the counts of the tiles before it, scans its own blocks and writes their
+// chunks, first chunk and chunk count.
+constexpr uint32_t CHUNK_ROW = 256;
+// Rows are grouped where most of them are in blocks of more than 18 particles
+// per cell.  48 substeps, all rows single / grouped, in us: 100,003 particles
+// at 17 per cell 1,500 / 1,723; 400,000 at 17 2,839 / 2,978; 524,288 at 10
+// 3,425 / 3,908; 262,144 at 21 2,210 / 2,118; 2^20 at 21 5,581 / 5,164;
+// 131,072 at 62 1,744 / 1,638.
+constexpr uint32_t GROUP_ABOVE = 18 * 64;
+// And single up to this many rows in all, one and a half per compute unit of
+// an MI355X: fewer, larger chunks would leave units without one (16,384
+// particles at 8 per cell 1,035 / 1,230).
+// Engines of many scenes (plain) cut a block into ceil(count / chunk) equal
+// chunks, without regard to rows: their tens of thousands of chunks come from
+// contended ticket queues, and single rows cost more there (64 scenes, 24
+// substeps with upload and download: 16,112 single, 14,827 rows grouped,
+// 15,160 plain; grouping moves the fixed-point scale of scenes with a fraction
+// of a particle per cell, whose light nodes it then decides).
+constexpr uint32_t FEW_ROWS = 384;
+
+// Of a block (or their sums over a tile): rows, chunks with rows grouped, rows
+// in dense blocks.  A block's pairs that would be less than 3/4 full stay
+// single (260 particles: 130 + 130, not 256 + 4).
+struct BlockRows {
+  uint32_t rows, chunks, dense;
+};
+__device__ __forceinline__ BlockRows block_rows(const uint32_t* __restrict__ bocc, const uint32_t* __restrict__ bstart,
+                                                const uint32_t* __restrict__ bend, int64_t b, uint32_t per_chunk,
+                                                int plain) {
+  if (!bocc[b]) return {0u, 0u, 0u};
+  const uint32_t cnt = bend[b] - bstart[b], rows = (cnt + CHUNK_ROW - 1u) / CHUNK_ROW;
+  if (plain) {
+    const uint32_t c = (cnt + per_chunk * CHUNK_ROW - 1u) / (per_chunk * CHUNK_ROW);
+    return {c, c, 0u};
+  }
+  const bool group = 4u * cnt >= 3u * CHUNK_ROW * rows;
+  return {rows, group ? (rows + per_chunk - 1u) / per_chunk : rows, cnt > GROUP_ABOVE ? rows : 0u};
 }
 
 __global__ __launch_bounds__(SCAN_THREADS) void block_tile_kernel(const uint32_t* __restrict__ bocc,
                                                                   const uint32_t* __restrict__ bstart,
                                                                   const uint32_t* __restrict__ bend,
-                                                                  int64_t nblocks, int chunk,
-                                                                  uint32_t* __restrict__ part) {
+                                                                  int64_t nblocks, uint32_t per_chunk,
+                                                                  uint4* __restrict__ part, int plain) {
   __shared__ uint32_t sh[SCAN_THREADS];
   const int64_t b = (int64_t)blockIdx.x * SCAN_THREADS + threadIdx.x;
-  const uint32_t c = b < nblocks ? block_chunks(bocc, bstart, bend, b, chunk) : 0u;
-  uint32_t tot;
-  block_exclusive_scan(c, sh, &tot);
-  if (threadIdx.x == 0) part[blockIdx.x] = tot;
+  const BlockRows r = b < nblocks ? block_rows(bocc, bstart, bend, b, per_chunk, plain) : BlockRows{0u, 0u, 0u};
+  uint32_t rows, chunks, dense;
+  block_exclusive_scan(r.rows, sh, &rows);
+  block_exclusive_scan(r.chunks, sh, &chunks);
+  block_exclusive_scan(r.dense, sh, &dense);
+  if (threadIdx.x == 0) part[blockIdx.x] = make_uint4(rows, chunks, dense, 0u);
 }
 
 __global__ __launch_bounds__(SCAN_THREADS) void block_chunks_kernel(
     const uint32_t* __restrict__ bocc, const uint32_t* __restrict__ bstart, const uint32_t* __restrict__ bend,
-    const int* __restrict__ block_scene, int64_t nblocks, int chunk, const uint32_t* __restrict__ part,
+    const int* __restrict__ block_scene, int64_t nblocks, uint32_t per_chunk, const uint4* __restrict__ part,
     int4* __restrict__ chunks, uint32_t* __restrict__ bfirst, uint32_t* __restrict__ bcount,
-    uint32_t* __restrict__ nchunks) {
+    uint32_t* __restrict__ nchunks, int plain) {
   __shared__ uint32_t sh[SCAN_THREADS];
-  uint32_t before = 0;
-  for (uint32_t q = threadIdx.x; q < blockIdx.x; q += SCAN_THREADS) before += part[q];
-  uint32_t tot_before;
-  block_exclusive_scan(before, sh, &tot_before);
+  uint32_t rows_before = 0, chunks_before = 0, rows = 0, dense = 0;
+  for (uint32_t q = threadIdx.x; q < gridDim.x; q += SCAN_THREADS) {
+    const uint4 v = part[q];
+    rows += v.x;
+    dense += v.z;
+    if (q < blockIdx.x) {
+      rows_before += v.x;
+      chunks_before += v.y;
+    }
+  }
+  uint32_t rows_all, dense_all, before;
+  block_exclusive_scan(rows, sh, &rows_all);
+  block_exclusive_scan(dense, sh, &dense_all);
+  // the same in every workgroup
+  const bool single = !plain && (rows_all <= FEW_ROWS || 2u * dense_all < rows_all);
+  block_exclusive_scan(single ? rows_before : chunks_before, sh, &before);
   const int64_t b = (int64_t)blockIdx.x * SCAN_THREADS + threadIdx.x;
-  const uint32_t c = b < nblocks ? block_chunks(bocc, bstart, bend, b, chunk) : 0u;
+  const BlockRows r = b < nblocks ? block_rows(bocc, bstart, bend, b, per_chunk, plain) : BlockRows{0u, 0u, 0u};
+  const uint32_t c = single ? r.rows : r.chunks;
   uint32_t tot;
-  const uint32_t run = block_exclusive_scan(c, sh, &tot) + tot_before;
+  const uint32_t run = block_exclusive_scan(c, sh, &tot) + before;
   if (b < nblocks) {
     bfirst[b] = run;
     bcount[b] = c;
     if (c) {
       const uint32_t p0 = bstart[b], cnt = bend[b] - p0;
       const int sc = block_scene[b];
-      // c chunks of (nearly) equal size rather than full ones and a
-      // remainder: less spread in per-chunk work, a shorter tail
       for (uint32_t j = 0; j < c; ++j) {
-        const uint32_t s0 = (uint32_t)(((uint64_t)cnt * j) / c), s1 = (uint32_t)(((uint64_t)cnt * (j + 1)) / c);
+        const uint32_t r0 = r.rows * j / c, r1 = r.rows * (j + 1u) / c;  // its rows
+        const uint32_t s0 = (uint32_t)(((uint64_t)cnt * r0) / r.rows), s1 = (uint32_t)(((uint64_t)cnt * r1) / r.rows);
         chunks[run + j] = make_int4((int)(p0 + s0), (int)(s1 - s0), (int)b, sc);
       }
     }
@@ -292,17 +346,19 @@ size_t radix_workspace_bytes(int64_t n) {
   return sizeof(uint32_t) * (4 * (size_t)n + 2 * (size_t)(hist > n ? hist : n) + RS_BINS + 64);
 }
 
-size_t chunk_list_part_words(int64_t nblocks) { return (size_t)cdiv(nblocks, SCAN_THREADS) + 1; }
+size_t chunk_list_part_words(int64_t nblocks) { return 4 * ((size_t)cdiv(nblocks, SCAN_THREADS) + 1); }
 
 void chunk_list(const uint32_t* bocc, const uint32_t* bstart, const uint32_t* bend, const int* block_scene,
                 int64_t nblocks, int chunk, uint32_t* part, int4* chunks, uint32_t* bfirst, uint32_t* bcount,
-                uint32_t* nchunks, hipStream_t st) {
+                uint32_t* nchunks, bool plain, hipStream_t st) {
   if (nblocks <= 0) return;
   const unsigned tiles = (unsigned)cdiv(nblocks, SCAN_THREADS);
+  const uint32_t per_chunk = (uint32_t)chunk / CHUNK_ROW;
+  uint4* part4 = reinterpret_cast<uint4*>(part);
   hipLaunchKernelGGL(block_tile_kernel, dim3(tiles), dim3(SCAN_THREADS), 0, st, bocc, bstart, bend, nblocks,
-                     chunk, part);
+                     per_chunk, part4, plain ? 1 : 0);
   hipLaunchKernelGGL(block_chunks_kernel, dim3(tiles), dim3(SCAN_THREADS), 0, st, bocc, bstart, bend,
-                     block_scene, nblocks, chunk, part, chunks, bfirst, bcount, nchunks);
+                     block_scene, nblocks, per_chunk, part4, chunks, bfirst, bcount, nchunks, plain ? 1 : 0);
 }
 
 int radix_passes(uint32_t max_key) {
