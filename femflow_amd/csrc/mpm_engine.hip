@@ -207,7 +207,7 @@ struct P2GTerms {
 // FP32 terms; false when the FP32 polar factor is not trustworthy (F near
 // singular or the iteration did not settle): the caller defers the particle.
 // P F^T = 2 mu (F - R) F^T + lam (J - 1) J (utils.py:120-135): the first
-// term from the series of stretch_series while F is within 15% of a
+// term from the series of stretch_series while F is within 3% of a
 // rotation (every snow particle after its clamp, and elastic ones under
 // moderate strain), else from the FP32 polar iteration.
 __device__ __forceinline__ bool p2g_terms(const SceneDev& sc, const MatParams& mp, float mass,

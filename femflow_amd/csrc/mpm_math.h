@@ -253,17 +253,12 @@ template <typename T> MPM_DEV T det3_minus_one(const T* F) {
 // R F^T = U S U^T = sqrt(B), B = F F^T, for either sign of det F, so
 // (F - R) F^T = B - sqrt(B).  With E = B - I = D + D^T + D D^T (D = F - I),
 //   B - sqrt(B) = E/2 + E^2/8 - E^3/16 + 5 E^4/128 - 7 E^5/256 + ...
-// (the binomial series of sqrt(I + E), which converges for ||E|| < 1).
-// By Cayley-Hamilton (E^3 = I1 E^2 - I2 E + I3 I) every partial sum is
-// a0 I + a1 E + a2 E^2, and one Horner step costs three FMAs on the a's
-// instead of a symmetric matrix product (thirty): twelve terms and the
-// invariants take about 110 instructions, where five terms with matrix
-// products took 195 and reached ||E||_F = 0.06, beyond which (strains of 3%)
-// a polar iteration of over 200 had to run.  Twelve terms leave a truncation
-// below 1e-8 of the result for ||E||_F <= 0.3 (strains up to 15%); in FP32
-// the error is that of E's rounding, 6e-8 relative where the rotation is
-// small, as with five terms (FP64 comparison over strains of 1e-4 to 0.12).
-// Out: the symmetric result as (00, 01, 02, 11, 12, 22).
+// (the binomial series of sqrt(I + E), which converges for ||E|| < 1).  Five
+// terms leave a relative error below 4e-8 while ||E||_F <= 0.06 (FP64
+// check against the SVD form: 1e-8 at 0.05, 4e-8 at 0.06); beyond that the
+// caller takes the polar iteration.  Out: the symmetric result as
+// (00, 01, 02, 11, 12, 22).  All products are of commuting symmetric
+// matrices (polynomials in E), so each stays symmetric.
 template <typename T> MPM_DEV bool stretch_series(const T* F, T out[6]) {
   const T D[9] = {F[0] - T(1), F[1], F[2], F[3], F[4] - T(1), F[5], F[6], F[7], F[8] - T(1)};
   T E[6];
@@ -273,44 +268,30 @@ template <typename T> MPM_DEV bool stretch_series(const T* F, T out[6]) {
   E[3] = T(2) * D[4] + (D[3] * D[3] + D[4] * D[4] + D[5] * D[5]);
   E[4] = (D[5] + D[7]) + (D[3] * D[6] + D[4] * D[7] + D[5] * D[8]);
   E[5] = T(2) * D[8] + (D[6] * D[6] + D[7] * D[7] + D[8] * D[8]);
-  // E^2 (its trace is ||E||_F^2) and the invariants
-  const T q01 = E[1] * E[1], q02 = E[2] * E[2], q12 = E[4] * E[4];
-  const T S00 = E[0] * E[0] + q01 + q02, S11 = q01 + E[3] * E[3] + q12, S22 = q02 + q12 + E[5] * E[5];
-  if (!(S00 + S11 + S22 <= T(0.09))) return false;  // also NaN
-  const T S01 = E[0] * E[1] + E[1] * E[3] + E[2] * E[4];
-  const T S02 = E[0] * E[2] + E[1] * E[4] + E[2] * E[5];
-  const T S12 = E[1] * E[2] + E[3] * E[4] + E[4] * E[5];
-  const T m0 = E[3] * E[5] - q12;
-  const T I1 = E[0] + E[3] + E[5];
-  const T I2 = m0 + (E[0] * E[5] - q02) + (E[0] * E[3] - q01);
-  const T I3 = E[0] * m0 - E[1] * (E[1] * E[5] - E[4] * E[2]) + E[2] * (E[1] * E[4] - E[3] * E[2]);
-  constexpr int N = 12;
-  constexpr double c[N] = {0.5,
-                           0.125,
-                           -0.0625,
-                           0.0390625,
-                           -0.02734375,
-                           0.0205078125,
-                           -0.01611328125,
-                           0.013092041015625,
-                           -0.0109100341796875,
-                           0.009273529052734375,
-                           -0.0080089569091796875,
-                           0.00700783729553222656};
-  T a0 = T(c[N - 1]), a1 = T(0), a2 = T(0);
+  const T fro2 = E[0] * E[0] + E[3] * E[3] + E[5] * E[5] + T(2) * (E[1] * E[1] + E[2] * E[2] + E[4] * E[4]);
+  if (!(fro2 <= T(0.0036))) return false;  // also NaN
+  // Horner: S <- E S + c I from S = c5 I, then out = E S
+  const T c[5] = {T(0.5), T(0.125), T(-0.0625), T(0.0390625), T(-0.02734375)};
+  T S[6] = {c[4], T(0), T(0), c[4], T(0), c[4]};
 #pragma unroll
-  for (int k = N - 2; k >= -1; --k) {
-    const T b0 = I3 * a2 + (k >= 0 ? T(c[k]) : T(0)), b1 = a0 - I2 * a2, b2 = a1 + I1 * a2;
-    a0 = b0;
-    a1 = b1;
-    a2 = b2;
+  for (int k = 3; k >= -1; --k) {
+    T P[6];
+    P[0] = E[0] * S[0] + E[1] * S[1] + E[2] * S[2];
+    P[1] = E[0] * S[1] + E[1] * S[3] + E[2] * S[4];
+    P[2] = E[0] * S[2] + E[1] * S[4] + E[2] * S[5];
+    P[3] = E[1] * S[1] + E[3] * S[3] + E[4] * S[4];
+    P[4] = E[1] * S[2] + E[3] * S[4] + E[4] * S[5];
+    P[5] = E[2] * S[2] + E[4] * S[4] + E[5] * S[5];
+    if (k >= 0) {
+      P[0] += c[k];
+      P[3] += c[k];
+      P[5] += c[k];
+    }
+#pragma unroll
+    for (int i = 0; i < 6; ++i) S[i] = P[i];
   }
-  out[0] = a0 + (a1 * E[0] + a2 * S00);
-  out[1] = a1 * E[1] + a2 * S01;
-  out[2] = a1 * E[2] + a2 * S02;
-  out[3] = a0 + (a1 * E[3] + a2 * S11);
-  out[4] = a1 * E[4] + a2 * S12;
-  out[5] = a0 + (a1 * E[5] + a2 * S22);
+#pragma unroll
+  for (int i = 0; i < 6; ++i) out[i] = S[i];
   return true;
 }
 
