@@ -22,12 +22,13 @@ MPM_KEY_BLOCKED, MPM_KEY_ROWMAJOR = 0, 1
 
 # every symbol include/mpm355.h declares (checked by the CPU test suite)
 EXPORTS = (
-    "mpm_last_error_string", "mpm_version", "mpm_device_count", "mpm_p2g", "mpm_p2g_workspace_bytes", "mpm_p2g_ws", "mpm_grid_op",
+    "mpm_last_error_string", "mpm_version", "mpm_device_count", "mpm_p2g", "mpm_p2g_workspace_bytes", "mpm_p2g_ws",
+    "mpm_p2g_uniform", "mpm_count_oob", "mpm_grid_op",
     "mpm_g2p", "mpm_ctx_create", "mpm_ctx_destroy", "mpm_ctx_set_stream", "mpm_ctx_tune", "mpm_ctx_set_spread",
     "mpm_ctx_kernel_timing", "mpm_ctx_kernel_times", "mpm_state_upload", "mpm_state_download",
     "mpm_run", "mpm_run_frames", "mpm_run_states", "mpm_run_states_grids", "mpm_state_positions", "mpm_substep", "mpm_ctx_oob_count", "mpm_ctx_fallback_count",
     "mpm_ctx_active_blocks", "mpm_ctx_request_rebin",
-    "mpm_particle_sums", "mpm_bin", "mpm_bin_noalloc", "mpm_dense_workspace_bytes", "mpm_dense_substep", "mpm_adjoint_step",
+    "mpm_particle_sums", "mpm_bin", "mpm_bin_workspace_bytes", "mpm_bin_ws", "mpm_bin_noalloc", "mpm_dense_workspace_bytes", "mpm_dense_substep", "mpm_adjoint_step",
     "mpm_adjoint_step_grids",
     "mpm_ctx_set_corrector", "mpm_corrector_sample", "mpm_grid_velocity",
     "mpm_collide_planes", "mpm_ctx_set_planes",
@@ -90,6 +91,8 @@ def load():
             "mpm_p2g": ([vp, Q, P, i32, dbl, M, i32, vp, vp, vp], i32),
             "mpm_p2g_workspace_bytes": ([Q, i64, ct.POINTER(i64)], i32),
             "mpm_p2g_ws": ([vp, Q, P, i32, dbl, M, i32, vp, vp, vp, vp, i64], i32),
+            "mpm_p2g_uniform": ([vp, Q, P, i32, dbl, dbl, dbl, dbl, vp, vp, vp, i64], i32),
+            "mpm_count_oob": ([vp, Q, P, vp], i32),
             "mpm_grid_op": ([vp, Q, i32, vp, vp], i32),
             "mpm_collide_planes": ([vp, i32, i32, dbl, i32, vp, vp, i32, vp], i32),
             "mpm_ctx_set_planes": ([vp, i32, i32, vp, vp, i32], i32),
@@ -115,6 +118,8 @@ def load():
             "mpm_ctx_request_rebin": ([vp], i32),
             "mpm_particle_sums": ([vp, ct.POINTER(dbl)], i32),
             "mpm_bin": ([vp, i32, i32, dbl, i32, vp, i64, vp, vp], i32),
+            "mpm_bin_workspace_bytes": ([i64, ct.POINTER(i64)], i32),
+            "mpm_bin_ws": ([vp, i32, i32, dbl, i32, vp, i64, vp, vp, vp, i64], i32),
             "mpm_bin_noalloc": ([vp, i32, i32, dbl, i32, vp, i64, vp, vp], i32),
             "mpm_dense_workspace_bytes": ([Q, ct.POINTER(i64)], i32),
             "mpm_dense_substep": ([vp, Q, P, dbl, vp, vp], i32),

@@ -67,9 +67,10 @@ int32_t mpm_device_count(void) {
 
 static int p2g_call(void* stream, const mpm_params* prm, const mpm_particles* p, int32_t kind_override,
                     double hardening, const mpm_material* materials, int32_t nmat, void* grid_v, void* grid_m,
-                    int64_t* oob_count, void* work, int64_t work_bytes, const char* fn) {
+                    int64_t* oob_count, void* work, int64_t work_bytes, const char* fn,
+                    const double* uniform = nullptr) {
   int rc;
-  if ((rc = check_params(prm, fn)) || (rc = check_particles(p, fn, true))) return rc;
+  if ((rc = check_params(prm, fn)) || (rc = check_particles(p, fn, !uniform))) return rc;
   if (!grid_v || !grid_m) {
     set_error(std::string(fn) + ": null grid");
     return MPM_ERR_ARG;
@@ -81,7 +82,7 @@ static int p2g_call(void* stream, const mpm_params* prm, const mpm_particles* p,
   const size_t need = mpm::phase_p2g_workspace_bytes(prm, p->n);
   if (need == 0 || work_bytes < (int64_t)need) work = nullptr;
   mpm::phase_p2g((hipStream_t)stream, prm, p, kind_override, hardening, materials, nmat, grid_v,
-                 grid_m, (unsigned long long*)oob_count, work);
+                 grid_m, (unsigned long long*)oob_count, work, uniform);
   CHECK_HIP(hipGetLastError());
   return MPM_OK;
 }
@@ -109,6 +110,30 @@ int32_t mpm_p2g_ws(void* stream, const mpm_params* prm, const mpm_particles* p, 
                    int64_t* oob_count, void* work, int64_t work_bytes) {
   return p2g_call(stream, prm, p, kind_override, hardening, materials, nmat, grid_v, grid_m, oob_count, work,
                   work_bytes, "mpm_p2g_ws");
+}
+
+int32_t mpm_p2g_uniform(void* stream, const mpm_params* prm, const mpm_particles* p, int32_t kind, double hardening,
+                        double mass, double mu0, double lambda0, void* grid_v, void* grid_m, void* work,
+                        int64_t work_bytes) {
+  if (kind < 0) {
+    set_error("mpm_p2g_uniform: needs a material kind");
+    return MPM_ERR_ARG;
+  }
+  const double uniform[3] = {mass, mu0, lambda0};
+  return p2g_call(stream, prm, p, kind, hardening, nullptr, 0, grid_v, grid_m, nullptr, work, work_bytes,
+                  "mpm_p2g_uniform", uniform);
+}
+
+int32_t mpm_count_oob(void* stream, const mpm_params* prm, const mpm_particles* p, int64_t* oob_count) {
+  int rc;
+  if ((rc = check_params(prm, "mpm_count_oob"))) return rc;
+  if (!p || p->n < 0 || (p->dtype != MPM_F32 && p->dtype != MPM_F64) || (p->n > 0 && !p->x) || !oob_count) {
+    set_error("mpm_count_oob: null positions or counter, n < 0 or a bad dtype");
+    return MPM_ERR_ARG;
+  }
+  mpm::phase_oob((hipStream_t)stream, prm, p, (unsigned long long*)oob_count);
+  CHECK_HIP(hipGetLastError());
+  return MPM_OK;
 }
 
 static int check_dense(const mpm_params* prm, const mpm_particles* p, const void* work, const char* fn) {
@@ -569,44 +594,77 @@ int32_t mpm_particle_sums(mpm_ctx* ctx, double* out) {
   return ctx->eng.particle_sums(out);
 }
 
-int32_t mpm_bin(mpm_ctx* ctx, int32_t dim, int32_t res, double inv_dx, int32_t layout, const float* x,
-                int64_t n, uint32_t* keys, uint32_t* perm) {
-  (void)ctx;
+// Largest key of a binning, or a message why there is none.
+static const char* bin_key_space(int32_t dim, int32_t res, int32_t layout, const float* x, int64_t n,
+                                 const uint32_t* keys, const uint32_t* perm, uint32_t* max_key) {
   if ((dim != 2 && dim != 3) || res < 1 || res > 4096 || n < 0 || (n > 0 && (!x || !keys || !perm)) ||
-      (layout != MPM_KEY_BLOCKED && layout != MPM_KEY_ROWMAJOR)) {
-    set_error("mpm_bin: bad argument");
+      (layout != MPM_KEY_BLOCKED && layout != MPM_KEY_ROWMAJOR))
+    return "bad argument";
+  const uint64_t r1 = (uint64_t)res + 1, nb = (r1 + 3) / 4;
+  uint64_t m;
+  if (layout == MPM_KEY_ROWMAJOR) m = dim == 3 ? r1 * r1 * r1 - 1 : r1 * r1 - 1;
+  else m = dim == 3 ? nb * nb * nb * 64 - 1 : nb * nb * 16 - 1;
+  if (n > 0 && m >= (1ull << 32)) return "key space exceeds 32 bits";
+  *max_key = (uint32_t)m;
+  return nullptr;
+}
+
+// Words of the sort's copy of the keys, ahead of its own workspace.
+static size_t bin_keys_words(int64_t n) { return ((size_t)n + 63) & ~(size_t)63; }
+
+static void bin_on(hipStream_t st, int32_t dim, int32_t res, double inv_dx, int32_t layout, const float* x, int64_t n,
+                   uint32_t max_key, uint32_t* keys, uint32_t* perm, uint32_t* work) {
+  uint32_t *ks, *vs;
+  mpm::bin_keys(x, n, dim, res, (float)inv_dx, layout, keys, st);
+  hipMemcpyAsync(work, keys, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st);
+  mpm::radix_sort(work, perm, n, max_key, work + bin_keys_words(n), true, &ks, &vs, st);
+  if (vs != perm) hipMemcpyAsync(perm, vs, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st);
+}
+
+int32_t mpm_bin_workspace_bytes(int64_t n, int64_t* bytes) {
+  if (!bytes || n < 0) {
+    set_error("mpm_bin_workspace_bytes: null output or n < 0");
+    return MPM_ERR_ARG;
+  }
+  *bytes = (int64_t)(sizeof(uint32_t) * bin_keys_words(n) + mpm::radix_workspace_bytes(n));
+  return MPM_OK;
+}
+
+int32_t mpm_bin_ws(void* stream, int32_t dim, int32_t res, double inv_dx, int32_t layout, const float* x, int64_t n,
+                   uint32_t* keys, uint32_t* perm, void* work, int64_t work_bytes) {
+  uint32_t max_key;
+  if (const char* why = bin_key_space(dim, res, layout, x, n, keys, perm, &max_key)) {
+    set_error(std::string("mpm_bin_ws: ") + why);
     return MPM_ERR_ARG;
   }
   if (n == 0) return MPM_OK;
-  const uint64_t r1 = (uint64_t)res + 1;
-  uint64_t max_key;
-  if (layout == MPM_KEY_ROWMAJOR) {
-    max_key = dim == 3 ? r1 * r1 * r1 - 1 : r1 * r1 - 1;
-  } else {
-    const uint64_t nb = (r1 + 3) / 4;
-    max_key = dim == 3 ? nb * nb * nb * 64 - 1 : nb * nb * 16 - 1;
-  }
-  if (max_key >= (1ull << 32)) {
-    set_error("mpm_bin: key space exceeds 32 bits");
+  int64_t need;
+  mpm_bin_workspace_bytes(n, &need);
+  if (!work || work_bytes < need) {
+    set_error("mpm_bin_ws: workspace missing or too small");
     return MPM_ERR_ARG;
   }
-  hipStream_t st = nullptr;
-  mpm::bin_keys(x, n, dim, res, (float)inv_dx, layout, keys, st);
-  uint32_t* tmp = nullptr;
-  void* ws = nullptr;
-  CHECK_HIP(hipMalloc(&tmp, sizeof(uint32_t) * n));
-  if (hipMalloc(&ws, mpm::radix_workspace_bytes(n)) != hipSuccess) {
-    hipFree(tmp);
-    set_error("mpm_bin: workspace allocation failed");
-    return MPM_ERR_HIP;
+  bin_on((hipStream_t)stream, dim, res, inv_dx, layout, x, n, max_key, keys, perm, (uint32_t*)work);
+  CHECK_HIP(hipGetLastError());
+  return MPM_OK;
+}
+
+int32_t mpm_bin(mpm_ctx* ctx, int32_t dim, int32_t res, double inv_dx, int32_t layout, const float* x,
+                int64_t n, uint32_t* keys, uint32_t* perm) {
+  (void)ctx;
+  uint32_t max_key;
+  if (const char* why = bin_key_space(dim, res, layout, x, n, keys, perm, &max_key)) {
+    set_error(std::string("mpm_bin: ") + why);
+    return MPM_ERR_ARG;
   }
-  hipMemcpyAsync(tmp, keys, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st);
-  uint32_t *ks, *vs;
-  mpm::radix_sort(tmp, perm, n, (uint32_t)max_key, ws, true, &ks, &vs, st);
-  if (vs != perm) hipMemcpyAsync(perm, vs, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st);
-  hipError_t e = hipStreamSynchronize(st);
-  hipFree(tmp);
-  hipFree(ws);
+  if (n == 0) return MPM_OK;
+  int64_t bytes;
+  mpm_bin_workspace_bytes(n, &bytes);
+  void* work = nullptr;
+  CHECK_HIP(hipMalloc(&work, (size_t)bytes));
+  bin_on(nullptr, dim, res, inv_dx, layout, x, n, max_key, keys, perm, (uint32_t*)work);
+  hipError_t e = hipStreamSynchronize(nullptr);
+  hipFree(work);
   if (e != hipSuccess) {
     set_error(std::string("mpm_bin: ") + hipGetErrorString(e));
     return MPM_ERR_HIP;

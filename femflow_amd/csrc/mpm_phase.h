@@ -12,7 +12,8 @@ namespace mpm {
 
 void phase_p2g(hipStream_t st, const mpm_params* prm, const mpm_particles* p, int kind_override,
                double hardening, const mpm_material* mats, int nmat, void* gv, void* gm,
-               unsigned long long* oob, void* work = nullptr);
+               unsigned long long* oob, void* work = nullptr, const double* uniform = nullptr);
+void phase_oob(hipStream_t st, const mpm_params* prm, const mpm_particles* p, unsigned long long* oob);
 size_t phase_p2g_workspace_bytes(const mpm_params* prm, int64_t n);
 void phase_grid_op(hipStream_t st, const mpm_params* prm, int dtype, void* gv, const void* gm);
 void phase_planes(hipStream_t st, int dtype, int res, const PlaneDev* planes, int n, void* gv);

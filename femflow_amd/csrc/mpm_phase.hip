@@ -12,8 +12,9 @@ namespace mpm {
 
 template <typename T> struct PhaseArgs {
   int64_t n;
-  int res, quirks, boundary, bound, mat_scalar, kind_override;
+  int res, quirks, boundary, bound, mat_scalar, kind_override, uniform;
   T inv_dx, dx, dt, vol, gravity, hardening, theta_c, theta_s;
+  T mass1, mu1, lam1;  // every particle's, when uniform
   T* x;
   T* v;
   T* F;
@@ -49,6 +50,20 @@ __device__ __forceinline__ void material_of(const PhaseArgs<T>& a, int64_t p, in
   ts = (T)m.theta_s;
 }
 
+template <typename T>
+__device__ __forceinline__ void constants_of(const PhaseArgs<T>& a, int64_t p, T& m, T& mu0, T& lam0) {
+  if (a.uniform) {
+    m = a.mass1;
+    mu0 = a.mu1;
+    lam0 = a.lam1;
+    return;
+  }
+  const int64_t i = a.mat_scalar ? 0 : p;
+  m = a.mass[i];
+  mu0 = a.mu0[i];
+  lam0 = a.lam0[i];
+}
+
 // base = trunc(x inv_dx - 0.5) (three_d/p2g.py:50) with the stencil inside
 // [0, R] (utils.py:138-150): valid iff -1 < x inv_dx - 0.5 < R - 1.
 template <typename T, int DIM>
@@ -57,7 +72,7 @@ __device__ __forceinline__ bool locate(const T* xp, T inv_dx, int res, int base[
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
     const T s = xp[d] * inv_dx;
-    const T t = s - T(0.5);
+    const T t = fma(xp[d], inv_dx, T(-0.5));  // one rounding in every kernel, so that all agree on who is off the grid
     ok = ok && (t > T(-1)) && (t < T(res - 1));
     base[d] = ok ? (int)t : 0;
     fx[d] = s - (T)base[d];
@@ -90,10 +105,10 @@ __global__ void phase_p2g_kernel(PhaseArgs<T> a) {
   int kind;
   T h, tc, ts;
   material_of(a, p, kind, h, tc, ts);
-  const int64_t mi = a.mat_scalar ? 0 : p;
-  const T m = valid ? a.mass[mi] : T(0);
-  T mu, lam;
-  lame<T>(kind, h, a.mu0[mi], a.lam0[mi], a.Jp[p], mu, lam);
+  T m, mu0, lam0, mu, lam;
+  constants_of(a, p, m, mu0, lam0);
+  if (!valid) m = T(0);
+  lame<T>(kind, h, mu0, lam0, a.Jp[p], mu, lam);
   const bool textbook = a.quirks == MPM_QUIRKS_TEXTBOOK;
   const int64_t r1 = a.res + 1;
   if constexpr (DIM == 3) {
@@ -151,6 +166,22 @@ __global__ void phase_p2g_kernel(PhaseArgs<T> a) {
   }
 }
 
+// Particles whose stencil leaves the grid.  A launch of its own ahead of a
+// phase's kernels lets the host read the count, and raise, while those still
+// run: with the count taken inside the phase kernels and read after them, each
+// call left the GPU idle for the 20-25 us that the host needs to see the end
+// of one call and to launch the next.
+template <typename T, int DIM>
+__global__ __launch_bounds__(256) void phase_oob_kernel(const T* __restrict__ x, int64_t n, int res, T inv_dx,
+                                                        unsigned long long* __restrict__ oob) {
+  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  int base[DIM];
+  T fx[DIM];
+  const bool out = p < n && !locate<T, DIM>(x + p * DIM, inv_dx, res, base, fx);
+  const unsigned long long m = __ballot(out);
+  if (m && (threadIdx.x & 63) == 0) atomicAdd(oob, (unsigned long long)__popcll(m));
+}
+
 // Sort keys of the particles' stencil bases: blocks of 4^3 (3D) or 8^2 (2D)
 // cells, then the cell inside the block, so that consecutive particles of
 // the sorted order share cells and, 256 at a time, a small bounding box.
@@ -195,10 +226,9 @@ __global__ __launch_bounds__(CELLSUM_THREADS) void phase_p2g_sorted_kernel(Phase
     int kind;
     T h, tc, ts;
     material_of(a, p, kind, h, tc, ts);
-    const int64_t mi = a.mat_scalar ? 0 : p;
-    const T m = a.mass[mi];
-    T mu, lam;
-    lame<T>(kind, h, a.mu0[mi], a.lam0[mi], a.Jp[p], mu, lam);
+    T m, mu0, lam0, mu, lam;
+    constants_of(a, p, m, mu0, lam0);
+    lame<T>(kind, h, mu0, lam0, a.Jp[p], mu, lam);
     const bool textbook = a.quirks == MPM_QUIRKS_TEXTBOOK;
     T A[DIM * DIM];
     if constexpr (DIM == 3)
@@ -534,22 +564,50 @@ static void launch_p2g(hipStream_t st, const PhaseArgs<T>& a, int64_t key_space,
                      dim3(CELLSUM_THREADS), 0, st, a, perm);
 }
 
+template <typename T>
+static void set_uniform(PhaseArgs<T>& a, const double* uniform) {
+  if (!uniform) return;
+  a.uniform = 1;
+  a.mass1 = (T)uniform[0];
+  a.mu1 = (T)uniform[1];
+  a.lam1 = (T)uniform[2];
+}
+
 // work: phase_p2g_workspace_bytes() bytes for the sorted form, null for the
-// direct one.
+// direct one.  uniform: mass, mu0 and lambda0 of every particle (host), or
+// null to read them from p.
 void phase_p2g(hipStream_t st, const mpm_params* prm, const mpm_particles* p, int kind_override,
                double hardening, const mpm_material* mats, int nmat, void* gv, void* gm,
-               unsigned long long* oob, void* work) {
+               unsigned long long* oob, void* work, const double* uniform) {
   if (p->n <= 0) return;
   const int64_t keys = p2g_key_space(prm, p->n);
   if (p->dtype == MPM_F64) {
     auto a = make_args<double>(prm, p, kind_override, hardening, 0, 0, mats, nmat, gv, gm, oob);
+    set_uniform(a, uniform);
     if (prm->dim == 3) launch_p2g<double, 3>(st, a, keys, work);
     else launch_p2g<double, 2>(st, a, keys, work);
   } else {
     auto a = make_args<float>(prm, p, kind_override, hardening, 0, 0, mats, nmat, gv, gm, oob);
+    set_uniform(a, uniform);
     if (prm->dim == 3) launch_p2g<float, 3>(st, a, keys, work);
     else launch_p2g<float, 2>(st, a, keys, work);
   }
+}
+
+void phase_oob(hipStream_t st, const mpm_params* prm, const mpm_particles* p, unsigned long long* oob) {
+  if (p->n <= 0) return;
+  const unsigned nb = blocks_for(p->n, 256);
+#define MPM_OOB(T, D)                                                                                          \
+  hipLaunchKernelGGL((phase_oob_kernel<T, D>), dim3(nb), dim3(256), 0, st, (const T*)p->x, p->n, prm->res, \
+                     (T)prm->inv_dx, oob)
+  if (p->dtype == MPM_F64) {
+    if (prm->dim == 3) MPM_OOB(double, 3);
+    else MPM_OOB(double, 2);
+  } else {
+    if (prm->dim == 3) MPM_OOB(float, 3);
+    else MPM_OOB(float, 2);
+  }
+#undef MPM_OOB
 }
 
 void phase_grid_op(hipStream_t st, const mpm_params* prm, int dtype, void* gv, const void* gm) {

@@ -313,7 +313,8 @@ class Engine:
 
 
 def bin_particles(x: torch.Tensor, res: int, inv_dx: float, layout: str = "blocked"):
-    """Cell keys and their stable ordering for FP32 CUDA positions (N, d)."""
+    """Cell keys and their stable ordering for FP32 CUDA positions (N, d), in
+    the order of the current stream."""
     _lib.require_gpu()
     L = _lib.load()
     if not (x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and x.dim() == 2):
@@ -321,8 +322,12 @@ def bin_particles(x: torch.Tensor, res: int, inv_dx: float, layout: str = "block
     n, dim = x.shape
     keys = torch.empty(n, dtype=torch.int32, device=x.device)
     perm = torch.empty(n, dtype=torch.int32, device=x.device)
-    torch.cuda.current_stream(x.device).synchronize()
+    nbytes = ct.c_int64()
+    _lib.check(L.mpm_bin_workspace_bytes(int(n), ct.byref(nbytes)), "mpm_bin")
+    work = torch.empty(nbytes.value, dtype=torch.uint8, device=x.device)
     lay = _lib.MPM_KEY_BLOCKED if layout == "blocked" else _lib.MPM_KEY_ROWMAJOR
-    _lib.check(L.mpm_bin(None, int(dim), int(res), float(inv_dx), lay, x.data_ptr(), int(n),
-                         keys.data_ptr(), perm.data_ptr()), "mpm_bin")
+    with torch.cuda.device(x.device):
+        _lib.check(L.mpm_bin_ws(torch.cuda.current_stream().cuda_stream, int(dim), int(res), float(inv_dx), lay,
+                                x.data_ptr(), int(n), keys.data_ptr(), perm.data_ptr(), work.data_ptr(),
+                                nbytes.value), "mpm_bin")
     return keys, perm

@@ -67,7 +67,8 @@ def materials_array(materials):
 
 
 class StagedParticles:
-    """Device views of (x, v, F, C, Jp, mass, mu0, lambda0[, material])."""
+    """Device views of (x, v, F, C, Jp, mass, mu0, lambda0[, material]); mass,
+    mu0 and lambda0 may be None where the phase does not read them."""
 
     def __init__(self, pos, v, F, C, Jp, mass, mu0, lam0, material=None, mat_scalar=False,
                  records=None):
@@ -81,19 +82,18 @@ class StagedParticles:
         self.F = Staged(F, dt, self.device)
         self.C = Staged(C, dt, self.device)
         self.Jp = Staged(Jp, dt, self.device)
-        self.mass = Staged(mass, dt, self.device, writable=False)
-        self.mu0 = Staged(mu0, dt, self.device, writable=False)
-        self.lam0 = Staged(lam0, dt, self.device, writable=False)
+        constant = lambda a: None if a is None else Staged(a, dt, self.device, writable=False)  # noqa: E731
+        self.mass, self.mu0, self.lam0 = constant(mass), constant(mu0), constant(lam0)
         self.material = None if material is None else Staged(material, torch.int32, self.device,
                                                               writable=False)
         self.mat_scalar = mat_scalar
         self.records = records
 
     def struct(self):
+        ptr = lambda s: None if s is None else s.ptr  # noqa: E731
         return _lib.Particles(
             self.n, mpm_dtype(self.dtype), 1 if self.mat_scalar else 0, self.x.ptr, self.v.ptr,
-            self.F.ptr, self.C.ptr, self.Jp.ptr, self.mass.ptr, self.mu0.ptr, self.lam0.ptr,
-            self.material.ptr if self.material is not None else None)
+            self.F.ptr, self.C.ptr, self.Jp.ptr, ptr(self.mass), ptr(self.mu0), ptr(self.lam0), ptr(self.material))
 
     def commit(self, state=True, positions=True):
         if positions:
@@ -116,24 +116,65 @@ def stage_3d(particles, v, F, C, Jp):
     return StagedParticles(ps.pos, v, F, C, Jp, ps.mass, ps.mu_0, ps.lambda_0, records=records)
 
 
-def run_p2g(sp, prm, kind_override, hardening, grid_velocity, grid_mass, materials=None):
-    _lib.require_gpu()
+class OutOfGrid:
+    """Counts the particles whose stencil leaves the grid, ahead of a phase's
+    own launches, so that the host can wait for the count while they run."""
+
+    def __init__(self, sp, prm):
+        count = torch.zeros(1, dtype=torch.int64, device=sp.device)
+        p = sp.struct()
+        _lib.check(_lib.load().mpm_count_oob(stream_ptr(sp.device), ct.byref(prm), ct.byref(p), count.data_ptr()),
+                   "count_oob")
+        self.host = torch.empty(1, dtype=torch.int64, pin_memory=True)
+        self.host.copy_(count, non_blocking=True)
+        self.counted = torch.cuda.Event()
+        self.counted.record(torch.cuda.current_stream(sp.device))
+
+    def wait(self):
+        self.counted.synchronize()
+        return self.host.item()
+
+
+def _workspace(sp, prm):
+    nbytes = ct.c_int64()
+    _lib.check(_lib.load().mpm_p2g_workspace_bytes(ct.byref(prm), sp.n, ct.byref(nbytes)), "p2g")
+    work = torch.empty(nbytes.value, dtype=torch.uint8, device=sp.device) if nbytes.value else None
+    return work, None if work is None else work.data_ptr(), nbytes.value
+
+
+def launch_p2g(sp, prm, kind_override, hardening, grid_velocity, grid_mass, materials=None):
     L = _lib.load()
     gv = Staged(grid_velocity, sp.dtype, sp.device)
     gm = Staged(grid_mass, sp.dtype, sp.device)
-    oob = torch.zeros(1, dtype=torch.int64, device=sp.device)
     mats, nmat = materials_array(materials)
     p = sp.struct()
-    nbytes = ct.c_int64()
-    _lib.check(L.mpm_p2g_workspace_bytes(ct.byref(prm), sp.n, ct.byref(nbytes)), "p2g")
-    work = torch.empty(nbytes.value, dtype=torch.uint8, device=sp.device) if nbytes.value else None
+    work, ptr, nbytes = _workspace(sp, prm)
     _lib.check(L.mpm_p2g_ws(stream_ptr(sp.device), ct.byref(prm), ct.byref(p), int(kind_override),
-                            float(hardening), mats, nmat, gv.ptr, gm.ptr, oob.data_ptr(),
-                            None if work is None else work.data_ptr(), nbytes.value), "p2g")
-    n_oob = int(oob.item())
+                            float(hardening), mats, nmat, gv.ptr, gm.ptr, None, ptr, nbytes), "p2g")
     gv.commit()
     gm.commit()
-    return n_oob
+
+
+def run_p2g(sp, prm, kind_override, hardening, grid_velocity, grid_mass, materials=None):
+    """P2G; the number of particles off the grid."""
+    _lib.require_gpu()
+    out = OutOfGrid(sp, prm)
+    launch_p2g(sp, prm, kind_override, hardening, grid_velocity, grid_mass, materials)
+    return out.wait()
+
+
+def run_p2g_uniform(sp, prm, kind, hardening, mass, mu0, lam0, grid_velocity, grid_mass):
+    """P2G of particles of one material, given by value; nothing is counted."""
+    _lib.require_gpu()
+    gv = Staged(grid_velocity, sp.dtype, sp.device)
+    gm = Staged(grid_mass, sp.dtype, sp.device)
+    p = sp.struct()
+    work, ptr, nbytes = _workspace(sp, prm)
+    _lib.check(_lib.load().mpm_p2g_uniform(stream_ptr(sp.device), ct.byref(prm), ct.byref(p), int(kind),
+                                           float(hardening), float(mass), float(mu0), float(lam0), gv.ptr, gm.ptr,
+                                           ptr, nbytes), "p2g")
+    gv.commit()
+    gm.commit()
 
 
 def run_grid_op(prm, grid_velocity, grid_mass):
@@ -169,13 +210,19 @@ def run_collide_planes(points, normals, res, dx, grid_velocity, quirks):
     gv.commit()
 
 
-def run_g2p(sp, prm, kind_override, grid_velocity, theta_c=THETA_C, theta_s=THETA_S, materials=None):
+def launch_g2p(sp, prm, kind_override, grid_velocity, theta_c=THETA_C, theta_s=THETA_S, materials=None):
     _lib.require_gpu()
     L = _lib.load()
     gv = Staged(grid_velocity, sp.dtype, sp.device, writable=False)
-    oob = torch.zeros(1, dtype=torch.int64, device=sp.device)
     mats, nmat = materials_array(materials)
     p = sp.struct()
     _lib.check(L.mpm_g2p(stream_ptr(sp.device), ct.byref(prm), ct.byref(p), int(kind_override),
-                         float(theta_c), float(theta_s), mats, nmat, gv.ptr, oob.data_ptr()), "g2p")
-    return int(oob.item())
+                         float(theta_c), float(theta_s), mats, nmat, gv.ptr, None), "g2p")
+
+
+def run_g2p(sp, prm, kind_override, grid_velocity, theta_c=THETA_C, theta_s=THETA_S, materials=None):
+    """G2P; the number of particles off the grid."""
+    _lib.require_gpu()
+    out = OutOfGrid(sp, prm)
+    launch_g2p(sp, prm, kind_override, grid_velocity, theta_c, theta_s, materials)
+    return out.wait()

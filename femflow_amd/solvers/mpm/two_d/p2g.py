@@ -14,12 +14,6 @@ def p2g(inv_dx, hardening, mu_0, lambda_0, mass, dx, dt, volume, grid_velocity, 
     (the reference broadcasts it to every entry, utils.py:86)."""
     res = int(grid_velocity.shape[0]) - 1
     q = _phase.quirks_code(quirks)
-    import torch
-
-    dev = _phase.device_of(x, v, F)
-    dt_ = _phase.compute_dtype(v, F, x)
-    scal = lambda s: torch.tensor([float(s)], dtype=dt_, device=dev)  # noqa: E731
-    sp = _phase.StagedParticles(x, v, F, C, Jp, scal(mass), scal(mu_0), scal(lambda_0),
-                                mat_scalar=True)
+    sp = _phase.StagedParticles(x, v, F, C, Jp, None, None, None)
     prm = _phase.make_params(2, res, inv_dx, dx, dt, volume, quirks=q, check_oob=False)
-    _phase.run_p2g(sp, prm, _phase.p2g_kind(model), hardening, grid_velocity, grid_mass)
+    _phase.run_p2g_uniform(sp, prm, _phase.p2g_kind(model), hardening, mass, mu_0, lambda_0, grid_velocity, grid_mass)

@@ -124,6 +124,19 @@ int32_t mpm_p2g_ws(void* stream, const mpm_params* prm, const mpm_particles* p, 
                    double hardening, const mpm_material* materials, int32_t nmat, void* grid_v, void* grid_m,
                    int64_t* oob_count, void* work, int64_t work_bytes);
 
+/* mpm_p2g_ws with one material for all particles, by value (the 2D
+ * signature, two_d/p2g.py:12-29): p->mass, mu0 and lambda0 are not read and
+ * may be NULL.  Particles whose stencil leaves the grid are skipped and not
+ * counted. */
+int32_t mpm_p2g_uniform(void* stream, const mpm_params* prm, const mpm_particles* p, int32_t kind, double hardening,
+                        double mass, double mu0, double lambda0, void* grid_v, void* grid_m, void* work,
+                        int64_t work_bytes);
+
+/* Adds the number of particles whose stencil leaves the grid to *oob_count
+ * (device int64), reading p's positions only: what mpm_p2g and mpm_g2p count
+ * for the same particles, before they run. */
+int32_t mpm_count_oob(void* stream, const mpm_params* prm, const mpm_particles* p, int64_t* oob_count);
+
 /* Replaces three_d.grid_op (three_d/grid_op.py:5-47) and two_d.grid_op
  * (two_d/grid_op.py:5-24). In place on grid_v. */
 int32_t mpm_grid_op(void* stream, const mpm_params* prm, int32_t dtype, void* grid_v,
@@ -238,6 +251,12 @@ int32_t mpm_particle_sums(mpm_ctx* ctx, double* out);
  * three_d/p2g.py:49); the key derives from its base, three_d/p2g.py:50. */
 int32_t mpm_bin(mpm_ctx* ctx, int32_t dim, int32_t res, double inv_dx, int32_t layout,
                 const float* x, int64_t n, uint32_t* keys, uint32_t* perm);
+/* mpm_bin on a stream, with scratch memory (device, 16-byte aligned) of
+ * mpm_bin_workspace_bytes() bytes: it allocates nothing and returns before
+ * the work is done, in stream order. */
+int32_t mpm_bin_workspace_bytes(int64_t n, int64_t* bytes);
+int32_t mpm_bin_ws(void* stream, int32_t dim, int32_t res, double inv_dx, int32_t layout, const float* x, int64_t n,
+                   uint32_t* keys, uint32_t* perm, void* work, int64_t work_bytes);
 /* mpm_bin that allocates nothing: the same arguments and bit-identical keys
  * and perm, with the sort's workspace in a fixed device array of the library
  * (about 20 MiB per GPU, held until the process ends) instead of per-call
