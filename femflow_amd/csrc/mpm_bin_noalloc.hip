@@ -2,10 +2,10 @@
 // (mpm_capi.hip), with the sort's workspace in one file-scope device array
 // instead of per-call hipMalloc/hipFree, for callers that cannot allocate.
 //
-// The array holds, for n <= NOALLOC_MAX_N particles: the sort's working copy
-// of the keys (n words), the key/value ping-pong buffers (2n), and the
-// per-tile digit histograms with their offsets (2 * max(RS_BINS * tiles, n))
-// and the RS_BINS digit totals.  Each GPU holds its own copy for the life of the
+// The array holds, for n <= NOALLOC_MAX_N particles: the sort's scratch keys
+// (n words), the key/value ping-pong buffers (2n), and the per-tile digit
+// histograms with their offsets (2 * RS_MAX_BINS * tiles) and the RS_MAX_BINS
+// digit totals.  Each GPU holds its own copy for the life of the
 // process; its address is looked up once per device (hipGetSymbolAddress)
 // and only that address is handed to kernels.  Nothing in it needs to start
 // at zero: every word a call reads was written earlier in the same call.
@@ -21,10 +21,8 @@ namespace mpm {
 void set_error(const std::string& msg);
 
 constexpr int64_t NOALLOC_MAX_N = int64_t(1) << 20;
-constexpr int64_t NOALLOC_TILES = (NOALLOC_MAX_N + RS_TILE - 1) / RS_TILE;
-constexpr int64_t NOALLOC_BIG =
-    RS_BINS * NOALLOC_TILES > NOALLOC_MAX_N ? RS_BINS * NOALLOC_TILES : NOALLOC_MAX_N;
-constexpr int64_t NOALLOC_WORDS = NOALLOC_MAX_N + 2 * NOALLOC_MAX_N + 2 * NOALLOC_BIG + RS_BINS + 64;
+constexpr int64_t NOALLOC_TILES = 512;  // the most that radix_plan gives for n <= NOALLOC_MAX_N
+constexpr int64_t NOALLOC_WORDS = 3 * NOALLOC_MAX_N + 2 * RS_MAX_BINS * NOALLOC_TILES + RS_MAX_BINS + 64;
 static_assert(NOALLOC_WORDS * 4 <= (int64_t(24) << 20), "scratch stays under 24 MiB");
 
 static __device__ __align__(256) uint32_t scratch[NOALLOC_WORDS];
@@ -86,15 +84,16 @@ extern "C" int32_t mpm_bin_noalloc(mpm_ctx* ctx, int32_t dim, int32_t res, doubl
   uint32_t* s = mpm::scratch_for_current_device();
   if (!s) return MPM_ERR_HIP;
   hipStream_t st = nullptr;
-  uint32_t* tmp = s;            // n words: the sort's copy of the keys
-  uint32_t* ws = s + mpm::NOALLOC_MAX_N;  // radix_sort's workspace
-  mpm::bin_keys(x, n, dim, res, (float)inv_dx, layout, keys, st);
-  if (hipMemcpyAsync(tmp, keys, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st) != hipSuccess) {
-    mpm::set_error("mpm_bin_noalloc: copying the keys failed");
-    return MPM_ERR_HIP;
+  if (mpm::radix_workspace_bytes(n) > sizeof(uint32_t) * (mpm::NOALLOC_WORDS - mpm::NOALLOC_MAX_N)) {
+    mpm::set_error("mpm_bin_noalloc: the sort needs more than the fixed workspace");
+    return MPM_ERR_ARG;
   }
-  uint32_t *ks, *vs;
-  mpm::radix_sort(tmp, perm, n, (uint32_t)max_key, ws, true, &ks, &vs, st);
+  uint32_t* tmp = s;            // n words: the sort's scratch keys
+  uint32_t* ws = s + mpm::NOALLOC_MAX_N;  // radix_sort's workspace
+  const mpm::RadixPlan pl = mpm::radix_plan(n, (uint32_t)max_key);
+  mpm::bin_keys(pl, x, n, dim, res, (float)inv_dx, layout, keys, mpm::radix_first_hist(ws, n), st);
+  uint32_t* vs;
+  mpm::radix_sort(pl, keys, tmp, perm, n, ws, true, true, nullptr, &vs, st);
   if (vs != perm) hipMemcpyAsync(perm, vs, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st);
   const hipError_t e = hipStreamSynchronize(st);
   if (e != hipSuccess) {

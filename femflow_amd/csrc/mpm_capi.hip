@@ -609,15 +609,15 @@ static const char* bin_key_space(int32_t dim, int32_t res, int32_t layout, const
   return nullptr;
 }
 
-// Words of the sort's copy of the keys, ahead of its own workspace.
+// Words of the sort's scratch keys, ahead of its own workspace.
 static size_t bin_keys_words(int64_t n) { return ((size_t)n + 63) & ~(size_t)63; }
 
 static void bin_on(hipStream_t st, int32_t dim, int32_t res, double inv_dx, int32_t layout, const float* x, int64_t n,
                    uint32_t max_key, uint32_t* keys, uint32_t* perm, uint32_t* work) {
-  uint32_t *ks, *vs;
-  mpm::bin_keys(x, n, dim, res, (float)inv_dx, layout, keys, st);
-  hipMemcpyAsync(work, keys, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st);
-  mpm::radix_sort(work, perm, n, max_key, work + bin_keys_words(n), true, &ks, &vs, st);
+  uint32_t *vs, *ws = work + bin_keys_words(n);
+  const mpm::RadixPlan pl = mpm::radix_plan(n, max_key);
+  mpm::bin_keys(pl, x, n, dim, res, (float)inv_dx, layout, keys, mpm::radix_first_hist(ws, n), st);
+  mpm::radix_sort(pl, keys, work, perm, n, ws, true, true, nullptr, &vs, st);
   if (vs != perm) hipMemcpyAsync(perm, vs, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st);
 }
 

@@ -1249,40 +1249,41 @@ __device__ __forceinline__ int cell_of(float x, float inv_dx, int res) {
   return b < 0 ? 0 : (b > res ? res : b);
 }
 
-// Cell keys of the new binning, one sort tile (RS_TILE particles) per
+// Cell keys of the new binning, one sort tile (256 * ITEMS particles) per
 // workgroup, with the tile histogram of the sort's first digit, so the sort
 // starts at that pass's scan.  Also starts the segment that rebins (the
 // counters' segment_begin) and clears the block occupancy that
 // block_bounds_kernel sets: two launches fewer ahead of the sort.
+template <int ITEMS>
 __global__ __launch_bounds__(RS_THREADS) void engine_keys_kernel(EngineArgs a, int64_t n,
                                                                  uint32_t* __restrict__ keys,
                                                                  uint32_t* __restrict__ bocc, int64_t nblocks,
-                                                                 int len, int with_sums,
+                                                                 int len, int with_sums, int bits,
                                                                  uint32_t* __restrict__ hist) {
-  __shared__ uint32_t h[RS_BINS];
+  __shared__ uint32_t h[RS_MAX_BINS];
   const int64_t gid = (int64_t)blockIdx.x * RS_THREADS + threadIdx.x;
   if (gid == 0) segment_begin(a.counters, len, with_sums, 1);
   if (blockIdx.x == 0) segment_speeds(a);
   for (int64_t j = gid; j < nblocks; j += (int64_t)gridDim.x * RS_THREADS) bocc[j] = 0u;
   const bool one_scene = a.nscenes == 1;
   const SceneDev sc0 = a.scenes[0];
-  const int64_t base = (int64_t)blockIdx.x * RS_TILE;
+  const int64_t base = (int64_t)blockIdx.x * (ITEMS * RS_THREADS);
   // every position of the thread is loaded before the first key is stored
   // (the key stores could alias the positions as far as the compiler knows,
   // which would otherwise put one memory round trip per key in series)
-  float px[RS_ITEMS][3];
-  uint32_t sid[RS_ITEMS];
+  float px[ITEMS][3];
+  uint32_t sid[ITEMS];
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const int64_t i = base + (int64_t)r * RS_THREADS + threadIdx.x;
     const int64_t j = i < n ? i : 0;
 #pragma unroll
     for (int d = 0; d < 3; ++d) px[r][d] = a.s.x[tix(j, 3, d)];
     sid[r] = one_scene ? 0u : a.s.attr[j] >> 8;
   }
-  uint32_t k[RS_ITEMS];
+  uint32_t k[ITEMS];
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const int64_t i = base + (int64_t)r * RS_THREADS + threadIdx.x;
     const SceneDev sc = one_scene ? sc0 : a.scenes[sid[r]];
     const int b0 = cell_of(px[r][0], sc.inv_dx, sc.res);
@@ -1292,7 +1293,7 @@ __global__ __launch_bounds__(RS_THREADS) void engine_keys_kernel(EngineArgs a, i
     k[r] = blk * 64u + (uint32_t)(((b0 & 3) << 4) | ((b1 & 3) << 2) | (b2 & 3));
     if (i < n) keys[i] = k[r];
   }
-  rs_tile_histogram(k, n, 0, h, hist);
+  rs_tile_histogram<ITEMS>(k, n, 0, bits, h, hist);
 }
 
 __global__ void block_bounds_kernel(const uint32_t* __restrict__ keys, int64_t n,
@@ -1926,12 +1927,16 @@ void Engine::enqueue_bin(hipStream_t s, int len, int with_sums) {
     return;
   }
   EngineArgs a = args(nullptr, 0, 0);
-  const int64_t tiles = radix_tiles(n);
-  hipLaunchKernelGGL(engine_keys_kernel, dim3((unsigned)tiles), dim3(RS_THREADS), 0, s, a, n, d_keys, d_bocc,
-                     (int64_t)total_blocks, len, with_sums, radix_first_hist(d_ws, n));
+  const RadixPlan pl = radix_plan(n, (uint32_t)(total_blocks * 64 - 1));
+#define MPM_KEYS(I)                                                                                                  \
+  hipLaunchKernelGGL((engine_keys_kernel<I>), dim3((unsigned)pl.tiles), dim3(RS_THREADS), 0, s, a, n, d_keys, d_bocc, \
+                     (int64_t)total_blocks, len, with_sums, pl.bits, radix_first_hist(d_ws, n))
+  if (pl.items == 4) MPM_KEYS(4);
+  else if (pl.items == 8) MPM_KEYS(8);
+  else MPM_KEYS(16);
+#undef MPM_KEYS
   uint32_t *ks, *vs;
-  const uint32_t max_key = (uint32_t)(total_blocks * 64 - 1);
-  radix_sort(d_keys, d_vals, n, max_key, d_ws, true, &ks, &vs, s, true);
+  radix_sort(pl, d_keys, d_keys, d_vals, n, d_ws, true, true, &ks, &vs, s);
   // the particles move into binned order in the segment's first P2G, which
   // reads slot perm[p] of the current buffer and writes slot p of the other
   cur ^= 1;

@@ -7,6 +7,7 @@
 #include "mpm_math.h"
 #include "mpm_phase.h"
 #include "mpm_sort.h"
+#include "mpm_sort_dev.h"
 
 namespace mpm {
 
@@ -187,21 +188,42 @@ __global__ __launch_bounds__(256) void phase_oob_kernel(const T* __restrict__ x,
 // the sorted order share cells and, 256 at a time, a small bounding box.
 // Bases off the grid (and NaN) are clamped; the P2G tests them again.
 template <typename T, int DIM>
-__global__ __launch_bounds__(256) void phase_keys_kernel(const T* __restrict__ x, int64_t n, int res, T inv_dx,
-                                                         uint32_t* __restrict__ keys) {
-  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= n) return;
+__device__ __forceinline__ uint32_t phase_key(const T* x, int res, T inv_dx) {
   constexpr int SH = DIM == 3 ? 2 : 3, MASK = (1 << SH) - 1;
   const uint32_t nb = (uint32_t)(res + 1 + MASK) >> SH;
   uint32_t blk = 0, cell = 0;
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
-    const T t = x[p * DIM + d] * inv_dx - T(0.5);
+    const T t = x[d] * inv_dx - T(0.5);
     const int b = !(t > T(0)) ? 0 : (t < T(res) ? (int)t : res);
     blk = blk * nb + (uint32_t)(b >> SH);
     cell = (cell << SH) | (uint32_t)(b & MASK);
   }
-  keys[p] = (blk << 6) | cell;
+  return (blk << 6) | cell;
+}
+
+// One sort tile per workgroup, with its histogram of the sort's first digit.
+template <typename T, int DIM, int ITEMS>
+__global__ __launch_bounds__(RS_THREADS) void phase_keys_kernel(const T* __restrict__ x, int64_t n, int res, T inv_dx,
+                                                                uint32_t* __restrict__ keys, int bits,
+                                                                uint32_t* __restrict__ hist) {
+  __shared__ uint32_t h[RS_MAX_BINS];
+  const int64_t base = (int64_t)blockIdx.x * (ITEMS * RS_THREADS);
+  T px[ITEMS][DIM];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int64_t i = base + (int64_t)r * RS_THREADS + threadIdx.x, at = i < n ? i : 0;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) px[r][d] = x[at * DIM + d];
+  }
+  uint32_t k[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int64_t i = base + (int64_t)r * RS_THREADS + threadIdx.x;
+    k[r] = phase_key<T, DIM>(px[r], res, inv_dx);
+    if (i < n) keys[i] = k[r];
+  }
+  rs_tile_histogram<ITEMS>(k, n, 0, bits, h, hist);
 }
 
 // P2G of particles in cell order (perm), summed per cell and workgroup
@@ -557,9 +579,16 @@ static void launch_p2g(hipStream_t st, const PhaseArgs<T>& a, int64_t key_space,
     return;
   }
   uint32_t* keys = (uint32_t*)work;
-  uint32_t *ks, *perm;
-  hipLaunchKernelGGL((phase_keys_kernel<T, DIM>), dim3(nb), dim3(256), 0, st, a.x, a.n, a.res, a.inv_dx, keys);
-  radix_sort(keys, keys + a.n, a.n, (uint32_t)(key_space - 1), keys + 2 * a.n, true, &ks, &perm, st);
+  uint32_t *perm, *ws = keys + 2 * a.n;
+  const RadixPlan pl = radix_plan(a.n, (uint32_t)(key_space - 1));
+#define MPM_KEYS(I)                                                                                                 \
+  hipLaunchKernelGGL((phase_keys_kernel<T, DIM, I>), dim3((unsigned)pl.tiles), dim3(RS_THREADS), 0, st, a.x, a.n, \
+                     a.res, a.inv_dx, keys, pl.bits, radix_first_hist(ws, a.n))
+  if (pl.items == 4) MPM_KEYS(4);
+  else if (pl.items == 8) MPM_KEYS(8);
+  else MPM_KEYS(16);
+#undef MPM_KEYS
+  radix_sort(pl, keys, keys, keys + a.n, a.n, ws, true, true, nullptr, &perm, st);
   hipLaunchKernelGGL((phase_p2g_sorted_kernel<T, DIM>), dim3(blocks_for(a.n, CELLSUM_THREADS)),
                      dim3(CELLSUM_THREADS), 0, st, a, perm);
 }

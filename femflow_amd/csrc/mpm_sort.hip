@@ -1,5 +1,5 @@
 // Cell binning: key generation, a stable LSD radix sort on 32-bit keys
-// (11-bit digits; three launches per pass: tile histograms, a per-digit scan
+// (digits of 8 to 11 bits; three launches per pass: tile histograms, a per-digit scan
 // over tiles, the stable scatter), and the chunk list (a two-launch scan of
 // per-block chunk counts) that gives the engine its work items for the
 // transfer kernels.
@@ -20,21 +20,22 @@ constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_ITEMS = 16;
 constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;
 
-// Per-tile digit histogram, written tile-major: hist[tile * RS_BINS + d].
+// Per-tile digit histogram, written tile-major: hist[(tile << bits) + d].
+template <int ITEMS>
 __global__ __launch_bounds__(RS_THREADS) void rs_upsweep(const uint32_t* __restrict__ keys,
-                                                         int64_t n, int shift,
+                                                         int64_t n, int shift, int bits,
                                                          uint32_t* __restrict__ hist) {
-  __shared__ uint32_t h[RS_BINS];
-  const int64_t base = (int64_t)blockIdx.x * RS_TILE;
+  __shared__ uint32_t h[RS_MAX_BINS];
+  const int64_t base = (int64_t)blockIdx.x * (ITEMS * RS_THREADS);
   // every key of the thread in flight at once: one memory round trip per
   // tile rather than one per few rounds
-  uint32_t k[RS_ITEMS];
+  uint32_t k[ITEMS];
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const int64_t idx = base + (int64_t)r * RS_THREADS + threadIdx.x;
-    k[r] = idx < n ? keys[idx] : 0u;
+    k[r] = keys[idx < n ? idx : 0];
   }
-  rs_tile_histogram(k, n, shift, h, hist);
+  rs_tile_histogram<ITEMS>(k, n, shift, bits, h, hist);
 }
 
 // Exclusive prefix sum over the 256 threads of a workgroup (one value each):
@@ -57,100 +58,115 @@ __device__ __forceinline__ uint32_t excl_scan_256(uint32_t v, uint32_t* wave_tot
 }
 
 // Per digit d: the exclusive prefix over tiles of the tile-major histogram
-// hist[tile * RS_BINS + d] (written to offs in the same layout) and the
+// hist[tile * bins + d] (written to offs in the same layout) and the
 // digit's total (dtot[d]); the scatter adds the exclusive prefix of the
-// totals over digits.  A workgroup takes 64 digits (lane = digit, so every
-// read and write is one contiguous 256-byte row piece) and splits the tiles
-// into DS_WAVES contiguous ranges, one per wave: each wave sums its range,
-// the waves' sums are prefixed in LDS, and each wave then writes its range's
-// running prefix.  Sixteen waves keep each wave's serial walk short (16
-// tiles for 2^20 keys).
-constexpr int DS_WAVES = 16;
-__global__ __launch_bounds__(DS_WAVES * 64) void rs_digit_scan(const uint32_t* __restrict__ hist, int ntiles,
-                                                              uint32_t* __restrict__ offs,
-                                                              uint32_t* __restrict__ dtot) {
-  __shared__ uint32_t part[DS_WAVES][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int d = blockIdx.x * 64 + lane;
-  const int per = (ntiles + DS_WAVES - 1) / DS_WAVES;
-  const int t0 = w * per < ntiles ? w * per : ntiles;
+// totals over digits.  A workgroup takes DS_DIGITS digits (neighbouring lanes,
+// so that every read and write is whole 64-byte pieces of rows) and splits the
+// tiles into DS_GROUPS contiguous ranges: each group sums its range, the sums
+// are prefixed in LDS, and each group then writes its range's running prefix.
+// The serial walk is what bounds it, so the ranges are many and short: 512
+// tiles of 2,048 digits in groups of 8 tiles on 128 workgroups; with 64 digits
+// and 16 ranges per workgroup (32 of 32 tiles) it took 9.3 us.
+constexpr int DS_DIGITS = 16, DS_GROUPS = 64;
+__global__ __launch_bounds__(DS_DIGITS * DS_GROUPS) void rs_digit_scan(const uint32_t* __restrict__ hist, int ntiles,
+                                                                       int bits, uint32_t* __restrict__ offs,
+                                                                       uint32_t* __restrict__ dtot) {
+  __shared__ uint32_t part[DS_GROUPS][DS_DIGITS];
+  const int dl = threadIdx.x % DS_DIGITS, g = threadIdx.x / DS_DIGITS;
+  const int d = blockIdx.x * DS_DIGITS + dl;
+  const int per = (ntiles + DS_GROUPS - 1) / DS_GROUPS;
+  const int t0 = g * per < ntiles ? g * per : ntiles;
   const int t1 = t0 + per < ntiles ? t0 + per : ntiles;
   uint32_t sum = 0;
-#pragma unroll 16
-  for (int tl = t0; tl < t1; ++tl) sum += hist[(int64_t)tl * RS_BINS + d];
-  part[w][lane] = sum;
+#pragma unroll 8
+  for (int tl = t0; tl < t1; ++tl) sum += hist[((int64_t)tl << bits) + d];
+  part[g][dl] = sum;
   __syncthreads();
   uint32_t run = 0;
-#pragma unroll
-  for (int i = 0; i < DS_WAVES; ++i) run += i < w ? part[i][lane] : 0u;
-  if (w == DS_WAVES - 1) dtot[d] = run + sum;
-#pragma unroll 16
+  const int used = ntiles < DS_GROUPS ? ntiles : DS_GROUPS;
+#pragma unroll 8
+  for (int i = 0; i < used; ++i) run += i < g ? part[i][dl] : 0u;
+  if (g == DS_GROUPS - 1) dtot[d] = run + sum;
+#pragma unroll 8
   for (int tl = t0; tl < t1; ++tl) {
-    const uint32_t v = hist[(int64_t)tl * RS_BINS + d];
-    offs[(int64_t)tl * RS_BINS + d] = run;
+    const uint32_t v = hist[((int64_t)tl << bits) + d];
+    offs[((int64_t)tl << bits) + d] = run;
     run += v;
   }
 }
 
+// Tile of a workgroup: each XCD (workgroup id mod 8) takes a contiguous run of
+// tiles, whose keys of one digit are neighbours in the output, so that their
+// partial lines meet in that XCD's L2.
+__device__ __forceinline__ uint32_t xcd_tile() {
+  const uint32_t xcd = blockIdx.x & 7u, per = gridDim.x >> 3, rem = gridDim.x & 7u;
+  return xcd * per + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
+}
+
+// kout null: the sorted keys are not wanted.
+template <int ITEMS>
 __global__ __launch_bounds__(RS_THREADS) void rs_downsweep(
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin, uint32_t* __restrict__ kout,
-    uint32_t* __restrict__ vout, int64_t n, int shift, const uint32_t* __restrict__ offs,
-    const uint32_t* __restrict__ dtot, int ntiles, int iota_values) {
-  __shared__ uint32_t cnt[RS_WAVES][RS_BINS];
-  __shared__ uint32_t goff[RS_BINS];
+    uint32_t* __restrict__ vout, int64_t n, int shift, int bits, const uint32_t* __restrict__ offs,
+    const uint32_t* __restrict__ dtot, int iota_values) {
+  __shared__ uint32_t cnt[RS_WAVES][RS_MAX_BINS];
+  __shared__ uint32_t goff[RS_MAX_BINS];
   __shared__ uint32_t wt[RS_WAVES];
   const int t = threadIdx.x;
   const int w = t >> 6;
   const unsigned lane = __lane_id();
-  constexpr int DPT = RS_BINS / RS_THREADS;  // digits per thread
+  constexpr int MAX_DPT = RS_MAX_BINS / RS_THREADS;
+  const int bins = 1 << bits, dpt = bins / RS_THREADS;  // digits per thread
+  // keys and values of the wave's run in flight from the start
+  const uint32_t tile = xcd_tile();
+  const int64_t base = (int64_t)tile * (ITEMS * RS_THREADS) + (int64_t)w * 64 * ITEMS;
+  uint32_t k[ITEMS], val[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int64_t idx = base + r * 64 + lane, at = idx < n ? idx : 0;
+    k[r] = kin[at];
+    val[r] = iota_values ? (uint32_t)idx : vin[at];
+  }
 #pragma unroll
   for (int i = 0; i < RS_WAVES; ++i)
-    for (int d = t; d < RS_BINS; d += RS_THREADS) cnt[i][d] = 0;
+    for (int d = t; d < bins; d += RS_THREADS) cnt[i][d] = 0;
   // global start of digit d in this tile: keys of smaller digits (all tiles)
   // plus keys of digit d in earlier tiles; thread t takes digits
-  // t * DPT .. t * DPT + DPT - 1
+  // t * dpt .. t * dpt + dpt - 1
   {
-    uint32_t tot[DPT], sum = 0;
+    uint32_t tot[MAX_DPT], before[MAX_DPT], sum = 0;
 #pragma unroll
-    for (int j = 0; j < DPT; ++j) {
-      tot[j] = dtot[t * DPT + j];
+    for (int j = 0; j < MAX_DPT; ++j) {
+      if (j >= dpt) break;
+      tot[j] = dtot[t * dpt + j];
+      before[j] = offs[((int64_t)tile << bits) + t * dpt + j];
       sum += tot[j];
     }
     uint32_t run = excl_scan_256(sum, wt);
 #pragma unroll
-    for (int j = 0; j < DPT; ++j) {
-      const int d = t * DPT + j;
-      goff[d] = run + offs[(int64_t)blockIdx.x * RS_BINS + d];
+    for (int j = 0; j < MAX_DPT; ++j) {
+      if (j >= dpt) break;
+      goff[t * dpt + j] = run + before[j];
       run += tot[j];
     }
   }
   __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * RS_TILE + (int64_t)w * 64 * RS_ITEMS;
-  uint32_t k[RS_ITEMS], val[RS_ITEMS];
-  uint32_t rank[RS_ITEMS];
+  uint32_t rank[ITEMS];
   const uint64_t lt = lanemask_lt();
-  // keys and values of the wave's run loaded together, ahead of the ranking
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const int64_t idx = base + r * 64 + lane;
     const bool valid = idx < n;
-    k[r] = valid ? kin[idx] : 0u;
-    val[r] = iota_values ? (uint32_t)idx : (valid ? vin[idx] : 0u);
-  }
-#pragma unroll
-  for (int r = 0; r < RS_ITEMS; ++r) {
-    const int64_t idx = base + r * 64 + lane;
-    const bool valid = idx < n;
-    const uint32_t d = (k[r] >> shift) & (uint32_t)(RS_BINS - 1);
+    const uint32_t d = (k[r] >> shift) & (uint32_t)(bins - 1);
     const uint64_t vm = __ballot(valid);
-    const uint64_t m = match_digit(d, vm);
+    const uint64_t m = match_digit(d, bits, vm);
     uint32_t prev = 0;
     if (valid) prev = cnt[w][d];
     rank[r] = prev + (uint32_t)__popcll(m & lt);
     if (valid && lane == 63u - (unsigned)__clzll(m)) cnt[w][d] = prev + (uint32_t)__popcll(m);
   }
   __syncthreads();
-  for (int d = t; d < RS_BINS; d += RS_THREADS) {
+  for (int d = t; d < bins; d += RS_THREADS) {
     uint32_t run = 0;
 #pragma unroll
     for (int i = 0; i < RS_WAVES; ++i) {
@@ -161,12 +177,12 @@ __global__ __launch_bounds__(RS_THREADS) void rs_downsweep(
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     const int64_t idx = base + r * 64 + lane;
     if (idx < n) {
-      const uint32_t d = (k[r] >> shift) & (uint32_t)(RS_BINS - 1);
+      const uint32_t d = (k[r] >> shift) & (uint32_t)(bins - 1);
       const uint32_t dst = goff[d] + cnt[w][d] + rank[r];
-      kout[dst] = k[r];
+      if (kout) kout[dst] = k[r];
       vout[dst] = val[r];
     }
   }
@@ -313,37 +329,93 @@ __device__ __forceinline__ int cell_coord(float x, float inv_dx, int res) {
   return b < 0 ? 0 : (b > res ? res : b);
 }
 
-__global__ void bin_keys_kernel(const float* __restrict__ x, int64_t n, int dim, int res,
-                                float inv_dx, int layout, uint32_t* __restrict__ keys) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int b[3] = {0, 0, 0};
-  for (int d = 0; d < dim; ++d) b[d] = cell_coord(x[i * dim + d], inv_dx, res);
+template <int DIM>
+__device__ __forceinline__ uint32_t bin_key(const float* x, int res, float inv_dx, int layout) {
+  int b[DIM];
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) b[d] = cell_coord(x[d], inv_dx, res);
   const uint32_t r1 = (uint32_t)res + 1u;
   uint32_t key;
   if (layout == MPM_KEY_ROWMAJOR) {
     key = (uint32_t)b[0];
-    for (int d = 1; d < dim; ++d) key = key * r1 + (uint32_t)b[d];
+#pragma unroll
+    for (int d = 1; d < DIM; ++d) key = key * r1 + (uint32_t)b[d];
   } else {
     const uint32_t nb = (r1 + 3u) / 4u;
     uint32_t bid = (uint32_t)(b[0] >> 2), cid = (uint32_t)(b[0] & 3);
-    for (int d = 1; d < dim; ++d) {
+#pragma unroll
+    for (int d = 1; d < DIM; ++d) {
       bid = bid * nb + (uint32_t)(b[d] >> 2);
       cid = cid * 4u + (uint32_t)(b[d] & 3);
     }
-    key = bid * (dim == 3 ? 64u : 16u) + cid;
+    key = bid * (DIM == 3 ? 64u : 16u) + cid;
   }
-  keys[i] = key;
+  return key;
+}
+
+// Keys of one sort tile per workgroup, with the tile's histogram of the first
+// digit (the sort then starts at its scan: one launch and one read of the keys
+// fewer).
+template <int DIM, int ITEMS>
+__global__ __launch_bounds__(RS_THREADS) void bin_keys_kernel(const float* __restrict__ x, int64_t n, int res,
+                                                              float inv_dx, int layout, uint32_t* __restrict__ keys,
+                                                              int bits, uint32_t* __restrict__ hist) {
+  __shared__ uint32_t h[RS_MAX_BINS];
+  const int64_t base = (int64_t)blockIdx.x * (ITEMS * RS_THREADS);
+  float px[ITEMS][DIM];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int64_t i = base + (int64_t)r * RS_THREADS + threadIdx.x, at = i < n ? i : 0;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) px[r][d] = x[at * DIM + d];
+  }
+  uint32_t k[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int64_t i = base + (int64_t)r * RS_THREADS + threadIdx.x;
+    k[r] = bin_key<DIM>(px[r], res, inv_dx, layout);
+    if (i < n) keys[i] = k[r];
+  }
+  rs_tile_histogram<ITEMS>(k, n, 0, bits, h, hist);
 }
 
 // ------------------------------------------------------------ host side ----
 static inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Keys per thread: the fewest that keep the tiles within MAX_SMALL_TILES, since
+// a tile's rounds of ranking are a serial chain and few tiles leave most of the
+// chip idle; the histograms (one row of digits per tile) bound it from above.
+// mpm_bin at 4 / 8 / 16 keys in us: 4,096 keys 28 / 36 / 54; 131,072 32 / 39 /
+// 57; 524,288 56 / 57 / 72; 2^20 86 / 72 / 82; 2^21 142 / 113 / 103.
+constexpr int64_t MAX_SMALL_TILES = 512;
+static int radix_items(int64_t n) {
+  if (n <= MAX_SMALL_TILES * RS_THREADS * 4) return 4;
+  return n <= MAX_SMALL_TILES * RS_THREADS * 8 ? 8 : 16;
+}
+
+RadixPlan radix_plan(int64_t n, uint32_t max_key) {
+  int bits = 0;
+  while (bits < 32 && (max_key >> bits) != 0u) ++bits;
+  RadixPlan p;
+  p.passes = bits == 0 ? 1 : (bits + RS_MAX_BITS - 1) / RS_MAX_BITS;
+  p.bits = (bits + p.passes - 1) / p.passes;
+  if (p.bits < 8) p.bits = 8;  // one digit per thread of the scatter's offsets
+  p.items = radix_items(n);
+  p.tiles = cdiv(n > 0 ? n : 1, (int64_t)RS_THREADS * p.items);
+  return p;
+}
+
+// Words of one tile histogram table, enough for any key space and for any
+// count up to n (a caller may sort fewer keys in the same workspace).
+static size_t radix_hist_words(int64_t n) {
+  const int64_t small = cdiv(n > 0 ? n : 1, RS_THREADS * 4), large = cdiv(n > 0 ? n : 1, RS_THREADS * 16);
+  const int64_t most = small < MAX_SMALL_TILES ? small : MAX_SMALL_TILES;
+  return (size_t)RS_MAX_BINS * (size_t)(large > most ? large : most);
+}
+
 size_t radix_workspace_bytes(int64_t n) {
-  const int64_t ntiles = cdiv(n > 0 ? n : 1, RS_TILE);
-  const int64_t hist = (int64_t)RS_BINS * ntiles;
-  // keys/vals ping-pong (4 arrays of n) + hist + offs + digit totals
-  return sizeof(uint32_t) * (4 * (size_t)n + 2 * (size_t)(hist > n ? hist : n) + RS_BINS + 64);
+  // keys and values (ping-pong) + histogram + its prefix + digit totals
+  return sizeof(uint32_t) * (2 * (size_t)(n > 0 ? n : 0) + 2 * radix_hist_words(n) + RS_MAX_BINS);
 }
 
 size_t chunk_list_part_words(int64_t nblocks) { return 4 * ((size_t)cdiv(nblocks, SCAN_THREADS) + 1); }
@@ -361,54 +433,62 @@ void chunk_list(const uint32_t* bocc, const uint32_t* bstart, const uint32_t* be
                      block_scene, nblocks, per_chunk, part4, chunks, bfirst, bcount, nchunks, plain ? 1 : 0);
 }
 
-int radix_passes(uint32_t max_key) {
-  int bits = 0;
-  while (bits < 32 && (max_key >> bits) != 0u) ++bits;
-  return bits == 0 ? 1 : (bits + RS_BITS - 1) / RS_BITS;
-}
-
-int64_t radix_tiles(int64_t n) { return cdiv(n > 0 ? n : 1, RS_TILE); }
-
 uint32_t* radix_first_hist(void* ws, int64_t n) { return (uint32_t*)ws + 2 * n; }
 
-// Stable sort of keys[0..n) carrying values; result in (*kout, *vout), which
-// point into either the input arrays or the workspace.  iota_values: the
-// input values are 0..n-1 (not read).  first_hist_done: the first pass's
-// tile histogram is already in the workspace (radix_first_hist).
-void radix_sort(uint32_t* keys, uint32_t* vals, int64_t n, uint32_t max_key, void* ws,
-                bool iota_values, uint32_t** kout, uint32_t** vout, hipStream_t st, bool first_hist_done) {
-  const int64_t ntiles = radix_tiles(n);
-  const int64_t hist_n = (int64_t)RS_BINS * ntiles;
-  const int64_t big = hist_n > n ? hist_n : n;
-  uint32_t* w = (uint32_t*)ws;
-  uint32_t* k2 = w;
-  uint32_t* v2 = w + n;
-  uint32_t* hist = radix_first_hist(ws, n);
-  uint32_t* offs = hist + big;
-  uint32_t* dtot = offs + big;
-  uint32_t *ka = keys, *va = vals, *kb = k2, *vb = v2;
-  const int passes = radix_passes(max_key);
-  for (int p = 0; p < passes; ++p) {
-    const int shift = RS_BITS * p;
-    if (p > 0 || !first_hist_done)
-      hipLaunchKernelGGL(rs_upsweep, dim3((unsigned)ntiles), dim3(RS_THREADS), 0, st, ka, n, shift, hist);
-    hipLaunchKernelGGL(rs_digit_scan, dim3(RS_BINS / 64), dim3(DS_WAVES * 64), 0, st, hist, (int)ntiles, offs,
-                       dtot);
-    hipLaunchKernelGGL(rs_downsweep, dim3((unsigned)ntiles), dim3(RS_THREADS), 0, st, ka, va, kb, vb,
-                       n, shift, offs, dtot, (int)ntiles, (iota_values && p == 0) ? 1 : 0);
-    uint32_t* t;
-    t = ka; ka = kb; kb = t;
-    t = va; va = vb; vb = t;
-  }
-  *kout = ka;
-  *vout = va;
+template <int ITEMS>
+static void radix_pass(const RadixPlan& pl, int pass, bool hist_done, const uint32_t* kin, const uint32_t* vin,
+                       uint32_t* kout, uint32_t* vout, int64_t n, uint32_t* hist, uint32_t* offs, uint32_t* dtot,
+                       bool iota, hipStream_t st) {
+  const int shift = pl.bits * pass;
+  const dim3 tiles((unsigned)pl.tiles);
+  if (!hist_done)
+    hipLaunchKernelGGL((rs_upsweep<ITEMS>), tiles, dim3(RS_THREADS), 0, st, kin, n, shift, pl.bits, hist);
+  hipLaunchKernelGGL(rs_digit_scan, dim3((1u << pl.bits) / DS_DIGITS), dim3(DS_DIGITS * DS_GROUPS), 0, st, hist, (int)pl.tiles,
+                     pl.bits, offs, dtot);
+  hipLaunchKernelGGL((rs_downsweep<ITEMS>), tiles, dim3(RS_THREADS), 0, st, kin, vin, kout, vout, n, shift, pl.bits,
+                     offs, dtot, iota ? 1 : 0);
 }
 
-void bin_keys(const float* x, int64_t n, int dim, int res, float inv_dx, int layout, uint32_t* keys,
-              hipStream_t st) {
+void radix_sort(const RadixPlan& pl, const uint32_t* source, uint32_t* keys, uint32_t* vals, int64_t n, void* ws,
+                bool iota_values, bool first_hist_done, uint32_t** kout, uint32_t** vout, hipStream_t st) {
+  uint32_t* hist = radix_first_hist(ws, n);
+  uint32_t* offs = hist + radix_hist_words(n);
+  uint32_t* dtot = offs + radix_hist_words(n);
+  const uint32_t *ka = source, *va = vals;
+  uint32_t *kb = (uint32_t*)ws, *vb = (uint32_t*)ws + n, *knext = keys, *vnext = vals;
+  for (int p = 0; p < pl.passes; ++p) {
+    uint32_t* ko = !kout && p == pl.passes - 1 ? nullptr : kb;
+    const bool done = p == 0 && first_hist_done, iota = iota_values && p == 0;
+    if (pl.items == 4) radix_pass<4>(pl, p, done, ka, va, ko, vb, n, hist, offs, dtot, iota, st);
+    else if (pl.items == 8) radix_pass<8>(pl, p, done, ka, va, ko, vb, n, hist, offs, dtot, iota, st);
+    else radix_pass<16>(pl, p, done, ka, va, ko, vb, n, hist, offs, dtot, iota, st);
+    ka = kb;
+    va = vb;
+    uint32_t* t;
+    t = kb; kb = knext; knext = t;
+    t = vb; vb = vnext; vnext = t;
+  }
+  // the last pass's outputs
+  if (kout) *kout = knext;
+  *vout = vnext;
+}
+
+void bin_keys(const RadixPlan& pl, const float* x, int64_t n, int dim, int res, float inv_dx, int layout,
+              uint32_t* keys, uint32_t* hist, hipStream_t st) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(bin_keys_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st, x, n, dim, res,
-                     inv_dx, layout, keys);
+#define MPM_BIN_KEYS(D, I)                                                                                      \
+  hipLaunchKernelGGL((bin_keys_kernel<D, I>), dim3((unsigned)pl.tiles), dim3(RS_THREADS), 0, st, x, n, res,     \
+                     inv_dx, layout, keys, pl.bits, hist)
+  if (dim == 3) {
+    if (pl.items == 4) MPM_BIN_KEYS(3, 4);
+    else if (pl.items == 8) MPM_BIN_KEYS(3, 8);
+    else MPM_BIN_KEYS(3, 16);
+  } else {
+    if (pl.items == 4) MPM_BIN_KEYS(2, 4);
+    else if (pl.items == 8) MPM_BIN_KEYS(2, 8);
+    else MPM_BIN_KEYS(2, 16);
+  }
+#undef MPM_BIN_KEYS
 }
 
 }  // namespace mpm
