@@ -33,11 +33,15 @@ template <typename T, int DIM, int NCH> struct CellSum {
   static constexpr int PAD = 16 / (int)sizeof(T);
   static constexpr int ENTRY = (NCH * ROW + 3 * DIM + PAD - 1) / PAD * PAD;
   typedef T Row3 __attribute__((ext_vector_type(4), aligned(16)));
-  static constexpr int ARENA = sizeof(T) == 8 ? 576 : 1024;  // nodes
+  // nodes; FP64 for FP32 particles too, since LDS adds of floats run at a
+  // third of a lane per cycle and those of doubles at about five (131,072 FP32
+  // particles, sort included, 80 -> 65 us at 2 per cell and 83 -> 64 at 16,
+  // with an arena of 1,024 FP32 nodes before)
+  static constexpr int ARENA = 576;
 
   struct alignas(16) Shared {
     T table[CELLSUM_THREADS * ENTRY];
-    T arena[ARENA * NCH];
+    double arena[ARENA * NCH];
     int box_w[CELLSUM_THREADS / 64][2 * DIM];
     int box[2 * DIM];  // low corner, extent (0: the box does not fit the arena)
   };
@@ -86,7 +90,7 @@ template <typename T, int DIM, int NCH> struct CellSum {
     }
     __syncthreads();
     const int n = volume(sh) * NCH;
-    for (int e = t; e < n; e += CELLSUM_THREADS) sh.arena[e] = T(0);
+    for (int e = t; e < n; e += CELLSUM_THREADS) sh.arena[e] = 0.0;
     __syncthreads();
   }
 
@@ -154,8 +158,8 @@ template <typename T, int DIM, int NCH> struct CellSum {
       if (arena) {
         int at = (b[0] + i - sh.box[0]) * sh.box[DIM + 1] + (b[1] + j - sh.box[1]);
         if constexpr (DIM == 3) at = at * sh.box[DIM + 2] + (b[2] + k - sh.box[2]);
-        if (on0) atomicAdd(&sh.arena[at * NCH + c0], a0);
-        if (on1) atomicAdd(&sh.arena[at * NCH + c0 + 1], a1);
+        if (on0) atomicAdd(&sh.arena[at * NCH + c0], (double)a0);
+        if (on1) atomicAdd(&sh.arena[at * NCH + c0 + 1], (double)a1);
       } else {
         b[0] += i;
         b[1] += j;
@@ -171,7 +175,7 @@ template <typename T, int DIM, int NCH> struct CellSum {
     __syncthreads();
     const int n = volume(sh) * NCH;
     for (int e = threadIdx.x; e < n; e += CELLSUM_THREADS) {
-      const T v = sh.arena[e];
+      const T v = (T)sh.arena[e];
       if (v != T(0)) {
         const int c = e % NCH;
         int sl = e / NCH;

@@ -2,7 +2,10 @@
 // grid_v (R+1)^d x d and grid_m (R+1)^d, row-major [i, j(, k)].  These back
 // the drop-in phase functions three_d.{p2g,grid_op,g2p} and
 // two_d.{p2g,grid_op,g2p} (FP32 or FP64, whichever the caller's arrays are).
-// One thread per particle (P2G, G2P) or per node (grid update).
+// One thread per particle (P2G, G2P) or per node (grid update).  P2G has two
+// forms, by size: see p2g_sort_from.
+#include <climits>
+
 #include "mpm_cellsum.h"
 #include "mpm_math.h"
 #include "mpm_phase.h"
@@ -81,89 +84,143 @@ __device__ __forceinline__ bool locate(const T* xp, T inv_dx, int res, int base[
   return ok;
 }
 
+// P2G of few particles (or without scratch memory) in any order: a workgroup
+// takes THREADS of them and sums into an LDS arena over their stencils'
+// bounding box, which goes to memory once.  What bounds it: up to a few
+// thousand particles the chain of loads, stress and LDS adds of one workgroup,
+// then the arenas' flushes (each workgroup's box is that of the whole body
+// when the order is arbitrary).  Layers of the box that the arena cannot hold
+// go to memory particle by particle.
+// Small workgroups spread few particles over more compute units: 2,048 3D
+// particles at 256 / 512 / 1,024 threads 17 / 26 / 46 us at 16 per cell and 23
+// / 30 / 47 at 2; in 2D, with a third of the adds, 512 is the best from 8,192
+// on (16,384 at 2 per cell 29 / 27 / 26, 8,192 16 / 13 / 15).
+// The arena is FP64 for FP32 particles too: LDS adds of floats run at a third
+// of a lane per cycle here, those of doubles at about five (8,192 2D FP32
+// particles 41 us with an FP32 arena, 9 with this one).
+// Per-particle device atomics, which this replaces: 8,192 2D FP64 particles at
+// 16 per cell 46 us (8.7 here), 2,048 3D 78 us (17).
+template <int DIM> constexpr int BOX_THREADS_OF = DIM == 3 ? 256 : 512;
+constexpr int BOX_WORDS = (144 << 10) / (int)sizeof(double);
+
 template <typename T, int DIM>
-__global__ void phase_p2g_kernel(PhaseArgs<T> a) {
-  // lanes past the end or out of the grid stay in the wave (its segmented
-  // atomics need every lane) with a zero contribution
-  const int64_t p0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(BOX_THREADS_OF<DIM>) void phase_p2g_box_kernel(PhaseArgs<T> a) {
+  constexpr int NCH = DIM + 1, THREADS = BOX_THREADS_OF<DIM>, WAVES = THREADS / 64;
+  __shared__ double arena[BOX_WORDS];
+  __shared__ int box_w[WAVES][2 * DIM];
+  const int t = threadIdx.x;
+  const int64_t p0 = (int64_t)blockIdx.x * THREADS + t;
   const bool inrange = p0 < a.n;
-  const int64_t p = inrange ? p0 : a.n - 1;
+  const int64_t p = inrange ? p0 : 0;
   int base[DIM];
   T fx[DIM];
   const bool located = locate<T, DIM>(a.x + p * DIM, a.inv_dx, a.res, base, fx);
   if (inrange && !located && a.oob) atomicAdd(a.oob, 1ull);
   const bool valid = inrange && located;
-  if (!located) {
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-      base[d] = 0;
-      fx[d] = T(1);
+  for (int d = 0; d < DIM; ++d) {
+    int lo = valid ? base[d] : INT_MAX, hi = valid ? base[d] : INT_MIN;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      lo = min(lo, __shfl_xor(lo, o));
+      hi = max(hi, __shfl_xor(hi, o));
+    }
+    if ((t & 63) == 0) {
+      box_w[t >> 6][d] = lo;
+      box_w[t >> 6][DIM + d] = hi;
     }
   }
-  T w[DIM][3];
+  __syncthreads();
+  int low[DIM], ext[DIM];
+  int64_t vol = 1;
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) bspline(fx[d], w[d]);
-  int kind;
-  T h, tc, ts;
-  material_of(a, p, kind, h, tc, ts);
-  T m, mu0, lam0, mu, lam;
-  constants_of(a, p, m, mu0, lam0);
-  if (!valid) m = T(0);
-  lame<T>(kind, h, mu0, lam0, a.Jp[p], mu, lam);
-  const bool textbook = a.quirks == MPM_QUIRKS_TEXTBOOK;
-  const int64_t r1 = a.res + 1;
-  if constexpr (DIM == 3) {
-    const WaveSeg sg = wave_segments(valid, (int)((base[0] * r1 + base[1]) * r1 + base[2]));
-    T A[9];
-    affine3<T>(a.F + 9 * p, a.C + 9 * p, m, mu, lam, kind, a.inv_dx, a.dt, a.vol, textbook, A);
-    if (!valid) {
+  for (int d = 0; d < DIM; ++d) {
+    int lo = INT_MAX, hi = INT_MIN;
 #pragma unroll
-      for (int e = 0; e < 9; ++e) A[e] = T(0);
+    for (int w = 0; w < WAVES; ++w) {
+      lo = min(lo, box_w[w][d]);
+      hi = max(hi, box_w[w][DIM + d]);
     }
-    const T mv[3] = {a.v[3 * p] * m, a.v[3 * p + 1] * m, a.v[3 * p + 2] * m};
+    low[d] = lo;
+    ext[d] = lo <= hi ? hi - lo + 3 : 0;
+    vol *= ext[d];
+  }
+  // the layers of the first axis that the arena holds
+  const int64_t layer = ext[0] ? vol / ext[0] * NCH : 1;
+  const int held = (int)min((int64_t)ext[0], BOX_WORDS / layer);
+  const int words = held * (int)layer;
+  for (int e = t; e < words; e += THREADS) arena[e] = 0.0;
+  __syncthreads();
+  if (valid) {
+    T w[DIM][3];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) bspline(fx[d], w[d]);
+    int kind;
+    T h, tc, ts, m, mu0, lam0, mu, lam;
+    material_of(a, p, kind, h, tc, ts);
+    constants_of(a, p, m, mu0, lam0);
+    lame<T>(kind, h, mu0, lam0, a.Jp[p], mu, lam);
+    const bool textbook = a.quirks == MPM_QUIRKS_TEXTBOOK;
+    T A[DIM * DIM];
+    if constexpr (DIM == 3)
+      affine3<T>(a.F + 9 * p, a.C + 9 * p, m, mu, lam, kind, a.inv_dx, a.dt, a.vol, textbook, A);
+    else
+      affine2<T>(a.F + 4 * p, a.C + 4 * p, m, mu, lam, kind, a.inv_dx, a.dt, a.vol, textbook, A);
+    T mv[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) mv[d] = a.v[DIM * p + d] * m;
+    const int64_t r1 = a.res + 1;
+    constexpr int K = DIM == 3 ? 3 : 1;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
       for (int j = 0; j < 3; ++j)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const T dp[3] = {(T(i) - fx[0]) * a.dx, (T(j) - fx[1]) * a.dx, (T(k) - fx[2]) * a.dx};
-          const T weight = w[0][i] * w[1][j] * w[2][k];
-          const int64_t node = ((int64_t)(base[0] + i) * r1 + (base[1] + j)) * r1 + (base[2] + k);
+        for (int k = 0; k < K; ++k) {
+          const int o[3] = {i, j, k};
+          T dp[DIM], weight = w[0][i] * w[1][j];
+          if constexpr (DIM == 3) weight *= w[2][k];
+          const bool inside = base[0] + i - low[0] < held;
+          uint32_t at = 0;  // (only used inside)
+          int64_t node = 0;
 #pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            const T ad = A[3 * d] * dp[0] + A[3 * d + 1] * dp[1] + A[3 * d + 2] * dp[2];
-            const T r = seg_reduce(weight * (mv[d] + ad), sg);
-            if (sg.tail) atomicAdd(a.grid_v + 3 * node + d, r);
+          for (int d = 0; d < DIM; ++d) {
+            dp[d] = (T(o[d]) - fx[d]) * a.dx;
+            at = at * (uint32_t)ext[d] + (uint32_t)(base[d] + o[d] - low[d]);
+            node = node * r1 + (base[d] + o[d]);
           }
-          const T rm = seg_reduce(weight * m, sg);
-          if (sg.tail) atomicAdd(a.grid_m + node, rm);
-        }
-  } else {
-    const WaveSeg sg = wave_segments(valid, (int)(base[0] * r1 + base[1]));
-    T A[4];
-    affine2<T>(a.F + 4 * p, a.C + 4 * p, m, mu, lam, kind, a.inv_dx, a.dt, a.vol, textbook, A);
-    if (!valid) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) A[e] = T(0);
+          for (int c = 0; c < NCH; ++c) {
+            T v = m;
+            if (c < DIM) {
+              T ad = A[DIM * c] * dp[0];
+#pragma unroll
+              for (int e = 1; e < DIM; ++e) ad += A[DIM * c + e] * dp[e];
+              v = mv[c] + ad;
+            }
+            v *= weight;
+            if (inside) atomicAdd(&arena[at * NCH + c], (double)v);
+            else if (c < DIM) atomicAdd(a.grid_v + DIM * node + c, v);
+            else atomicAdd(a.grid_m + node, v);
+          }
+        }
+  }
+  __syncthreads();
+  for (int e = t; e < words; e += THREADS) {
+    const T v = (T)arena[e];
+    if (v == T(0)) continue;
+    const int c = e % NCH;
+    int sl = e / NCH;
+    int64_t node = 0, stride = 1;
+#pragma unroll
+    for (int d = DIM - 1; d >= 0; --d) {
+      const int q = d > 0 ? sl % ext[d] : sl;
+      sl = d > 0 ? sl / ext[d] : 0;
+      node += (low[d] + q) * stride;
+      stride *= a.res + 1;
     }
-    const T mv[2] = {a.v[2 * p] * m, a.v[2 * p + 1] * m};
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const T dp[2] = {(T(i) - fx[0]) * a.dx, (T(j) - fx[1]) * a.dx};
-        const T weight = w[0][i] * w[1][j];
-        const int64_t node = (int64_t)(base[0] + i) * r1 + (base[1] + j);
-#pragma unroll
-        for (int d = 0; d < 2; ++d) {
-          const T ad = A[2 * d] * dp[0] + A[2 * d + 1] * dp[1];
-          const T r = seg_reduce(weight * (mv[d] + ad), sg);
-          if (sg.tail) atomicAdd(a.grid_v + 2 * node + d, r);
-        }
-        const T rm = seg_reduce(weight * m, sg);
-        if (sg.tail) atomicAdd(a.grid_m + node, rm);
-      }
+    if (c < DIM) atomicAdd(a.grid_v + DIM * node + c, v);
+    else atomicAdd(a.grid_m + node, v);
   }
 }
 
@@ -228,9 +285,9 @@ __global__ __launch_bounds__(RS_THREADS) void phase_keys_kernel(const T* __restr
 
 // P2G of particles in cell order (perm), summed per cell and workgroup
 // before memory (mpm_cellsum.h).  At 131,072 FP64 particles in arbitrary
-// order on a 64^3 grid the per-particle scatter of phase_p2g_kernel issues
-// 14 million device atomics and takes 1,426 us; sort and sums together take
-// about 80 us (p2g_sort_from has both forms by size).
+// order on a 64^3 grid a scatter with device atomics per particle issues 14
+// million of them and takes 1,426 us; sort and sums together take about 65 us
+// (p2g_sort_from compares it with phase_p2g_box_kernel by size).
 template <typename T, int DIM>
 __global__ __launch_bounds__(CELLSUM_THREADS) void phase_p2g_sorted_kernel(PhaseArgs<T> a,
                                                                          const uint32_t* __restrict__ perm) {
@@ -550,13 +607,14 @@ static PhaseArgs<T> make_args(const mpm_params* prm, const mpm_particles* p, int
 
 static inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
-// Smallest particle count of the sorted form, which pays for its sort (seven
-// small launches), where the direct one pays for its atomics.  Measured on
-// particles in arbitrary order, direct / sorted in us, at 2 and 16 per cell:
-//   3D FP64   2,048: 50 / 60, 78 / 53    8,192: 73 / 67, 106 / 59
-//           131,072: 781 / 87, 912 / 83   (FP32 1,189 / 96, 1,113 / 98)
-//   2D FP64  16,384: 40 / 60, 56 / 55   32,768: 57 / 60, 110 / 54
-//           131,072: 218 / 65, 326 / 66
+// Smallest particle count of the sorted form, which pays for its sort (six
+// small launches), where the other pays for its workgroups' boxes.  Measured on
+// particles in arbitrary order, box / sorted in us, at 2 and 16 per cell:
+//   3D FP64   2,048: 23 / 45, 17 / 38    8,192: 51 / 50, 20 / 41
+//            32,768: 193 / 61, 34 / 46   (FP32 226 / 57, 40 / 42)
+//           131,072: 772 / 72, 779 / 70
+//   2D FP64  16,384: 27 / 41, 10 / 34    32,768: 64 / 41, 15 / 35
+//           131,072: 198 / 50, 144 / 49
 static int64_t p2g_sort_from(int dim) { return dim == 3 ? 4096 : 24576; }
 
 // Cells of the key space, or 0 when the sorted form does not apply.
@@ -573,9 +631,9 @@ size_t phase_p2g_workspace_bytes(const mpm_params* prm, int64_t n) {
 
 template <typename T, int DIM>
 static void launch_p2g(hipStream_t st, const PhaseArgs<T>& a, int64_t key_space, void* work) {
-  const unsigned nb = blocks_for(a.n, 256);
   if (!work) {
-    hipLaunchKernelGGL((phase_p2g_kernel<T, DIM>), dim3(nb), dim3(256), 0, st, a);
+    constexpr int THREADS = BOX_THREADS_OF<DIM>;
+    hipLaunchKernelGGL((phase_p2g_box_kernel<T, DIM>), dim3(blocks_for(a.n, THREADS)), dim3(THREADS), 0, st, a);
     return;
   }
   uint32_t* keys = (uint32_t*)work;

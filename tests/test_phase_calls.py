@@ -110,3 +110,48 @@ def test_bin_ws_on_another_stream(gpu):
     side.synchronize()
     _lib.check(L.mpm_bin(None, 3, 64, 64.0, _lib.MPM_KEY_BLOCKED, x.data_ptr(), n, out[2].data_ptr(), out[3].data_ptr()))
     assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,n,res,spread", [
+    (2, 1, 40, 0.1),
+    (2, 511, 60, 0.5),      # one workgroup, not full
+    (2, 513, 60, 0.5),      # a second one of one particle
+    (2, 3000, 200, 0.9),    # the arena holds a part of the box
+    (3, 255, 20, 0.5),
+    (3, 257, 20, 0.5),
+    (3, 2000, 60, 0.8),
+    (3, 300, 150, 0.9),     # not one layer of it
+])
+@pytest.mark.parametrize("dtype", (torch.float32, torch.float64))
+def test_few_particles_match_oracle(gpu, dim, n, res, spread, dtype):
+    """P2G by workgroup boxes against the oracle's FP64 sums: 1e-12 of the
+    largest value in FP64; in FP32 2e-6 (some ten roundings of a contribution,
+    whose terms reach several times their sum) and 2e-7 res (x / dx rounds by
+    up to 6e-8 res cells, on each axis)."""
+    from oracle import mpm_oracle as O
+
+    rng, L, r1 = np.random.default_rng(n), _lib.load(), res + 1
+    x = 0.5 + spread * (rng.random((n, dim)) - 0.5)
+    up = lambda a: torch.tensor(np.ascontiguousarray(a), dtype=dtype, device=gpu)  # noqa: E731
+    x, v = up(x), up(rng.normal(size=(n, dim)))
+    F = up(np.eye(dim) + 0.02 * rng.normal(size=(n, dim, dim)))
+    C, Jp = up(rng.normal(size=(n, dim, dim))), up(np.ones((n, 1)))
+    mass, mu, lam = (up(np.full(n, a)) for a in (0.5, 3.0, 2.0))
+    sp = _phase.StagedParticles(x, v, F, C, Jp, mass, mu, lam)
+    prm = _phase.make_params(dim, res, float(res), 1.0 / res, 1e-4, 1e-4)
+    gv = torch.zeros((r1,) * dim + (dim,), dtype=dtype, device=gpu)
+    gm = torch.zeros((r1,) * dim, dtype=dtype, device=gpu)
+    p = sp.struct()
+    _lib.check(L.mpm_p2g(_stream(), ct.byref(prm), ct.byref(p), _lib.MPM_ELASTIC, 1.0, None, 0, gv.data_ptr(),
+                         gm.data_ptr(), None))
+    host = lambda a: a.double().cpu().numpy()  # noqa: E731
+    ev, em = np.zeros(gv.shape), np.zeros(gm.shape + (1,) * (dim == 3))
+    args = [host(a) for a in (x, v, F, C, Jp)]
+    if dim == 3:
+        O.p2g_3d(float(res), 1.0, 1 / res, 1e-4, 1e-4, ev, em, args[0], host(mass), host(mu), host(lam), *args[1:])
+    else:
+        O.p2g_2d(float(res), 1.0, 3.0, 2.0, 0.5, 1 / res, 1e-4, 1e-4, ev, em, *args)
+    bar = 2e-6 + 2e-7 * res if dtype == torch.float32 else 1e-12
+    for g, e in ((gv, ev), (gm, em.reshape(gm.shape))):
+        assert np.abs(host(g) - e).max() <= bar * np.abs(e).max()
