@@ -348,3 +348,26 @@ def test_mlp_gradients_at_row_edges(gpu, rows):
         torch.cuda.current_stream().cuda_stream, net.packed.data_ptr(), Xg.data_ptr(), rows, net.H1.data_ptr(),
         net.H2.data_ptr(), net.dY.data_ptr(), net.dH2.data_ptr(), net.dH1.data_ptr(), atomic.data_ptr()))
     assert float((atomic - net.grads).norm()) <= 1e-5 * float(net.grads.norm())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [127, 129, 32_768 + 17])
+def test_mlp_rows_beyond_a_turn(gpu, rows):
+    """Row counts around the 128 rows that a workgroup takes at a time and the
+    32,768 of one turn of every workgroup: the outputs of a row do not depend
+    on where it stands (equal to those of a call on the last rows alone), and
+    the gradients hold the bars of the test above."""
+    import torch
+
+    from femflow_amd.corrector import CorrectorMLP, to_bf16_features
+
+    X, T, w = _data(rows, 3)
+    p = _params(7)
+    net = CorrectorMLP(device=gpu, params=torch.from_numpy(p))
+    Xg = to_bf16_features(X, gpu)
+    Y = net.forward(Xg).clone()
+    tail = min(rows, 70)
+    assert torch.equal(Y[-tail:], net.forward(Xg[-tail:].contiguous())[:tail])
+    net.loss_grads(Xg, torch.tensor(T, dtype=torch.float32), torch.tensor(w, dtype=torch.float32))
+    _, gref, _ = M.loss_and_grads(p.astype(np.float64), X, T, w)
+    assert np.linalg.norm(net.grads.double().cpu().numpy() - gref) <= 1e-3 * np.linalg.norm(gref)
