@@ -221,9 +221,13 @@ __global__ void adj_grid_kernel(AdjArgs a) {
   const int64_t r1 = a.res + 1;
   const int64_t node = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (node >= r1 * r1 * r1) return;
-  float* gb = a.gbar + 4 * node;
+  float4* gb = reinterpret_cast<float4*>(a.gbar) + node;
+  const float4 in = *gb;
+  // most nodes of the dense grid have no particle near: nothing to reverse
+  // (and the cleared fourth value stands)
+  if (in.x == 0.f && in.y == 0.f && in.z == 0.f) return;
   const int64_t I[3] = {node / (r1 * r1), (node / r1) % r1, node % r1};
-  float ub[3] = {gb[0], gb[1], gb[2]};
+  float ub[3] = {in.x, in.y, in.z};
   if (a.boundary == MPM_BC_REFERENCE) {
 #pragma unroll
     for (int d = 0; d < 3; ++d)
@@ -248,10 +252,7 @@ __global__ void adj_grid_kernel(AdjArgs a) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) ub[d] *= im;
   }
-  gb[0] = ub[0];
-  gb[1] = ub[1];
-  gb[2] = ub[2];
-  gb[3] = mb;
+  *gb = make_float4(ub[0], ub[1], ub[2], mb);
 }
 
 // ---------------------------------------------------------------- P2G^T ----
@@ -293,7 +294,10 @@ __device__ __forceinline__ void polar_adjoint(const float F[9], const float R[9]
     for (int c = 0; c < 3; ++c) Fb[3 * r + c] += R[3 * r] * Y[c] + R[3 * r + 1] * Y[3 + c] + R[3 * r + 2] * Y[6 + c];
 }
 
-__global__ __launch_bounds__(128) void adj_p2g_kernel(AdjArgs a) {
+// A thread's 27 node adjoints are loaded together, ahead of the polar factor:
+// at 2^17 particles there are two waves per SIMD, and nine dependent rows were
+// latency (14.6 us per substep -> 13.2).
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void adj_p2g_kernel(AdjArgs a) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= a.n) return;
   int base[3];
@@ -302,6 +306,17 @@ __global__ __launch_bounds__(128) void adj_p2g_kernel(AdjArgs a) {
   float w[3][3], dw[3][3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) bspline_d(fx[d], w[d], dw[d]);
+  const int64_t r1 = a.res + 1;
+  float4 g[27];
+  {
+    const float4* g0 = reinterpret_cast<const float4*>(a.gbar) + (((int64_t)base[0] * r1 + base[1]) * r1 + base[2]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) g[9 * i + 3 * j + k] = g0[(i * r1 + j) * r1 + k];
+  }
   const int64_t mi = a.mat_scalar ? 0 : p;
   const float m = a.mass[mi];
   const float mu = a.mu0[mi] * a.hardening, lam = a.lam0[mi] * a.hardening;
@@ -336,20 +351,20 @@ __global__ __launch_bounds__(128) void adj_p2g_kernel(AdjArgs a) {
       }
   }
   const float mv[3] = {m * v[0], m * v[1], m * v[2]};
-  const int64_t r1 = a.res + 1;
   // gather
   float P[3] = {0.f, 0.f, 0.f}, Ab[9], gx[3] = {0.f, 0.f, 0.f};
 #pragma unroll
   for (int e = 0; e < 9; ++e) Ab[e] = 0.f;
+#pragma unroll
   for (int i = 0; i < 3; ++i)
+#pragma unroll
     for (int j = 0; j < 3; ++j)
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         const float wt = w[0][i] * w[1][j] * w[2][k];
-        const int64_t node = ((int64_t)(base[0] + i) * r1 + (base[1] + j)) * r1 + (base[2] + k);
-        const float* gb = a.gbar + 4 * node;
-        const float pb[3] = {gb[0], gb[1], gb[2]};
-        const float mb = gb[3];
+        const float4 gb = g[9 * i + 3 * j + k];
+        const float pb[3] = {gb.x, gb.y, gb.z};
+        const float mb = gb.w;
         const float dp[3] = {((float)i - fx[0]) * a.dx, ((float)j - fx[1]) * a.dx, ((float)k - fx[2]) * a.dx};
         float s = mb * m;
 #pragma unroll
@@ -422,9 +437,9 @@ __global__ __launch_bounds__(128) void adj_p2g_kernel(AdjArgs a) {
   }
 }
 
-__global__ void adj_fill_kernel(float* p, int64_t n, float v) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
+__global__ __launch_bounds__(256) void adj_clear_kernel(float4* __restrict__ p, int64_t n4) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n4) p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 __global__ void adj_copy_kernel(float* dst, const float* src, int64_t n) {
@@ -436,7 +451,7 @@ static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / 
 
 size_t adjoint_workspace_floats(int res) {
   const size_t r1 = (size_t)res + 1;
-  return 11 * r1 * r1 * r1;
+  return 11 * r1 * r1 * r1 + 3;  // forward grids, then the node adjoints on a 16-byte boundary
 }
 
 // Forward substep on the dense workspace: gp, gm = P2G; gv = grid update of gp.
@@ -446,7 +461,7 @@ void dense_forward_grids(hipStream_t st, const mpm_params* prm, const mpm_partic
   float* gp = work;
   float* gm = gp + 3 * nn;
   float* gv = gm + nn;
-  hipLaunchKernelGGL(adj_fill_kernel, dim3(nblk(4 * nn, 256)), dim3(256), 0, st, gp, 4 * nn, 0.f);
+  hipLaunchKernelGGL(adj_clear_kernel, dim3(nblk(nn, 256)), dim3(256), 0, st, (float4*)gp, nn);
   phase_p2g(st, prm, p, MPM_ELASTIC, hardening, nullptr, 0, gp, gm, oob);
   hipLaunchKernelGGL(adj_copy_kernel, dim3(nblk(3 * nn, 256)), dim3(256), 0, st, gv, gp, 3 * nn);
   phase_grid_op(st, prm, MPM_F32, gv, gm);
@@ -482,7 +497,7 @@ static void adjoint_from_grids(hipStream_t st, const mpm_params* prm, const mpm_
   a.gp = grids;
   a.gm = grids + 3 * nn;
   a.gv = grids + 4 * nn;
-  a.gbar = work + 7 * nn;
+  a.gbar = work + (7 * nn + 3) / 4 * 4;  // 16-byte records
   a.xb = xb;
   a.vb = vb;
   a.Fb = Fb;
@@ -490,7 +505,7 @@ static void adjoint_from_grids(hipStream_t st, const mpm_params* prm, const mpm_
   a.mub = mub;
   a.lamb = lamb;
   a.oob = oob;
-  hipLaunchKernelGGL(adj_fill_kernel, dim3(nblk(4 * nn, 256)), dim3(256), 0, st, a.gbar, 4 * nn, 0.f);
+  hipLaunchKernelGGL(adj_clear_kernel, dim3(nblk(nn, 256)), dim3(256), 0, st, (float4*)a.gbar, nn);
   if (a.n > 0) hipLaunchKernelGGL(adj_g2p_kernel, dim3(nblk(a.n, CELLSUM_THREADS)), dim3(CELLSUM_THREADS), 0, st,
                                   a);
   hipLaunchKernelGGL(adj_grid_kernel, dim3(nblk(nn, 256)), dim3(256), 0, st, a);

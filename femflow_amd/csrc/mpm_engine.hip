@@ -2068,9 +2068,11 @@ void Engine::enqueue_segment(int k0, int len, bool bin, hipStream_t s, double* s
     return a;
   };
   // the deferred FP64 particles are finished by the grid update unless the
-  // particles are read in between (cell-F sums, per-substep state output);
-  // per-substep state output also needs each substep's v and C in memory
-  const bool sep = corr_on || sink != nullptr;
+  // particles are read before it (cell-F sums); frames and per-substep states
+  // are written after it, which spares them a launch of its own that mostly
+  // finds an empty list (4.5 us a substep), and need each substep's v and C in
+  // memory
+  const bool sep = corr_on;
   store_vc = sink != nullptr;
   // step0: the run's index of this call's first substep
   if (k0 == 0) {
@@ -2079,20 +2081,20 @@ void Engine::enqueue_segment(int k0, int len, bool bin, hipStream_t s, double* s
     a0.rec = in_records ? rec_mem[0] : nullptr;  // a segment after an upload rebins
     pending_perm = nullptr;
     launch_transfer(cont ? 3 : 0, s, a0, sep);
+    if (corr_on) launch_cellf(s, args(sums, max_steps, 0));
+    launch_grid(s, grid_args(0), ws, len, 0, sep ? 0 : 1);
     if (cont) {  // the previous segment's last substep finished its G2P
       enqueue_frame(s, frames, step0 - 1);
       enqueue_state(s, sink, step0 - 1);
     }
-    if (corr_on) launch_cellf(s, args(sums, max_steps, 0));
-    launch_grid(s, grid_args(0), ws, len, 0, sep ? 0 : 1);
     if (corr_on) launch_corrector(s, args(sums, max_steps, 0), nullptr);
   }
   for (int k = k0 > 0 ? k0 : 1; k < k0 + len; ++k) {
     launch_transfer(1, s, args(sums, max_steps, k & 1), sep);
-    enqueue_frame(s, frames, step0 + k - k0 - 1);  // substep k-1 finished its G2P
-    enqueue_state(s, sink, step0 + k - k0 - 1);
     if (corr_on) launch_cellf(s, args(sums, max_steps, k & 1));
     launch_grid(s, grid_args(k), ws, len, k, sep ? 0 : 1);
+    enqueue_frame(s, frames, step0 + k - k0 - 1);  // substep k-1 finished its G2P
+    enqueue_state(s, sink, step0 + k - k0 - 1);
     if (corr_on) launch_corrector(s, args(sums, max_steps, k & 1), nullptr);
   }
   if (fin) {
