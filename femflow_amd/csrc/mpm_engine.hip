@@ -1943,7 +1943,7 @@ void Engine::enqueue_bin(hipStream_t s, int len, int with_sums) {
   pending_perm = vs;
   hipLaunchKernelGGL(block_bounds_kernel, dim3(nblk(n, 256)), dim3(256), 0, s, ks, n, d_bstart, d_bend, d_bocc);
   chunk_list(d_bocc, d_bstart, d_bend, d_block_scene, (int64_t)total_blocks, chunk, d_part, d_chunks, d_bfirst,
-             d_bcount, d_nchunks, dyn_sched, s);
+             d_bcount, d_nchunks, dyn_sched || corr_on, s);
   d_sorted_keys = ks;
   hipLaunchKernelGGL(cand_build_kernel, dim3(num_cus * 2), dim3(256), 0, s, args(nullptr, 0, 0), d_cand_list,
                      d_counters + 4, d_cand_flag);
