@@ -55,6 +55,7 @@ struct StateSink {
 struct TimedLaunch {
   int kind;  // 0 P2G, 1 G2P2G, 2 G2P, 3 grid update
   hipEvent_t e0, e1;
+  int launches;  // 0: a part of the launch that follows
 };
 
 struct Engine {
@@ -110,6 +111,8 @@ struct Engine {
   uint32_t* d_speeds = nullptr;
   uint32_t* h_speeds = nullptr;  // pinned: totals per class, then the sent flag
   int4* d_chunks = nullptr;
+  int4* d_split = nullptr;  // engines of many scenes: see EngineArgs::split
+  int64_t chunk_cap = 0;
   uint32_t *d_nchunks = nullptr, *d_keys = nullptr, *d_vals = nullptr,
            *d_bocc = nullptr, *d_part = nullptr;
   uint32_t* d_sorted_keys = nullptr;
@@ -140,6 +143,8 @@ struct Engine {
   void release();
   int alloc(void** p, size_t bytes);
   int init(int64_t n_max, int nscenes, const mpm_scene* sc, int nmat, const mpm_material* mats);
+  // small chunks in launches of their own
+  bool split_small() const { return d_split && chunk == 512 && spread == 9; }
   EngineArgs args(double* sums, int max_steps, int sel) const;
   int upload(const mpm_particles* p, const int32_t* scene_ids);
   int download(mpm_particles* p);

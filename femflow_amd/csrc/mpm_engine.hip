@@ -469,9 +469,22 @@ __device__ __forceinline__ int here(int v) {
 // a fixed interleave.  With tens of thousands of uneven chunks (many scenes
 // of different densities) the queue balances the tail; with a few thousand
 // the 8 contended counters cost more than they save, so only the fused pass
-// of multi-scene engines uses it.
-template <int MODE, int P, int SPREAD, bool DYN = false>
-__global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
+// of multi-scene engines uses it.  The first chunk of a workgroup needs no
+// ticket, and no more workgroups start than fit at once (three per compute
+// unit): with eight, each taking its first chunk from the queue, the launch
+// took 26 us over an empty list.
+//
+// WAVES: 4, or 1 for chunks of at most SMALL_CHUNK particles (chunk_list's
+// split).  A chunk takes 12 us from its first load to its last store however
+// few particles it has, at three workgroups per compute unit; with one wave
+// (no barriers, a table of its size) seven fit.  Fused pass of 64 scenes of
+// 16,384 particles on 32,768 blocks: 531 -> 364 us; of 64 scenes of 4,096 to
+// 262,144 particles (44% of the chunks small, 9% of the particles): 478 -> 424.
+// Row r of one wave sums its bounds as wave r of four does, so a chunk's scale
+// and its results are the same either way.
+template <int MODE, int P, int SPREAD, bool DYN = false, int WAVES = 4>
+__global__ __launch_bounds__(64 * WAVES) void transfer_kernel(EngineArgs a) {
+  constexpr int THREADS = 64 * WAVES;
   static_assert(SPREAD == 3 || SPREAD == 9, "scatter spread is 3 or 9");
   // The velocity arena (read by the G2P half) and the accumulation arena
   // (written by the P2G half after every gather of the chunk is done) share
@@ -482,7 +495,8 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
   float4* const vel_s = reinterpret_cast<float4*>(arena_s);
   unsigned long long(*const acc2)[MODE == 2 ? 1 : ACC_NODES] =
       reinterpret_cast<unsigned long long(*)[MODE == 2 ? 1 : ACC_NODES]>(arena_s);
-  __shared__ float red_s[ENG_THREADS / 64][4];
+  // bounds by wave, or by row of a single wave
+  __shared__ float red_s[WAVES == 1 ? P : WAVES][4];
   __shared__ ChunkScale cs;
   __shared__ uint32_t wg_oob, wg_fb;
   // P2G term table, four float4 per chunk entry, (fx0, fx1, fx2, m),
@@ -490,7 +504,7 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
   // time, and the arena cell of each entry (-1: not in the table).  Entry q
   // sits at slot q + q/16, which spreads the scatter phase's strided reads
   // over the banks.
-  constexpr int TAB = MODE == 2 ? 1 : P * ENG_THREADS;
+  constexpr int TAB = MODE == 2 ? 1 : P * THREADS;
   constexpr int TABS = TAB + TAB / 16;
   __shared__ float4 pt4[4][TABS];
   __shared__ int pb_s[TABS];
@@ -503,7 +517,16 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
   // before any wave counts into them (the first P2G has no barrier ahead of
   // its particle phase)
   __syncthreads();
-  const uint32_t nch = *a.nchunks;
+  // sums of one wave's bounds, which are cleared for its next row
+  auto sum_row = [&](int row, float(&bs)[4]) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const float m = warp_sum(bs[d]);
+      if (lane == 0) red_s[row][d] = m;
+      bs[d] = 0.f;
+    }
+  };
+  const uint32_t nch = WAVES == 1 ? a.nchunks[1] : (a.split ? a.nchunks[0] - a.nchunks[1] : a.nchunks[0]);
   const int xcd = blockIdx.x & 7;
   const int l = blockIdx.x >> 3;
   const int L = ((int)gridDim.x - xcd + 7) >> 3;
@@ -515,38 +538,58 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
   const SceneDev sc0 = a.scenes[0];
   __shared__ uint32_t next_s;
   uint32_t* const queue = a.counters + 8 + xcd;  // this XCD's ticket counter
-  if constexpr (DYN) {
-    if (t == 0) next_s = lo + atomicAdd(queue, 1u);
-    __syncthreads();
-  }
-  for (uint32_t c = DYN ? next_s : lo + (uint32_t)l; c < hi;) {
+  for (uint32_t c = lo + (uint32_t)l; c < hi;) {
     uint32_t nxt = 0u;
     if constexpr (DYN) {
-      if (t == 0) nxt = lo + atomicAdd(queue, 1u);  // in flight while this chunk runs
+      if (t == 0) nxt = lo + (uint32_t)L + atomicAdd(queue, 1u);  // in flight while this chunk runs
     }
-    const int4 ch = a.chunks[c];
+    int4 ch;
+    uint32_t id = c;  // its number: its place in the staging memory
+    if (WAVES == 1 || a.split) {
+      ch = a.split[WAVES == 1 ? a.split_cap - 1u - c : c];
+      id = (uint32_t)ch.w;
+      ch.w = (int)((uint32_t)ch.y >> SPLIT_COUNT_BITS);
+      ch.y &= (1 << SPLIT_COUNT_BITS) - 1;
+    } else {
+      ch = a.chunks[c];
+    }
     const SceneDev sc = one_scene ? sc0 : a.scenes[ch.w];
     const int local = ch.z - sc.block_base;
     const int nb = sc.nb;
     const int bi = local / (nb * nb), bj = (local / nb) % nb, bk = local % nb;
     const int O0 = bi * 4 - 1, O1 = bj * 4 - 1, O2 = bk * 4 - 1;
     if constexpr (MODE != 0) {
-      for (int e = here(t); e < ARENA_NODES; e += ENG_THREADS) {
+      // every load of the thread in flight before the first is stored (nodes
+      // off the grid read the block's first node instead)
+      constexpr int ROUNDS = ARENA_NODES / THREADS;
+      const int te = here(t);
+      float4 vn[ROUNDS];
+#pragma unroll
+      for (int r = 0; r < ROUNDS; ++r) {
+        const int e = te + r * THREADS;
         const int gi = O0 + (e >> 6), gj = O1 + ((e >> 3) & 7), gk = O2 + (e & 7);
         const bool in = gi >= 0 && gj >= 0 && gk >= 0 && gi <= sc.res && gj <= sc.res && gk <= sc.res;
-        vel_s[(e >> 6) * VEL_S0 + ((e >> 3) & 7) * VEL_S1 + (e & 7)] =
-            in ? a.vel[node_addr(sc, gi, gj, gk)] : make_float4(0.f, 0.f, 0.f, 0.f);
+        vn[r] = a.vel[in ? node_addr(sc, gi, gj, gk) : (size_t)ch.z * 64];
+        if (!in) vn[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+#pragma unroll
+      for (int r = 0; r < ROUNDS; ++r) {
+        const int e = te + r * THREADS;
+        vel_s[(e >> 6) * VEL_S0 + ((e >> 3) & 7) * VEL_S1 + (e & 7)] = vn[r];
       }
     }
     __syncthreads();
-    // Phase 1: particle q = r * ENG_THREADS + t of the chunk (coalesced).
+    // Phase 1: particle q = r * THREADS + t of the chunk (coalesced).
     // G2P modes gather, advance and store the particle; P2G modes then
     // compute its terms into the LDS term table (or send it down the global
     // path when it left the arena or its terms are not finite).
     float bsum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
     for (int r = 0; r < P; ++r) {
-      const int q = r * ENG_THREADS + t;
+      const int q = r * THREADS + t;
+      if constexpr (WAVES == 1 && MODE != 2) {
+        if (r > 0) sum_row(r - 1, bsum);  // (lanes reconverge here)
+      }
       if (q >= ch.y) continue;
       const int qs = q + (q >> 4);
       if constexpr (MODE != 2) pb_s[qs] = -1;
@@ -698,8 +741,13 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
 #pragma unroll
           for (int d = 0; d < 4; ++d) finite = finite && tfinite(b[d]);
           if (finite) {
+            if constexpr (WAVES == 1) {
 #pragma unroll
-            for (int d = 0; d < 4; ++d) bsum[d] += b[d];
+              for (int d = 0; d < 4; ++d) bsum[d] = b[d];
+            } else {
+#pragma unroll
+              for (int d = 0; d < 4; ++d) bsum[d] += b[d];
+            }
             pt4[0][qs] = make_float4(fx[0], fx[1], fx[2], tm.m);
             pt4[1][qs] = make_float4(tm.q0[0], tm.q0[1], tm.q0[2], tm.Adx[0]);
             pt4[2][qs] = make_float4(tm.Adx[1], tm.Adx[2], tm.Adx[3], tm.Adx[4]);
@@ -714,17 +762,19 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
     }
     if constexpr (MODE != 2) {
       // chunk-wide bound per channel -> fixed-point scales
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const float m = warp_sum(bsum[d]);
-        if (lane == 0) red_s[wv][d] = m;
-      }
+      sum_row(WAVES == 1 ? P - 1 : wv, bsum);
       __syncthreads();
-      for (int e = here(t); e < 2 * ACC_NODES; e += ENG_THREADS) acc2[0][e] = 0ull;
+      {
+        uint4* const acc4 = reinterpret_cast<uint4*>(arena_s);
+        const int te = here(t);
+#pragma unroll
+        for (int r = 0; r < ACC_NODES / THREADS; ++r) acc4[te + r * THREADS] = make_uint4(0u, 0u, 0u, 0u);
+        if (te < ACC_NODES % THREADS) acc4[te + ACC_NODES / THREADS * THREADS] = make_uint4(0u, 0u, 0u, 0u);
+      }
       if (t < 4) {
         float m = 0.f;
 #pragma unroll
-        for (int w2 = 0; w2 < ENG_THREADS / 64; ++w2) m += red_s[w2][t];
+        for (int w2 = 0; w2 < (WAVES == 1 ? P : WAVES); ++w2) m += red_s[w2][t];
         m *= 1.0001f;  // round-up margin for the FP32 sums above
         const float s = m > 0.f ? 1073741824.f / m : 1.f;  // 2^30 / bound
         cs.s[t] = s;
@@ -737,7 +787,7 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
       // node slabs (q mod 3), so their atomics hit different arena words.
       const float scl[4] = {cs.s[0], cs.s[1], cs.s[2], cs.s[3]};
       const int S = (ch.y + 63) >> 6;
-      const int PP = (S + 3) >> 2;  // <= P
+      const int PP = (S + WAVES - 1) / WAVES;  // <= P
 #pragma unroll 1
       for (int r = 0; r < PP; ++r) {
         const int jj = wv * PP + r;
@@ -821,10 +871,10 @@ __global__ __launch_bounds__(ENG_THREADS) void transfer_kernel(EngineArgs a) {
       }
       __syncthreads();
       const double inv[4] = {cs.inv[0], cs.inv[1], cs.inv[2], cs.inv[3]};
-      const bool staged = c < a.stage_cap;
-      float4* stage = a.stage + (size_t)c * STAGE_REC;
+      const bool staged = id < a.stage_cap;
+      float4* stage = a.stage + (size_t)id * STAGE_REC;
 #pragma unroll 1
-      for (int e = here(t); e < ARENA_NODES; e += ENG_THREADS) {
+      for (int e = here(t); e < ARENA_NODES; e += THREADS) {
         const int e0 = e >> 6, e1 = (e >> 3) & 7, e2 = e & 7;
         const int ph = e0 * ACC_S0 + e1 * ACC_S1 + e2;
         int q0, q1, q2, q3;
@@ -1771,7 +1821,9 @@ int Engine::init(int64_t n_max_, int nscenes, const mpm_scene* sc, int nmat_, co
   HIPCHK(hipHostMalloc((void**)&h_speeds, sizeof(uint32_t) * SPEED_WORDS, hipHostMallocDefault));
   // binning workspace
   const int64_t max_chunks = n / 256 + blocks + 1;
-  if ((rc = alloc((void**)&d_chunks, sizeof(int4) * (max_chunks < n + 1 ? max_chunks : n + 1)))) return rc;
+  chunk_cap = max_chunks < n + 1 ? max_chunks : n + 1;
+  if ((rc = alloc((void**)&d_chunks, sizeof(int4) * chunk_cap))) return rc;
+  if (dyn_sched && (rc = alloc((void**)&d_split, sizeof(int4) * chunk_cap))) return rc;
   if ((rc = alloc((void**)&d_nchunks, sizeof(uint32_t) * 4))) return rc;
   // staged P2G arenas: room for every chunk at the smallest chunk size unless
   // nearly every particle sits in its own block
@@ -1831,6 +1883,8 @@ EngineArgs Engine::args(double* sums, int max_steps, int sel) const {
   a.speeds_from = speeds_from;
   a.speeds_to = h_speeds;
   a.chunks = d_chunks;
+  a.split = split_small() ? d_split : nullptr;
+  a.split_cap = (uint32_t)chunk_cap;
   a.keys = d_sorted_keys;
   a.nchunks = d_nchunks;
   a.block_scene = d_block_scene;
@@ -1923,7 +1977,7 @@ void Engine::enqueue_bin(hipStream_t s, int len, int with_sums) {
   if (n <= 0) {
     hipLaunchKernelGGL(segment_begin_kernel, dim3(1), dim3(256), 0, s, args(nullptr, 0, 0), len,
                        with_sums, 1);
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, d_nchunks, (int64_t)1, 0u);
+    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, d_nchunks, (int64_t)2, 0u);
     return;
   }
   EngineArgs a = args(nullptr, 0, 0);
@@ -1943,7 +1997,7 @@ void Engine::enqueue_bin(hipStream_t s, int len, int with_sums) {
   pending_perm = vs;
   hipLaunchKernelGGL(block_bounds_kernel, dim3(nblk(n, 256)), dim3(256), 0, s, ks, n, d_bstart, d_bend, d_bocc);
   chunk_list(d_bocc, d_bstart, d_bend, d_block_scene, (int64_t)total_blocks, chunk, d_part, d_chunks, d_bfirst,
-             d_bcount, d_nchunks, dyn_sched || corr_on, s);
+             d_bcount, d_nchunks, dyn_sched || corr_on, d_split, chunk_cap, s);
   d_sorted_keys = ks;
   hipLaunchKernelGGL(cand_build_kernel, dim3(num_cus * 2), dim3(256), 0, s, args(nullptr, 0, 0), d_cand_list,
                      d_counters + 4, d_cand_flag);
@@ -1959,13 +2013,29 @@ void Engine::launch_transfer(int mode, hipStream_t s, const EngineArgs& a, bool 
     e0 = tevent();
     e1 = tevent();
   }
-#define MPM_LAUNCH_K(K)                                                                              \
+#define MPM_LAUNCH_G(K, G, T)                                                                        \
   do {                                                                                               \
     if (timing)                                                                                      \
-      hipExtLaunchKernelGGL(K, dim3(g), dim3(ENG_THREADS), 0, s, e0, e1, 0, a);                      \
+      hipExtLaunchKernelGGL(K, dim3(G), dim3(T), 0, s, e0, e1, 0, a);                                \
     else                                                                                             \
-      hipLaunchKernelGGL(K, dim3(g), dim3(ENG_THREADS), 0, s, a);                                    \
+      hipLaunchKernelGGL(K, dim3(G), dim3(T), 0, s, a);                                              \
   } while (0)
+#define MPM_LAUNCH_K(K) MPM_LAUNCH_G(K, g, ENG_THREADS)
+  // the small chunks of many scenes first, one wave each (seven per compute
+  // unit fit its LDS)
+#define MPM_LAUNCH_S(M) MPM_LAUNCH_G((transfer_kernel<M, 2, (M == 2 ? 3 : 9), false, 1>), num_cus * 7, 64)
+  if (split_small()) {
+    if (mode == 0) MPM_LAUNCH_S(0);
+    else if (mode == 1) MPM_LAUNCH_S(1);
+    else if (mode == 2) MPM_LAUNCH_S(2);
+    else MPM_LAUNCH_S(3);
+    if (timing) {
+      tpairs.push_back({mode == 3 ? 0 : mode, e0, e1, 0});
+      e0 = tevent();
+      e1 = tevent();
+    }
+  }
+#undef MPM_LAUNCH_S
 #define MPM_LAUNCH_T(M, PV)                                                                          \
   do {                                                                                               \
     if (M != 2 && spread == 9)                                                                       \
@@ -1973,8 +2043,8 @@ void Engine::launch_transfer(int mode, hipStream_t s, const EngineArgs& a, bool 
     else                                                                                             \
       MPM_LAUNCH_K((transfer_kernel<M, PV, 3>));                                                     \
   } while (0)
-  if (dyn_sched && mode == 1 && chunk == 512 && spread == 9) {
-    MPM_LAUNCH_K((transfer_kernel<1, 2, 9, true>));
+  if (split_small() && mode == 1) {
+    MPM_LAUNCH_G((transfer_kernel<1, 2, 9, true>), num_cus * (grid_mult < 3 ? grid_mult : 3), ENG_THREADS);
   } else if (chunk == 256) {
     if (mode == 0) MPM_LAUNCH_T(0, 1);
     else if (mode == 1) MPM_LAUNCH_T(1, 1);
@@ -1993,9 +2063,10 @@ void Engine::launch_transfer(int mode, hipStream_t s, const EngineArgs& a, bool 
   }
 #undef MPM_LAUNCH_T
 #undef MPM_LAUNCH_K
+#undef MPM_LAUNCH_G
   // timing slots: 0 the segment-start pass (P2G, or the moving fused pass),
   // 1 fused, 2 G2P (3 is the grid update's)
-  if (timing) tpairs.push_back({mode == 3 ? 0 : mode, e0, e1});
+  if (timing) tpairs.push_back({mode == 3 ? 0 : mode, e0, e1, 1});
   // one workgroup per CU: the usual empty list costs each workgroup one load,
   // and a violent step that defers tens of thousands of particles to FP64
   // (seen with dt several times the stable step) is spread over the chip
@@ -2012,7 +2083,7 @@ void Engine::launch_grid(hipStream_t s, const EngineArgs& a, int with_sums, int 
     e1 = tevent();
     hipExtLaunchKernelGGL(grid_update_kernel, dim3(g), dim3(ENG_THREADS), 0, s, e0, e1, 0, a, with_sums, len, k,
                           deferred);
-    tpairs.push_back({3, e0, e1});
+    tpairs.push_back({3, e0, e1, 1});
   } else {
     hipLaunchKernelGGL(grid_update_kernel, dim3(g), dim3(ENG_THREADS), 0, s, a, with_sums, len, k, deferred);
   }
@@ -2311,7 +2382,7 @@ int Engine::kernel_times(double* ms, int64_t* counts) {
     float t = 0;
     HIPCHK(hipEventElapsedTime(&t, tp.e0, tp.e1));
     ms[tp.kind] += t;
-    counts[tp.kind] += 1;
+    counts[tp.kind] += tp.launches;
   }
   tpairs.clear();
   tnext = 0;

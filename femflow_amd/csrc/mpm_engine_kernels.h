@@ -146,6 +146,11 @@ struct EngineArgs {
   const uint32_t* speeds_from;
   uint32_t* speeds_to;
   const int4* chunks;  // start, count, global block, scene (one per occupied block)
+  // the chunks again, for engines of many scenes (null: none): start, count |
+  // scene << SPLIT_COUNT_BITS, global block, number; the small ones (nchunks[1])
+  // from the end of split_cap entries, the others from the start
+  const int4* split;
+  uint32_t split_cap;
   const uint32_t* keys;  // binned (sorted) cell keys of the current order
   const uint32_t* nchunks;
   const int* block_scene;

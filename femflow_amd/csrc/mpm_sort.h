@@ -21,11 +21,15 @@ size_t radix_workspace_bytes(int64_t n);  // for any key space
 // of 256; start, count, b, block_scene[b]), numbered after those of the blocks
 // before it; bfirst[b]
 // and bcount[b] are its first chunk and chunk count (0 for empty blocks);
-// *nchunks = the total.  plain: equal chunks (see FEW_ROWS).  part: chunk_list_part_words(nblocks) words.
+// nchunks[0] = the total.  plain: equal chunks (see FEW_ROWS).  part:
+// chunk_list_part_words(nblocks) words.  split (may be null; plain only): the
+// chunks once more, those of at most SMALL_CHUNK particles (nchunks[1] of them)
+// from the end of its split_cap entries, the others from the start.
+constexpr int SMALL_CHUNK = 128, SPLIT_COUNT_BITS = 11;
 size_t chunk_list_part_words(int64_t nblocks);
 void chunk_list(const uint32_t* bocc, const uint32_t* bstart, const uint32_t* bend, const int* block_scene,
                 int64_t nblocks, int chunk, uint32_t* part, int4* chunks, uint32_t* bfirst, uint32_t* bcount,
-                uint32_t* nchunks, bool plain, hipStream_t st);
+                uint32_t* nchunks, bool plain, int4* split, int64_t split_cap, hipStream_t st);
 // The first pass's tile histogram inside the workspace, for a key kernel that
 // also counts the first digit (rs_tile_histogram, mpm_sort_dev.h) and passes
 // first_hist_done.

@@ -246,19 +246,19 @@ constexpr uint32_t FEW_ROWS = 384;
 // in dense blocks.  A block's pairs that would be less than 3/4 full stay
 // single (260 particles: 130 + 130, not 256 + 4).
 struct BlockRows {
-  uint32_t rows, chunks, dense;
+  uint32_t rows, chunks, dense, small;
 };
 __device__ __forceinline__ BlockRows block_rows(const uint32_t* __restrict__ bocc, const uint32_t* __restrict__ bstart,
                                                 const uint32_t* __restrict__ bend, int64_t b, uint32_t per_chunk,
                                                 int plain) {
-  if (!bocc[b]) return {0u, 0u, 0u};
+  if (!bocc[b]) return {0u, 0u, 0u, 0u};
   const uint32_t cnt = bend[b] - bstart[b], rows = (cnt + CHUNK_ROW - 1u) / CHUNK_ROW;
   if (plain) {
     const uint32_t c = (cnt + per_chunk * CHUNK_ROW - 1u) / (per_chunk * CHUNK_ROW);
-    return {c, c, 0u};
+    return {c, c, 0u, cnt <= (uint32_t)SMALL_CHUNK ? 1u : 0u};  // (a small block is one chunk)
   }
   const bool group = 4u * cnt >= 3u * CHUNK_ROW * rows;
-  return {rows, group ? (rows + per_chunk - 1u) / per_chunk : rows, cnt > GROUP_ABOVE ? rows : 0u};
+  return {rows, group ? (rows + per_chunk - 1u) / per_chunk : rows, cnt > GROUP_ABOVE ? rows : 0u, 0u};
 }
 
 __global__ __launch_bounds__(SCAN_THREADS) void block_tile_kernel(const uint32_t* __restrict__ bocc,
@@ -268,21 +268,22 @@ __global__ __launch_bounds__(SCAN_THREADS) void block_tile_kernel(const uint32_t
                                                                   uint4* __restrict__ part, int plain) {
   __shared__ uint32_t sh[SCAN_THREADS];
   const int64_t b = (int64_t)blockIdx.x * SCAN_THREADS + threadIdx.x;
-  const BlockRows r = b < nblocks ? block_rows(bocc, bstart, bend, b, per_chunk, plain) : BlockRows{0u, 0u, 0u};
-  uint32_t rows, chunks, dense;
+  const BlockRows r = b < nblocks ? block_rows(bocc, bstart, bend, b, per_chunk, plain) : BlockRows{0u, 0u, 0u, 0u};
+  uint32_t rows, chunks, dense, small;
   block_exclusive_scan(r.rows, sh, &rows);
   block_exclusive_scan(r.chunks, sh, &chunks);
   block_exclusive_scan(r.dense, sh, &dense);
-  if (threadIdx.x == 0) part[blockIdx.x] = make_uint4(rows, chunks, dense, 0u);
+  block_exclusive_scan(r.small, sh, &small);
+  if (threadIdx.x == 0) part[blockIdx.x] = make_uint4(rows, chunks, dense, small);
 }
 
 __global__ __launch_bounds__(SCAN_THREADS) void block_chunks_kernel(
     const uint32_t* __restrict__ bocc, const uint32_t* __restrict__ bstart, const uint32_t* __restrict__ bend,
     const int* __restrict__ block_scene, int64_t nblocks, uint32_t per_chunk, const uint4* __restrict__ part,
     int4* __restrict__ chunks, uint32_t* __restrict__ bfirst, uint32_t* __restrict__ bcount,
-    uint32_t* __restrict__ nchunks, int plain) {
+    uint32_t* __restrict__ nchunks, int plain, int4* __restrict__ split, uint32_t split_cap) {
   __shared__ uint32_t sh[SCAN_THREADS];
-  uint32_t rows_before = 0, chunks_before = 0, rows = 0, dense = 0;
+  uint32_t rows_before = 0, chunks_before = 0, small_before = 0, rows = 0, dense = 0;
   for (uint32_t q = threadIdx.x; q < gridDim.x; q += SCAN_THREADS) {
     const uint4 v = part[q];
     rows += v.x;
@@ -290,6 +291,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void block_chunks_kernel(
     if (q < blockIdx.x) {
       rows_before += v.x;
       chunks_before += v.y;
+      small_before += v.w;
     }
   }
   uint32_t rows_all, dense_all, before;
@@ -299,10 +301,16 @@ __global__ __launch_bounds__(SCAN_THREADS) void block_chunks_kernel(
   const bool single = !plain && (rows_all <= FEW_ROWS || 2u * dense_all < rows_all);
   block_exclusive_scan(single ? rows_before : chunks_before, sh, &before);
   const int64_t b = (int64_t)blockIdx.x * SCAN_THREADS + threadIdx.x;
-  const BlockRows r = b < nblocks ? block_rows(bocc, bstart, bend, b, per_chunk, plain) : BlockRows{0u, 0u, 0u};
+  const BlockRows r = b < nblocks ? block_rows(bocc, bstart, bend, b, per_chunk, plain) : BlockRows{0u, 0u, 0u, 0u};
   const uint32_t c = single ? r.rows : r.chunks;
   uint32_t tot;
   const uint32_t run = block_exclusive_scan(c, sh, &tot) + before;
+  uint32_t small_run = 0;
+  if (split) {
+    uint32_t small_all;
+    block_exclusive_scan(small_before, sh, &small_all);
+    small_run = block_exclusive_scan(r.small, sh, &tot) + small_all;
+  }
   if (b < nblocks) {
     bfirst[b] = run;
     bcount[b] = c;
@@ -313,10 +321,16 @@ __global__ __launch_bounds__(SCAN_THREADS) void block_chunks_kernel(
         const uint32_t r0 = r.rows * j / c, r1 = r.rows * (j + 1u) / c;  // its rows
         const uint32_t s0 = (uint32_t)(((uint64_t)cnt * r0) / r.rows), s1 = (uint32_t)(((uint64_t)cnt * r1) / r.rows);
         chunks[run + j] = make_int4((int)(p0 + s0), (int)(s1 - s0), (int)b, sc);
+        if (split)
+          split[r.small ? split_cap - 1u - small_run : run + j - small_run] =
+              make_int4((int)(p0 + s0), (int)((s1 - s0) | ((uint32_t)sc << SPLIT_COUNT_BITS)), (int)b, (int)(run + j));
       }
     }
   }
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == SCAN_THREADS - 1) *nchunks = run + c;
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == SCAN_THREADS - 1) {
+    nchunks[0] = run + c;
+    nchunks[1] = small_run + r.small;
+  }
 }
 
 // ---------------------------------------------------------------- keys ----
@@ -425,7 +439,7 @@ size_t chunk_list_part_words(int64_t nblocks) { return 4 * ((size_t)cdiv(nblocks
 
 void chunk_list(const uint32_t* bocc, const uint32_t* bstart, const uint32_t* bend, const int* block_scene,
                 int64_t nblocks, int chunk, uint32_t* part, int4* chunks, uint32_t* bfirst, uint32_t* bcount,
-                uint32_t* nchunks, bool plain, hipStream_t st) {
+                uint32_t* nchunks, bool plain, int4* split, int64_t split_cap, hipStream_t st) {
   if (nblocks <= 0) return;
   const unsigned tiles = (unsigned)cdiv(nblocks, SCAN_THREADS);
   const uint32_t per_chunk = (uint32_t)chunk / CHUNK_ROW;
@@ -433,7 +447,7 @@ void chunk_list(const uint32_t* bocc, const uint32_t* bstart, const uint32_t* be
   hipLaunchKernelGGL(block_tile_kernel, dim3(tiles), dim3(SCAN_THREADS), 0, st, bocc, bstart, bend, nblocks,
                      per_chunk, part4, plain ? 1 : 0);
   hipLaunchKernelGGL(block_chunks_kernel, dim3(tiles), dim3(SCAN_THREADS), 0, st, bocc, bstart, bend,
-                     block_scene, nblocks, per_chunk, part4, chunks, bfirst, bcount, nchunks, plain ? 1 : 0);
+                     block_scene, nblocks, per_chunk, part4, chunks, bfirst, bcount, nchunks, plain ? 1 : 0, split, (uint32_t)split_cap);
 }
 
 uint32_t* radix_first_hist(void* ws, int64_t n) { return (uint32_t*)ws + 2 * n; }
