@@ -131,7 +131,9 @@ template <typename T, int DIM, int NCH> struct CellSum {
       }
       unsigned long long m = __ballot(same);
       left &= ~m;
-      T a0 = T(0), a1 = T(0);
+      // FP64 also over the group: its members' terms are of one size, and in
+      // dense cells FP32 sums of them were most of the error
+      double a0 = 0.0, a1 = 0.0;
       const T* wave = sh.table + (t & ~63) * ENTRY;
       if constexpr (DIM == 3) {
 #pragma unroll 2
@@ -140,8 +142,8 @@ template <typename T, int DIM, int NCH> struct CellSum {
           m &= m - 1;
           const T w = tab[wi] * tab[wj] * tab[wk];
           const Row3 q0 = *reinterpret_cast<const Row3*>(tab + r0), q1 = *reinterpret_cast<const Row3*>(tab + r1);
-          a0 += w * (q0.x + q0.y * fi + q0.z * fj + q0.w * fk);
-          a1 += w * (q1.x + q1.y * fi + q1.z * fj + q1.w * fk);
+          a0 += (double)(w * (q0.x + q0.y * fi + q0.z * fj + q0.w * fk));
+          a1 += (double)(w * (q1.x + q1.y * fi + q1.z * fj + q1.w * fk));
         }
       } else {
         while (m) {  // two particles at a time, one per group of lanes
@@ -152,20 +154,20 @@ template <typename T, int DIM, int NCH> struct CellSum {
           const int p = sub == 0 ? p0 : p1;
           const T* tab = wave + (p < 0 ? p0 : p) * ENTRY;
           const T v = tab[wi] * tab[wj] * (tab[r0] + tab[r0 + 1] * fi + tab[r0 + 2] * fj);
-          a0 += p < 0 ? T(0) : v;
+          a0 += (double)(p < 0 ? T(0) : v);
         }
       }
       if (arena) {
         int at = (b[0] + i - sh.box[0]) * sh.box[DIM + 1] + (b[1] + j - sh.box[1]);
         if constexpr (DIM == 3) at = at * sh.box[DIM + 2] + (b[2] + k - sh.box[2]);
-        if (on0) atomicAdd(&sh.arena[at * NCH + c0], (double)a0);
-        if (on1) atomicAdd(&sh.arena[at * NCH + c0 + 1], (double)a1);
+        if (on0) atomicAdd(&sh.arena[at * NCH + c0], a0);
+        if (on1) atomicAdd(&sh.arena[at * NCH + c0 + 1], a1);
       } else {
         b[0] += i;
         b[1] += j;
         if constexpr (DIM == 3) b[2] += k;
-        if (on0) direct(b, c0, a0);
-        if (on1) direct(b, c0 + 1, a1);
+        if (on0) direct(b, c0, (T)a0);
+        if (on1) direct(b, c0 + 1, (T)a1);
       }
     }
   }
