@@ -422,8 +422,14 @@ __global__ void phase_planes_kernel(T* __restrict__ gv, int res, PlaneSet ps) {
   }
 }
 
+// A thread loads its stencil's velocities, all in flight together, with its F
+// (3D: whole rows of three nodes), before it uses the first: particles in
+// arbitrary order touch a line per load, so what bounds it is the address rate
+// and the latency of those loads, with two or three waves per SIMD at 2^17
+// particles.  131,072 FP64 particles 28.6 -> 22.6 us, 200,001
+// FP32 snow 34 -> 27.
 template <typename T, int DIM>
-__global__ void phase_g2p_kernel(PhaseArgs<T> a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void phase_g2p_kernel(PhaseArgs<T> a) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= a.n) return;
   int base[DIM];
@@ -432,13 +438,25 @@ __global__ void phase_g2p_kernel(PhaseArgs<T> a) {
     if (a.oob) atomicAdd(a.oob, 1ull);
     return;
   }
+  const int64_t r1 = a.res + 1;
+  constexpr int ROWS = DIM == 3 ? 9 : 3;
+  T g[ROWS][3 * DIM], Fp[DIM * DIM];
+#pragma unroll
+  for (int q = 0; q < ROWS; ++q) {
+    const T* row = a.grid_v;
+    if constexpr (DIM == 3) row += 3 * (((int64_t)(base[0] + q / 3) * r1 + (base[1] + q % 3)) * r1 + base[2]);
+    else row += 2 * ((int64_t)(base[0] + q) * r1 + base[1]);
+#pragma unroll
+    for (int e = 0; e < 3 * DIM; ++e) g[q][e] = row[e];
+  }
+#pragma unroll
+  for (int e = 0; e < DIM * DIM; ++e) Fp[e] = a.F[DIM * DIM * p + e];
   T w[DIM][3];
 #pragma unroll
   for (int d = 0; d < DIM; ++d) bspline(fx[d], w[d]);
   int kind;
   T h, tc, ts;
   material_of(a, p, kind, h, tc, ts);
-  const int64_t r1 = a.res + 1;
   const T c4 = T(4) * a.inv_dx;
   if constexpr (DIM == 3) {
     T v[3] = {0, 0, 0}, C[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -448,12 +466,11 @@ __global__ void phase_g2p_kernel(PhaseArgs<T> a) {
       for (int j = 0; j < 3; ++j)
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-          const int64_t node = ((int64_t)(base[0] + i) * r1 + (base[1] + j)) * r1 + (base[2] + k);
           const T weight = w[0][i] * w[1][j] * w[2][k];
           const T dp[3] = {T(i) - fx[0], T(j) - fx[1], T(k) - fx[2]};
 #pragma unroll
           for (int d = 0; d < 3; ++d) {
-            const T wg = weight * a.grid_v[3 * node + d];
+            const T wg = weight * g[3 * i + j][3 * k + d];
             v[d] += wg;
 #pragma unroll
             for (int e = 0; e < 3; ++e) C[3 * d + e] += c4 * (wg * dp[e]);
@@ -471,7 +488,7 @@ __global__ void phase_g2p_kernel(PhaseArgs<T> a) {
       M[i] = a.dt * C[i] + ((i % 4 == 0) ? T(1) : T(0));
       a.C[9 * p + i] = C[i];
     }
-    matmul3(M, a.F + 9 * p, Fn);
+    matmul3(M, Fp, Fn);
     if (kind == MPM_SNOW) {
       T U[9], s[3], V[9];
       svd3_checked<T>(Fn, U, s, V);
@@ -504,12 +521,11 @@ __global__ void phase_g2p_kernel(PhaseArgs<T> a) {
     for (int i = 0; i < 3; ++i)
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        const int64_t node = (int64_t)(base[0] + i) * r1 + (base[1] + j);
         const T weight = w[0][i] * w[1][j];
         const T dp[2] = {T(i) - fx[0], T(j) - fx[1]};
 #pragma unroll
         for (int d = 0; d < 2; ++d) {
-          const T wg = weight * a.grid_v[2 * node + d];
+          const T wg = weight * g[i][2 * j + d];
           v[d] += wg;
 #pragma unroll
           for (int e = 0; e < 2; ++e) C[2 * d + e] += c4 * (wg * dp[e]);
@@ -521,7 +537,6 @@ __global__ void phase_g2p_kernel(PhaseArgs<T> a) {
       a.v[2 * p + d] = v[d];
       xp[d] += a.dt * v[d];
     }
-    const T* Fp = a.F + 4 * p;
     const T M[4] = {T(1) + a.dt * C[0], a.dt * C[1], a.dt * C[2], T(1) + a.dt * C[3]};
     T Fn[4] = {M[0] * Fp[0] + M[1] * Fp[2], M[0] * Fp[1] + M[1] * Fp[3], M[2] * Fp[0] + M[3] * Fp[2],
                M[2] * Fp[1] + M[3] * Fp[3]};
