@@ -1123,7 +1123,7 @@ __global__ __launch_bounds__(ENG_THREADS) __attribute__((amdgpu_waves_per_eu(3))
   const uint32_t stride = gridDim.x * 4u;
   uint32_t b = blockIdx.x * 4u + (uint32_t)wv;
   uint32_t g_next = b < a.list_cap ? a.cand_list[b] : 0u;
-  uint2 src_next = b < a.list_cap && inner < 27 ? a.cand_src[(size_t)b * 32 + inner] : make_uint2(0u, 0u);
+  uint2 src_next = b < a.list_cap && inner < 28 ? a.cand_src[(size_t)b * 32 + inner] : make_uint2(0u, 0u);
   const uint32_t ncand = *a.cand_count;
   if (deferred) grid_deferred(a);
   const uint32_t count = ncand + *a.list_count;
@@ -1132,20 +1132,20 @@ __global__ __launch_bounds__(ENG_THREADS) __attribute__((amdgpu_waves_per_eu(3))
     const uint32_t g = cand ? g_next : a.list[b - ncand];
     const uint2 src = src_next;
     g_next = b + stride < a.list_cap ? a.cand_list[b + stride] : 0u;
-    src_next = b + stride < a.list_cap && inner < 27 ? a.cand_src[(size_t)(b + stride) * 32 + inner]
+    src_next = b + stride < a.list_cap && inner < 28 ? a.cand_src[(size_t)(b + stride) * 32 + inner]
                                                      : make_uint2(0u, 0u);
-    const int sid = one_scene ? 0 : a.block_scene[g];
-    const SceneDev sc = a.scenes[sid];
-    const int local = (int)g - sc.block_base;
-    const int nb = sc.nb;
-    const int bi = local / (nb * nb), bj = (local / nb) % nb, bk = local % nb;
+    // a candidate's scene comes with its table, so that nothing the arenas'
+    // loads need waits for it
+    const int sid = one_scene ? 0 : (cand ? __builtin_amdgcn_readlane((int)src.x, 27) : a.block_scene[g]);
     const int o0 = inner >> 4, o1 = (inner >> 2) & 3, o2 = inner & 3;
-    const int i = bi * 4 + o0, j = bj * 4 + o1, k = bk * 4 + o2;
     const size_t addr = (size_t)g * 64 + inner;
     // lanes 0..26: first chunk and chunk count of the 27 blocks around this
     // one (candidates: from the rebin's table; marked blocks: looked up)
     uint32_t my_c0 = src.x, my_cn = src.y;
     if (!cand && inner < 27) {
+      const SceneDev sc = a.scenes[sid];
+      const int local = (int)g - sc.block_base, nb = sc.nb;
+      const int bi = local / (nb * nb), bj = (local / nb) % nb, bk = local % nb;
       const uint2 nc = neighbour_chunks(a, sc, bi - 1 + inner / 9, bj - 1 + (inner / 3) % 3, bk - 1 + inner % 3);
       my_c0 = nc.x;
       my_cn = nc.y;
@@ -1189,6 +1189,11 @@ __global__ __launch_bounds__(ENG_THREADS) __attribute__((amdgpu_waves_per_eu(3))
       for (int c = 0; c < 2; ++c)
         sv[c][sn] = cn[sn] > (uint32_t)c ? src[(size_t)c * STAGE_REC] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
+    const SceneDev sc = a.scenes[sid];
+    const int local = (int)g - sc.block_base;
+    const int nb = sc.nb;
+    const int bi = local / (nb * nb), bj = (local / nb) % nb, bk = local % nb;
+    const int i = bi * 4 + o0, j = bj * 4 + o1, k = bk * 4 + o2;
 #pragma unroll
     for (int sn = 0; sn < 8; ++sn) {
 #pragma unroll
@@ -1384,7 +1389,7 @@ __global__ void cand_build_kernel(EngineArgs a, uint32_t* __restrict__ list, uin
 }
 
 // Per candidate entry (one wave each, lanes 0..26): the staged chunks of
-// its 27 neighbouring blocks.  They are fixed until the next rebin, so the
+// its 27 neighbouring blocks, and its scene (lane 27).  They are fixed until the next rebin, so the
 // grid update reads them together with the entry instead of looking them
 // up through the block's neighbours.
 __global__ void cand_src_kernel(EngineArgs a, uint2* __restrict__ out) {
@@ -1392,9 +1397,13 @@ __global__ void cand_src_kernel(EngineArgs a, uint2* __restrict__ out) {
   const int lane = threadIdx.x & 63;
   const uint32_t waves = gridDim.x * (blockDim.x >> 6);
   for (uint32_t b = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); b < ncand; b += waves) {
-    if (lane >= 27) continue;
+    if (lane >= 28) continue;
     const uint32_t g = a.cand_list[b];
     const int sid = a.nscenes == 1 ? 0 : a.block_scene[g];
+    if (lane == 27) {
+      out[(size_t)b * 32 + 27] = make_uint2((uint32_t)sid, 0u);
+      continue;
+    }
     const SceneDev sc = a.scenes[sid];
     const int local = (int)g - sc.block_base;
     const int nb = sc.nb;
