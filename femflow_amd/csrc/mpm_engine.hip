@@ -36,7 +36,7 @@ constexpr int VEL_S0 = 81, VEL_S1 = 9, VEL_NODES = 7 * VEL_S0 + 7 * VEL_S1 + 7 +
 // taken axis by axis (w = wi wj wk): per row (i, j) the k-sums
 // sum wk g and sum k wk g, per slab i their j-weighted sums, so each node
 // costs 5 FMAs instead of 13.
-template <bool FROM_LDS>
+template <bool FROM_LDS, int S0 = VEL_S0, int S1 = VEL_S1>
 __device__ __forceinline__ void gather(const float4* __restrict__ vel_s, int abase,
                                        const float4* __restrict__ vel, const SceneDev& sc,
                                        const int base[3], const float w[3][3], const float fx[3],
@@ -66,7 +66,7 @@ __device__ __forceinline__ void gather(const float4* __restrict__ vel_s, int aba
     const float wi = weight_at(fx[0], i);
     size_t Xi = 0;
     if (!FROM_LDS) Xi = i == 0 ? X[0] : (i == 1 ? X[1] : X[2]);
-    const int ai = abase + i * VEL_S0;
+    const int ai = abase + i * S0;
     // accumulators start from their first term (an FMA onto +0 cannot be
     // folded into a product under IEEE signed zeros)
     float Vi[3], Tj[3], Tk[3];
@@ -76,7 +76,7 @@ __device__ __forceinline__ void gather(const float4* __restrict__ vel_s, int aba
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         float4 g;
-        if (FROM_LDS) g = vel_s[ai + j * VEL_S1 + k];
+        if (FROM_LDS) g = vel_s[ai + j * S1 + k];
         else g = vel[gbase + Xi + Y[j] + Z[k]];
         const float gg[3] = {g.x, g.y, g.z};
 #pragma unroll
@@ -477,24 +477,29 @@ __device__ __forceinline__ int here(int v) {
 // WAVES: 4, or 1 for chunks of at most SMALL_CHUNK particles (chunk_list's
 // split).  A chunk takes 12 us from its first load to its last store however
 // few particles it has, at three workgroups per compute unit; with one wave
-// (no barriers, a table of its size) seven fit.  Fused pass of 64 scenes of
-// 16,384 particles on 32,768 blocks: 531 -> 364 us; of 64 scenes of 4,096 to
-// 262,144 particles (44% of the chunks small, 9% of the particles): 478 -> 424.
+// (no barriers, a table of its size, tighter arenas) nine fit.  Fused pass of 64 scenes of
+// 16,384 particles on 32,768 blocks: 531 -> 348 us; of 64 scenes of 4,096 to
+// 262,144 particles (44% of the chunks small, 9% of the particles): 478 -> 415.
 // Row r of one wave sums its bounds as wave r of four does, so a chunk's scale
 // and its results are the same either way.
 template <int MODE, int P, int SPREAD, bool DYN = false, int WAVES = 4>
 __global__ __launch_bounds__(64 * WAVES) void transfer_kernel(EngineArgs a) {
   constexpr int THREADS = 64 * WAVES;
+  // arena strides: a wave by itself meets few bank conflicts, and with the
+  // tighter layout nine instead of seven fit a compute unit
+  constexpr int VS0 = WAVES == 1 ? 65 : VEL_S0, VS1 = WAVES == 1 ? 8 : VEL_S1, VN = 7 * VS0 + 7 * VS1 + 8;
+  constexpr int AS0 = WAVES == 1 ? 65 : ACC_S0, AS1 = WAVES == 1 ? 8 : ACC_S1, AN = 7 * AS0 + 7 * AS1 + 8;
+  static_assert(VS1 >= 8 && VS0 >= 7 * VS1 + 8 && AS1 >= 8 && AS0 >= 7 * AS1 + 8 && VN <= AN, "one-to-one arenas");
   static_assert(SPREAD == 3 || SPREAD == 9, "scatter spread is 3 or 9");
   // The velocity arena (read by the G2P half) and the accumulation arena
   // (written by the P2G half after every gather of the chunk is done) share
   // one LDS region.
-  constexpr int VEL_WORDS = MODE == 0 ? 4 : 4 * VEL_NODES;
-  constexpr int ACC_WORDS = MODE == 2 ? 4 : 4 * ACC_NODES;
+  constexpr int VEL_WORDS = MODE == 0 ? 4 : 4 * VN;
+  constexpr int ACC_WORDS = MODE == 2 ? 4 : 4 * AN;
   __shared__ __align__(16) uint32_t arena_s[VEL_WORDS > ACC_WORDS ? VEL_WORDS : ACC_WORDS];
   float4* const vel_s = reinterpret_cast<float4*>(arena_s);
-  unsigned long long(*const acc2)[MODE == 2 ? 1 : ACC_NODES] =
-      reinterpret_cast<unsigned long long(*)[MODE == 2 ? 1 : ACC_NODES]>(arena_s);
+  unsigned long long(*const acc2)[MODE == 2 ? 1 : AN] =
+      reinterpret_cast<unsigned long long(*)[MODE == 2 ? 1 : AN]>(arena_s);
   // bounds by wave, or by row of a single wave
   __shared__ float red_s[WAVES == 1 ? P : WAVES][4];
   __shared__ ChunkScale cs;
@@ -575,7 +580,7 @@ __global__ __launch_bounds__(64 * WAVES) void transfer_kernel(EngineArgs a) {
 #pragma unroll
       for (int r = 0; r < ROUNDS; ++r) {
         const int e = te + r * THREADS;
-        vel_s[(e >> 6) * VEL_S0 + ((e >> 3) & 7) * VEL_S1 + (e & 7)] = vn[r];
+        vel_s[(e >> 6) * VS0 + ((e >> 3) & 7) * VS1 + (e & 7)] = vn[r];
       }
     }
     __syncthreads();
@@ -685,7 +690,7 @@ __global__ __launch_bounds__(64 * WAVES) void transfer_kernel(EngineArgs a) {
         for (int d = 0; d < 3; ++d) bspline(fx[d], w[d]);
         const int a0 = base[0] - O0, a1 = base[1] - O1, a2 = base[2] - O2;
         if (a0 >= 0 && a0 <= 5 && a1 >= 0 && a1 <= 5 && a2 >= 0 && a2 <= 5)
-          gather<true>(vel_s, a0 * VEL_S0 + a1 * VEL_S1 + a2, a.vel, sc, base, w, fx, v, C);
+          gather<true, VS0, VS1>(vel_s, a0 * VS0 + a1 * VS1 + a2, a.vel, sc, base, w, fx, v, C);
         else
           gather<false>(vel_s, 0, a.vel, sc, base, w, fx, v, C);
         const bool ok = advance(sc, mp, x, v, C, F, Jp);
@@ -752,7 +757,7 @@ __global__ __launch_bounds__(64 * WAVES) void transfer_kernel(EngineArgs a) {
             pt4[1][qs] = make_float4(tm.q0[0], tm.q0[1], tm.q0[2], tm.Adx[0]);
             pt4[2][qs] = make_float4(tm.Adx[1], tm.Adx[2], tm.Adx[3], tm.Adx[4]);
             pt4[3][qs] = make_float4(tm.Adx[5], tm.Adx[6], tm.Adx[7], tm.Adx[8]);
-            pb_s[qs] = a0 * ACC_S0 + a1 * ACC_S1 + a2;
+            pb_s[qs] = a0 * AS0 + a1 * AS1 + a2;
           } else {  // NaN/Inf terms keep their value through the float path
             inside = false;
           }
@@ -768,8 +773,8 @@ __global__ __launch_bounds__(64 * WAVES) void transfer_kernel(EngineArgs a) {
         uint4* const acc4 = reinterpret_cast<uint4*>(arena_s);
         const int te = here(t);
 #pragma unroll
-        for (int r = 0; r < ACC_NODES / THREADS; ++r) acc4[te + r * THREADS] = make_uint4(0u, 0u, 0u, 0u);
-        if (te < ACC_NODES % THREADS) acc4[te + ACC_NODES / THREADS * THREADS] = make_uint4(0u, 0u, 0u, 0u);
+        for (int r = 0; r < AN / THREADS; ++r) acc4[te + r * THREADS] = make_uint4(0u, 0u, 0u, 0u);
+        if (te < AN % THREADS) acc4[te + AN / THREADS * THREADS] = make_uint4(0u, 0u, 0u, 0u);
       }
       if (t < 4) {
         float m = 0.f;
@@ -827,7 +832,7 @@ __global__ __launch_bounds__(64 * WAVES) void transfer_kernel(EngineArgs a) {
             const int j = SPREAD == 9 ? (j0 + jj >= 3 ? j0 + jj - 3 : j0 + jj) : jj;
             w1r[jj] = SPREAD == 9 ? (j == 0 ? w1[0] : (j == 1 ? w1[1] : w1[2])) : w1[jj];
             fjr[jj] = (float)j;
-            jor[jj] = j * ACC_S1;
+            jor[jj] = j * AS1;
           }
         }
         // the three slabs unrolled: the scheduler interleaves one slab's
@@ -837,7 +842,7 @@ __global__ __launch_bounds__(64 * WAVES) void transfer_kernel(EngineArgs a) {
           const int i = i0 + sl >= 3 ? i0 + sl - 3 : i0 + sl;
           const float wi = weight_at(fx0, i);
           const float fi = (float)i;
-          const int ai = pb + i * ACC_S0;
+          const int ai = pb + i * AS0;
           float qi[3];
 #pragma unroll
           for (int d = 0; d < 3; ++d) qi[d] = q0s[d] + A0s[d] * fi;
@@ -876,7 +881,7 @@ __global__ __launch_bounds__(64 * WAVES) void transfer_kernel(EngineArgs a) {
 #pragma unroll 1
       for (int e = here(t); e < ARENA_NODES; e += THREADS) {
         const int e0 = e >> 6, e1 = (e >> 3) & 7, e2 = e & 7;
-        const int ph = e0 * ACC_S0 + e1 * ACC_S1 + e2;
+        const int ph = e0 * AS0 + e1 * AS1 + e2;
         int q0, q1, q2, q3;
         unpack_fixed2(acc2[0][ph], q1, q0);
         unpack_fixed2_nn(acc2[1][ph], q2, q3);
@@ -2030,9 +2035,9 @@ void Engine::launch_transfer(int mode, hipStream_t s, const EngineArgs& a, bool 
       hipLaunchKernelGGL(K, dim3(G), dim3(T), 0, s, a);                                              \
   } while (0)
 #define MPM_LAUNCH_K(K) MPM_LAUNCH_G(K, g, ENG_THREADS)
-  // the small chunks of many scenes first, one wave each (seven per compute
+  // the small chunks of many scenes first, one wave each (nine per compute
   // unit fit its LDS)
-#define MPM_LAUNCH_S(M) MPM_LAUNCH_G((transfer_kernel<M, 2, (M == 2 ? 3 : 9), false, 1>), num_cus * 7, 64)
+#define MPM_LAUNCH_S(M) MPM_LAUNCH_G((transfer_kernel<M, 2, (M == 2 ? 3 : 9), false, 1>), num_cus * 9, 64)
   if (split_small()) {
     if (mode == 0) MPM_LAUNCH_S(0);
     else if (mode == 1) MPM_LAUNCH_S(1);
