@@ -86,8 +86,9 @@ class Engine:
 
     def tune(self, chunk: int = 512, sort_every: int = 48, grid_mult: int = 8, use_graph: bool = True,
              spread: int = 9):
-        """chunk: binned particles per work item (256, 512, 1024); sort_every:
-        substeps between rebinning; grid_mult: persistent workgroups per CU;
+        """chunk: binned particles per work item, at most (256, 512, 1024);
+        sort_every: substeps between rebinning, at most (fewer where the
+        particles' speeds make that cheaper); grid_mult: persistent workgroups per CU;
         use_graph: replay the substep sequence as a captured hipGraph;
         spread: scatter start offsets per cell (9, or 3: the narrower
         rotation, slower where many particles share a cell)."""
@@ -222,7 +223,8 @@ class Engine:
 
     def request_rebin(self):
         """Rebin the particles at the start of the next run (the engine otherwise
-        rebins after an upload and then every sort_every substeps, across calls)."""
+        rebins after an upload and then at least every sort_every substeps,
+        across calls)."""
         _lib.check(self._L.mpm_ctx_request_rebin(self._h), "request_rebin")
 
     def particle_sums(self):

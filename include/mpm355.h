@@ -170,8 +170,9 @@ int32_t mpm_ctx_create(mpm_ctx** out, int64_t n_max, int32_t nscenes, const mpm_
                        int32_t nmat, const mpm_material* materials, int32_t flags);
 int32_t mpm_ctx_destroy(mpm_ctx* ctx);
 int32_t mpm_ctx_set_stream(mpm_ctx* ctx, void* stream);
-/* Tunables: chunk = particles per work item (256, 512 or 1024); sort_every =
- * substeps between rebinning (>= 1); grid_mult = persistent workgroups per CU;
+/* Tunables: chunk = particles per work item, at most (256, 512 or 1024);
+ * sort_every = substeps between rebinning, at most (>= 1; fewer where the
+ * particles' speeds make that cheaper); grid_mult = persistent workgroups per CU;
  * use_graph = capture and replay the substep sequence as a hipGraph.  A new
  * context starts at chunk 512, sort_every 48, grid_mult 8, graphs on. */
 int32_t mpm_ctx_tune(mpm_ctx* ctx, int32_t chunk, int32_t sort_every, int32_t grid_mult,
@@ -236,8 +237,8 @@ int32_t mpm_ctx_fallback_count(mpm_ctx* ctx, int64_t* out);
  * per-node term of the algorithmic byte count. */
 int32_t mpm_ctx_active_blocks(mpm_ctx* ctx, int64_t* out);
 /* Rebin the particles at the start of the next mpm_run.  The engine rebins
- * after every upload and then every sort_every substeps, counting across
- * calls; this restarts that count.  No reference counterpart. */
+ * after every upload and then at the latest every sort_every substeps,
+ * counting across calls; this restarts that count.  No reference counterpart. */
 int32_t mpm_ctx_request_rebin(mpm_ctx* ctx);
 /* FP64 sums over the engine's particles: out[0] = sum m, out[1..3] = sum m v,
  * out[4..6] = sum m x (host double[7]). Synchronises the stream. */
