@@ -74,6 +74,10 @@ struct Engine {
   bool speeds_uploaded = false;  // an upload's counts wait for the next run
   bool speeds_waited = false;    // the last run's do, and the host has waited for that run
   const uint32_t* speeds_from = nullptr;  // see EngineArgs; set while a probing segment is enqueued
+  // a run's first kernel may still send its counts to h_speeds: the host's wait
+  // for them ran out.  Until they are there no other run asks for counts, so that
+  // what arrives is always the asking run's own.
+  bool speeds_pending = false;
   // set while a segment with per-substep state output is enqueued: the fused
   // pass then writes v and C every substep
   bool store_vc = false;

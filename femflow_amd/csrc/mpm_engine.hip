@@ -1695,6 +1695,9 @@ __global__ void particle_sums_kernel(EngineState s, int64_t n, double* out) {
 // 110 / 98, 2^21 213 / 200, 5,000,000 899 / 462.
 constexpr int64_t TWO_PASS_DOWNLOAD = 1 << 20;
 
+// Longest time that a run's host thread waits for the speed counts.
+constexpr std::chrono::milliseconds PROBE_WAIT(200);
+
 static inline unsigned nblk(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
 #define HIPCHK(expr)                                                                 \
@@ -2234,14 +2237,24 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
   // substeps are enqueued by themselves; the host waits for the counts while
   // the GPU works on those, and the cadence then holds for the rest of the
   // run (and until new counts).  The counts follow program order, so a
-  // sequence of calls always takes the same rebins.
+  // sequence of calls takes the same rebins each time, unless the caller's
+  // stream holds back the run's first kernel for longer than PROBE_WAIT: the
+  // run then keeps the cadence that it had.
   bool probe = (speeds_uploaded || speeds_waited) && n > 0 && nsteps > MIN_CADENCE && sort_every > MIN_CADENCE && !sums;
   if (probe) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     HIPCHK(hipStreamIsCapturing(user_stream, &cap));
     probe = cap == hipStreamCaptureStatusNone;
   }
-  if (probe) __atomic_store_n(h_speeds + SPEED_CLASSES, 0u, __ATOMIC_RELEASE);
+  uint32_t* const sent = h_speeds + SPEED_CLASSES;
+  if (probe && speeds_pending) {
+    speeds_pending = !__atomic_load_n(sent, __ATOMIC_ACQUIRE);
+    probe = !speeds_pending;
+  }
+  if (probe) {
+    __atomic_store_n(sent, 0u, __ATOMIC_RELEASE);
+    speeds_pending = true;  // (also if an error ends the run before its wait)
+  }
   speeds_from = probe ? d_speeds + (speeds_uploaded ? SPEED_SET : 0) : nullptr;
   const bool from_upload = speeds_uploaded;
   speeds_uploaded = speeds_waited = false;
@@ -2311,14 +2324,13 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
     if (probe) {
       probe = false;
       speeds_from = nullptr;
-      uint32_t* const sent = h_speeds + SPEED_CLASSES;
       // bounded: work that the caller's stream waits for may come from this
       // very thread, after the call
       const auto start = std::chrono::steady_clock::now();
-      while (!__atomic_load_n(sent, __ATOMIC_ACQUIRE) &&
-             std::chrono::steady_clock::now() - start < std::chrono::seconds(1))
+      while (!__atomic_load_n(sent, __ATOMIC_ACQUIRE) && std::chrono::steady_clock::now() - start < PROBE_WAIT)
         __builtin_ia32_pause();
-      if (__atomic_load_n(sent, __ATOMIC_ACQUIRE)) cadence = cadence_of(h_speeds);
+      speeds_pending = !__atomic_load_n(sent, __ATOMIC_ACQUIRE);
+      if (!speeds_pending) cadence = cadence_of(h_speeds);
     }
   }
   HIPCHK(hipEventRecord(ev_out, own_stream));

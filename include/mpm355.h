@@ -200,7 +200,12 @@ int32_t mpm_state_upload(mpm_ctx* ctx, const mpm_particles* p, const int32_t* sc
 int32_t mpm_state_download(mpm_ctx* ctx, mpm_particles* p);
 /* Advance every scene by nsteps substeps.  If sums != NULL (device double,
  * nsteps * 8 entries) each substep writes FP64 [grid mass, grid momentum x3
- * after P2G, grid momentum x3 after the update, number of nodes with mass]. */
+ * after P2G, grid momentum x3 after the update, number of nodes with mass].
+ * The call returns before the work is done, but the first run of more than 8
+ * substeps after an upload or the reading of a counter waits on the host until its
+ * first kernel has run (it reads the particles' speeds, see sort_every): at
+ * most 0.2 s, after which it goes on with the schedule it had.  The same holds
+ * for mpm_run_frames and mpm_run_states. */
 int32_t mpm_run(mpm_ctx* ctx, int32_t nsteps, double* sums);
 /* Like mpm_run (no sums), also writing each substep's positions in the
  * caller's order to frames (device float, nsteps * n * 3): the per-step frame
