@@ -71,8 +71,10 @@ struct Engine {
   // substeps between rebins for the speeds last seen (cadence_of; 0: none
   // seen, sort_every applies, which also bounds it)
   int cadence = 0;
-  bool speeds_uploaded = false;  // an upload's counts wait for the next run
-  bool speeds_waited = false;    // the last run's do, and the host has waited for that run
+  // Counts for the next run that is long enough to use them: none, of the last
+  // run (the host has waited for it, or it was too short to use the ones that it
+  // found), of an upload
+  enum { SPEEDS_NONE, SPEEDS_RUN, SPEEDS_UPLOAD } speeds_at = SPEEDS_NONE;
   const uint32_t* speeds_from = nullptr;  // see EngineArgs; set while a probing segment is enqueued
   // a run's first kernel may still send its counts to h_speeds: the host's wait
   // for them ran out.  Until they are there no other run asks for counts, so that

@@ -1945,7 +1945,7 @@ int Engine::upload(const mpm_particles* p, const int32_t* scene_ids) {
   in_records = n > 0;
   if (n > 0) {
     uint32_t* speeds = d_speeds + SPEED_SET;
-    if (speeds_uploaded) fill_u32(own_stream, speeds, SPEED_SET, 0u);  // a second upload without a run
+    if (speeds_at == SPEEDS_UPLOAD) fill_u32(own_stream, speeds, SPEED_SET, 0u);  // a second upload without a run
     const UploadArgs u{d_scenes,           speeds,
                        (const float*)p->x, (const float*)p->v,
                        (const float*)p->F, (const float*)p->C,
@@ -1953,7 +1953,7 @@ int Engine::upload(const mpm_particles* p, const int32_t* scene_ids) {
                        (const float*)p->mu0, (const float*)p->lambda0,
                        p->material,        scene_ids,
                        p->mat_scalar,      (int)scenes_host.size()};
-    speeds_uploaded = true;
+    speeds_at = SPEEDS_UPLOAD;
     cadence = 0;
     hipLaunchKernelGGL(upload_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[0], rec_mem[0], n, u);
   }
@@ -2233,14 +2233,15 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
   }
   if (nsteps == 0) return MPM_OK;
   // Probe (adaptive cadence): the run's first kernel sends the counts of the upload, or of the
-  // run before if the host has waited for that, and the first MIN_CADENCE
+  // run before (speeds_at), and the first MIN_CADENCE
   // substeps are enqueued by themselves; the host waits for the counts while
   // the GPU works on those, and the cadence then holds for the rest of the
   // run (and until new counts).  The counts follow program order, so a
   // sequence of calls takes the same rebins each time, unless the caller's
   // stream holds back the run's first kernel for longer than PROBE_WAIT: the
   // run then keeps the cadence that it had.
-  bool probe = (speeds_uploaded || speeds_waited) && n > 0 && nsteps > MIN_CADENCE && sort_every > MIN_CADENCE && !sums;
+  bool probe =
+      speeds_at != SPEEDS_NONE && n > 0 && nsteps > MIN_CADENCE && sort_every > MIN_CADENCE && !sums;
   if (probe) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     HIPCHK(hipStreamIsCapturing(user_stream, &cap));
@@ -2255,9 +2256,11 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
     __atomic_store_n(sent, 0u, __ATOMIC_RELEASE);
     speeds_pending = true;  // (also if an error ends the run before its wait)
   }
-  speeds_from = probe ? d_speeds + (speeds_uploaded ? SPEED_SET : 0) : nullptr;
-  const bool from_upload = speeds_uploaded;
-  speeds_uploaded = speeds_waited = false;
+  const bool from_upload = speeds_at == SPEEDS_UPLOAD;
+  speeds_from = probe ? d_speeds + (from_upload ? SPEED_SET : 0) : nullptr;
+  // counts that this run does not get to use are cleared by its first kernel,
+  // and its own take their place
+  if (speeds_at != SPEEDS_NONE) speeds_at = n > 0 ? SPEEDS_RUN : SPEEDS_NONE;
   HIPCHK(hipEventRecord(ev_in, user_stream));
   HIPCHK(hipStreamWaitEvent(own_stream, ev_in, 0));
   if (sums) {
@@ -2330,7 +2333,10 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
       while (!__atomic_load_n(sent, __ATOMIC_ACQUIRE) && std::chrono::steady_clock::now() - start < PROBE_WAIT)
         __builtin_ia32_pause();
       speeds_pending = !__atomic_load_n(sent, __ATOMIC_ACQUIRE);
-      if (!speeds_pending) cadence = cadence_of(h_speeds);
+      if (!speeds_pending) {
+        cadence = cadence_of(h_speeds);
+        speeds_at = SPEEDS_NONE;
+      }
     }
   }
   HIPCHK(hipEventRecord(ev_out, own_stream));
@@ -2372,7 +2378,7 @@ int Engine::take_counter(int which, int64_t* out) {
   unsigned long long v = 0;
   unsigned long long* p = which == 0 ? d_oob : d_fallback;
   HIPCHK(hipMemcpy(&v, p, sizeof(v), hipMemcpyDeviceToHost));
-  speeds_waited = !speeds_uploaded;  // the last run is over: its speeds can be had at once
+  if (speeds_at == SPEEDS_NONE) speeds_at = SPEEDS_RUN;  // the last run is over: its speeds can be had at once
   // cleared on the engine's own stream, ahead of its later work
   hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, own_stream, reinterpret_cast<uint32_t*>(p),
                      (int64_t)2, 0u);

@@ -42,3 +42,29 @@ def test_late_counts_reach_no_other_run(gpu, first, second, segments):
         _upload(eng, states[0])
         assert _segments(eng, 48) == (6 if first > 0.1 else 1)
     eng.close()
+
+
+@pytest.mark.parametrize("short", [(5,), (5, 2), (8, 8, 1)])
+def test_counts_outlast_runs_too_short_to_use_them(gpu, short):
+    """Unchecked runs of at most 8 substeps after an upload cannot use its
+    counts; the first longer one then uses those of the run before it, and
+    rebins as it would have right after the upload: 8 substeps (from the order
+    of the short runs), then by the fast particles' cadence of 8."""
+    fast = _state(gpu, 0.2)
+    eng = _engine(48)
+    _upload(eng, fast)
+    for k in short:
+        eng.run(k, check_oob=False)
+    assert _segments(eng, 48) == 1 + 5
+    eng.close()
+
+
+def test_recorded_sums_leave_the_counts(gpu):
+    """A run that records sums keeps its schedule in one piece; the next one
+    follows the speeds."""
+    fast = _state(gpu, 0.2)
+    eng = _engine(48)
+    _upload(eng, fast)
+    eng.run(12, sums=torch.empty(12, 8, dtype=torch.float64, device=gpu), check_oob=False)
+    assert _segments(eng, 48) == 1 + 5
+    eng.close()
