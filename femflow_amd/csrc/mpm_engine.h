@@ -155,8 +155,9 @@ struct Engine {
   int upload(const mpm_particles* p, const int32_t* scene_ids);
   int download(mpm_particles* p);
   void tiled();
-  // rebin; also starts the segment of len substeps (counters, sums index)
-  void enqueue_bin(hipStream_t s, int len, int with_sums);
+  // rebin; also starts the segment of len substeps (counters, sums index;
+  // keep_speeds: not the speed counts, for a segment that is no part of a run)
+  void enqueue_bin(hipStream_t s, int len, int with_sums, bool keep_speeds = false);
   void enqueue_segment(int k0, int len, bool bin, hipStream_t s, double* sums, int max_steps, float* frames,
                        int64_t step0, const StateSink* sink, bool cont, bool fin);
   // destroy every captured graph (after anything they baked in changes)

@@ -1031,8 +1031,9 @@ __device__ __forceinline__ void segment_begin(uint32_t* counters, int len, int w
 }
 
 // The segment start's part of the speed counts, by one workgroup: totals to
-// the host where it asked for them, then both sets cleared.
+// the host where it asked for them, then both sets cleared (speeds null: kept).
 __device__ __forceinline__ void segment_speeds(const EngineArgs& a) {
+  if (!a.speeds) return;
   const int t = threadIdx.x;
   if (a.speeds_from) {
     if (t < SPEED_CLASSES) {
@@ -1990,14 +1991,14 @@ int Engine::download(mpm_particles* p) {
 // Keys -> stable radix sort -> block ranges -> chunk list -> candidate blocks
 // and their neighbour table.  The particles themselves move into the new
 // order in the segment's first P2G (through pending_perm).
-void Engine::enqueue_bin(hipStream_t s, int len, int with_sums) {
+void Engine::enqueue_bin(hipStream_t s, int len, int with_sums, bool keep_speeds) {
+  EngineArgs a = args(nullptr, 0, 0);
+  if (keep_speeds) a.speeds = nullptr;
   if (n <= 0) {
-    hipLaunchKernelGGL(segment_begin_kernel, dim3(1), dim3(256), 0, s, args(nullptr, 0, 0), len,
-                       with_sums, 1);
+    hipLaunchKernelGGL(segment_begin_kernel, dim3(1), dim3(256), 0, s, a, len, with_sums, 1);
     hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, d_nchunks, (int64_t)2, 0u);
     return;
   }
-  EngineArgs a = args(nullptr, 0, 0);
   const RadixPlan pl = radix_plan(n, (uint32_t)(total_blocks * 64 - 1));
 #define MPM_KEYS(I)                                                                                                  \
   hipLaunchKernelGGL((engine_keys_kernel<I>), dim3((unsigned)pl.tiles), dim3(RS_THREADS), 0, s, a, n, d_keys, d_bocc, \

@@ -139,7 +139,7 @@ struct EngineArgs {
   uint32_t* other_hard;  // the other parity's count (cleared by the grid update)
   uint32_t* defer_ticket;  // counters[7]: start order of the grid update's workgroups
   // class counts, SPEED_COPIES rows of SPEED_WORDS each: of the run's last
-  // G2P, then of the upload; a segment's start clears both
+  // G2P, then of the upload; a segment's start clears both (unless null)
   uint32_t* speeds;
   // the set whose totals a run's first kernel sends to the host (null: none)
   // and where to (pinned; word SPEED_CLASSES is set last)

@@ -68,3 +68,21 @@ def test_recorded_sums_leave_the_counts(gpu):
     eng.run(12, sums=torch.empty(12, 8, dtype=torch.float64, device=gpu), check_oob=False)
     assert _segments(eng, 48) == 1 + 5
     eng.close()
+
+
+@pytest.mark.parametrize("after_run", [False, True])
+def test_a_sample_leaves_the_counts(gpu, after_run):
+    """One P2G and grid update between an upload (or a checked run) and a run
+    leaves the counts that the run reads: the fast particles' cadence of 8 from
+    the sample's order on."""
+    from femflow_amd.corrector import CorrectorMLP
+
+    fast = _state(gpu, 0.2)
+    eng = _engine(48)
+    eng.set_corrector(torch.zeros_like(CorrectorMLP(device=gpu).params), 1e-6, 1.0, enable=False)
+    _upload(eng, fast)
+    if after_run:
+        eng.run(4)
+    eng.p2g_grid_only()
+    assert _segments(eng, 48) == 6
+    eng.close()
