@@ -34,6 +34,12 @@ struct GraphKey {
 constexpr size_t MAX_GRAPHS = 32;
 // Shortest rebin cadence the engine takes by itself.
 constexpr int MIN_CADENCE = 8;
+// Substeps for which a cadence below sort_every holds without new counts.
+// Bodies that slowed down since would pay for rebins that they do not need: at
+// most 24 of some 75 us (a run of 1,000 substeps of a body that stops early
+// would pay for 125).  Bodies that stay fast go on as with sort_every until a
+// run that reads counts (after a counter was read, as Engine.run does).
+constexpr int CADENCE_HOLDS = 192;
 
 struct CorrExtract {
   uint16_t* X;      // rows x 352 BF16 features
@@ -71,6 +77,7 @@ struct Engine {
   // substeps between rebins for the speeds last seen (cadence_of; 0: none
   // seen, sort_every applies, which also bounds it)
   int cadence = 0;
+  int cadence_left = 0;  // substeps for which it still holds; taken back at a rebin
   // Counts for the next run that is long enough to use them: none, of the last
   // run (the host has waited for it, or it was too short to use the ones that it
   // found), of an upload

@@ -2236,8 +2236,8 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
   // Probe (adaptive cadence): the run's first kernel sends the counts of the upload, or of the
   // run before (speeds_at), and the first MIN_CADENCE
   // substeps are enqueued by themselves; the host waits for the counts while
-  // the GPU works on those, and the cadence then holds for the rest of the
-  // run (and until new counts).  The counts follow program order, so a
+  // the GPU works on those, and the cadence then holds for CADENCE_HOLDS
+  // substeps (or until new counts).  The counts follow program order, so a
   // sequence of calls takes the same rebins each time, unless the caller's
   // stream holds back the run's first kernel for longer than PROBE_WAIT: the
   // run then keeps the cadence that it had.
@@ -2286,9 +2286,13 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
   // also moves the particles into the new order.
   int done = 0, k0 = 0;  // k0: substeps of the current segment already enqueued
   while (done < nsteps) {
-    const int every = cadence > 0 && cadence < sort_every ? cadence : sort_every;
+    int every = cadence > 0 && cadence < sort_every ? cadence : sort_every;
     const bool bin = n <= 0 || since_bin < 0 || since_bin >= every;
     if (bin) k0 = 0;
+    if (bin && cadence > 0 && cadence_left <= 0) {
+      cadence = 0;
+      every = sort_every;
+    }
     int len = bin ? every : every - since_bin;
     if (probe && len > MIN_CADENCE) len = MIN_CADENCE;
     if (len > nsteps - done) len = nsteps - done;
@@ -2323,6 +2327,7 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
     in_records = false;
     since_bin = bin ? len : since_bin + len;
     k0 += len;
+    cadence_left -= cadence_left > 0 ? len : 0;
     last_list = (k0 - 1) & 1;
     done += len;
     if (probe) {
@@ -2336,6 +2341,7 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
       speeds_pending = !__atomic_load_n(sent, __ATOMIC_ACQUIRE);
       if (!speeds_pending) {
         cadence = cadence_of(h_speeds);
+        cadence_left = CADENCE_HOLDS;
         speeds_at = SPEEDS_NONE;
       }
     }

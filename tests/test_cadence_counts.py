@@ -86,3 +86,26 @@ def test_a_sample_leaves_the_counts(gpu, after_run):
     eng.p2g_grid_only()
     assert _segments(eng, 48) == 6
     eng.close()
+
+
+@pytest.mark.parametrize("split", [False, True])
+def test_a_cadence_ends_without_new_counts(gpu, split):
+    """Moving particles, counted after the upload only: the cadence K that the
+    counts give holds for the 8 substeps while they are read and 192 more, up to
+    the rebin after them, in one call or two; then sort_every."""
+    s = _state(gpu, 0.05)
+    eng = _engine(48)
+    _upload(eng, s)
+    per48 = _segments(eng, 48)
+    assert 2 <= per48 <= 4  # 24, 16 or 12
+    K = 48 // per48
+    held = -(-200 // K)  # segments
+    _upload(eng, s)
+    eng.kernel_timing(True)
+    for k in (held * K, 480 - held * K) if split else (480,):
+        eng.run(k, check_oob=False)
+    got = eng.kernel_times()["p2g"][1]
+    eng.kernel_timing(False)
+    assert got == held - (-(480 - held * K) // 48)
+    assert eng.oob_count() == 0
+    eng.close()
