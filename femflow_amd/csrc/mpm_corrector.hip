@@ -492,6 +492,7 @@ int Engine::corrector_sample(uint16_t* X, uint32_t* nodes, float* vel, int64_t m
   }
   enqueue_bin(s, 1, 0, true);  // also starts the one-substep segment
   since_bin = 0;  // freshly binned: the next run continues from this order
+  chunks_plain = true;
   const EngineArgs a = args(nullptr, 0, 0);
   {
     EngineArgs a0 = a;

@@ -74,6 +74,9 @@ struct Engine {
   // fused passes take chunks from per-XCD ticket queues (set for engines of
   // 8 or more scenes, whose many uneven chunks the queue balances)
   bool dyn_sched = false;
+  // the chunk list in use was built without regard to rows (see FEW_ROWS in
+  // mpm_sort.hip), as the corrector needs it
+  bool chunks_plain = false;
   // substeps between rebins for the speeds last seen (cadence_of; 0: none
   // seen, sort_every applies, which also bounds it)
   int cadence = 0;

@@ -2287,7 +2287,7 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
   int done = 0, k0 = 0;  // k0: substeps of the current segment already enqueued
   while (done < nsteps) {
     int every = cadence > 0 && cadence < sort_every ? cadence : sort_every;
-    const bool bin = n <= 0 || since_bin < 0 || since_bin >= every;
+    const bool bin = n <= 0 || since_bin < 0 || since_bin >= every || (corr_on && !chunks_plain);
     if (bin) k0 = 0;
     if (bin && cadence > 0 && cadence_left <= 0) {
       cadence = 0;
@@ -2326,6 +2326,7 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
     HIPCHK(hipGetLastError());
     in_records = false;
     since_bin = bin ? len : since_bin + len;
+    if (bin) chunks_plain = dyn_sched || corr_on;
     k0 += len;
     cadence_left -= cadence_left > 0 ? len : 0;
     last_list = (k0 - 1) & 1;
