@@ -167,9 +167,7 @@ class EngineStepper:
         return x, v, F, C
 
     def check_oob(self):
-        n = self.eng.oob_count()
-        if n:
-            raise RuntimeError(f"{n} particle stencil(s) left the grid")  # three_d/p2g.py:51-52
+        self.eng.check_oob()
 
     def close(self):
         self.eng.close()

@@ -148,11 +148,7 @@ class Engine:
         _lib.check(self._L.mpm_run(self._h, int(nsteps), None if sums is None else sums.data_ptr()),
                    "run")
         if check_oob:
-            n = self.oob_count()
-            if n >= 1 << 40:  # the grid update's wait for the FP64 pass ran out
-                raise RuntimeError("the FP64 pass for deferred particles did not finish in time")
-            if n:
-                raise RuntimeError(f"{n} particle stencil(s) left the grid")
+            self.check_oob()
 
     def run_states(self, nsteps: int, x, v, F, C, Jp, check_oob: bool = True, grids=None):
         """Advance ``nsteps`` substeps, writing the full state after substep k
@@ -179,9 +175,7 @@ class Engine:
                                                     F.data_ptr(), C.data_ptr(), Jp.data_ptr(), grids.data_ptr()),
                        "run_states")
         if check_oob:
-            k = self.oob_count()
-            if k:
-                raise RuntimeError(f"{k} particle stencil(s) left the grid")
+            self.check_oob()
 
     def run_frames(self, nsteps: int, frames: torch.Tensor, check_oob: bool = True):
         """Advance ``nsteps`` substeps, writing each substep's positions (caller
@@ -192,9 +186,7 @@ class Engine:
         self._sync_stream()
         _lib.check(self._L.mpm_run_frames(self._h, int(nsteps), frames.data_ptr()), "run_frames")
         if check_oob:
-            n = self.oob_count()
-            if n:
-                raise RuntimeError(f"{n} particle stencil(s) left the grid")
+            self.check_oob()
 
     def positions(self, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Current positions in the caller's order, (N, 3) float32 on the device."""
@@ -209,6 +201,15 @@ class Engine:
         out = ct.c_int64()
         _lib.check(self._L.mpm_ctx_oob_count(self._h, ct.byref(out)), "oob_count")
         return int(out.value)
+
+    def check_oob(self):
+        """Raise if a particle's stencil left its grid (three_d/p2g.py:51-52)
+        since the count was last read, or a grid update gave up its wait."""
+        n = self.oob_count()
+        if n >= 1 << 40:  # the grid update's wait for the FP64 pass ran out
+            raise RuntimeError("the FP64 pass for deferred particles did not finish in time")
+        if n:
+            raise RuntimeError(f"{n} particle stencil(s) left the grid")
 
     def fallback_count(self) -> int:
         out = ct.c_int64()

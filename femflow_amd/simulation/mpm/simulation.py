@@ -224,9 +224,7 @@ class MPMSimulation(SimulationBase):
             if pending is not None:
                 convert(*pending)  # overlaps this chunk's substeps
             pending = (slot, k)
-            oob = self.engine.oob_count()
-            if oob:
-                raise RuntimeError(f"{oob} particle stencil(s) left the grid")
+            self.engine.check_oob()
             done += k
             j += 1
         if pending is not None:
