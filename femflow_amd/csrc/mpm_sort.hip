@@ -317,9 +317,11 @@ __global__ __launch_bounds__(SCAN_THREADS) void block_chunks_kernel(
     if (c) {
       const uint32_t p0 = bstart[b], cnt = bend[b] - p0;
       const int sc = block_scene[b];
-      for (uint32_t j = 0; j < c; ++j) {
-        const uint32_t r0 = r.rows * j / c, r1 = r.rows * (j + 1u) / c;  // its rows
-        const uint32_t s0 = (uint32_t)(((uint64_t)cnt * r0) / r.rows), s1 = (uint32_t)(((uint64_t)cnt * r1) / r.rows);
+      uint32_t s0 = 0, s1;
+      for (uint32_t j = 0; j < c; ++j, s0 = s1) {
+        // its rows end at r1 (64 bits: rows^2 leaves 32 from 2^24 particles in one block on)
+        const uint32_t r1 = (uint32_t)((uint64_t)r.rows * (j + 1u) / c);
+        s1 = (uint32_t)((uint64_t)cnt * r1 / r.rows);
         chunks[run + j] = make_int4((int)(p0 + s0), (int)(s1 - s0), (int)b, sc);
         if (split)
           split[r.small ? split_cap - 1u - small_run : run + j - small_run] =
