@@ -77,9 +77,16 @@ __device__ __forceinline__ void bspline_d(float fx, float w[3], float dw[3]) {
 // in flight together, and keeps them for both uses (v', C' and the weight
 // derivatives): at 2^17 particles there are two waves per SIMD, so a chain
 // of nine dependent rows, twice, was latency, and 243 lane-shuffle sums per
-// particle were most of the rest (68 us per substep -> 28).
+// particle were most of the rest (68 us per substep -> 24).
+// Row-major cell order gives a workgroup a strip of cells, which wraps where a
+// row of the body ends: boxes are larger than those of the phase P2G's blocks.
+// The arena's LDS is spare (registers hold two workgroups per compute unit):
+// 576 / 1,024 / 2,048 nodes, before the particles drift, at 8 per cell: 4,096 on
+// 64^3 20 / 19 / 20 us, 131,072 on 64^3 45 / 29 / 30, 885,000 on 128^3 283 / 150 /
+// 159 (with FP32 sums of 1,024 nodes by runs of lanes 41, 54, 243).
+constexpr int ADJ_ARENA = 1024;
 __global__ __launch_bounds__(CELLSUM_THREADS) __attribute__((amdgpu_waves_per_eu(2))) void adj_g2p_kernel(AdjArgs a) {
-  using Sum = CellSum<float, 3, 3>;
+  using Sum = CellSum<float, 3, 3, ADJ_ARENA>;
   __shared__ __align__(16) Sum::Shared sh;
   // lanes past the end or out of the grid stay in the wave and write nothing
   const int64_t p0 = (int64_t)blockIdx.x * CELLSUM_THREADS + threadIdx.x;

@@ -25,7 +25,13 @@ namespace mpm {
 
 constexpr int CELLSUM_THREADS = 256;
 
-template <typename T, int DIM, int NCH> struct CellSum {
+// ARENA: nodes of the LDS arena; a workgroup whose box is larger adds each
+// group's sums to memory.  FP64 for FP32 particles too, since LDS adds of floats
+// run at a third of a lane per cycle and those of doubles at about five (131,072
+// FP32 particles, sort included, 80 -> 65 us at 2 per cell and 83 -> 64 at 16, with
+// an arena of 1,024 FP32 nodes before).  576 leaves room for two workgroups of the
+// phase P2G (FP64, 3D) per compute unit, whose particles come in blocks of cells.
+template <typename T, int DIM, int NCH, int ARENA = 576> struct CellSum {
   static constexpr int NODES = DIM == 3 ? 27 : 9;
   static constexpr int ROW = DIM == 3 ? 4 : 3;  // q, A[0..DIM-1] of a channel
   // per-particle table entry: NCH rows, then DIM x 3 weights, padded to 16
@@ -33,12 +39,6 @@ template <typename T, int DIM, int NCH> struct CellSum {
   static constexpr int PAD = 16 / (int)sizeof(T);
   static constexpr int ENTRY = (NCH * ROW + 3 * DIM + PAD - 1) / PAD * PAD;
   typedef T Row3 __attribute__((ext_vector_type(4), aligned(16)));
-  // nodes; FP64 for FP32 particles too, since LDS adds of floats run at a
-  // third of a lane per cycle and those of doubles at about five (131,072 FP32
-  // particles, sort included, 80 -> 65 us at 2 per cell and 83 -> 64 at 16,
-  // with an arena of 1,024 FP32 nodes before)
-  static constexpr int ARENA = 576;
-
   struct alignas(16) Shared {
     T table[CELLSUM_THREADS * ENTRY];
     double arena[ARENA * NCH];
