@@ -23,8 +23,8 @@ size_t radix_workspace_bytes(int64_t n);  // for any key space
 // and bcount[b] are its first chunk and chunk count (0 for empty blocks);
 // nchunks[0] = the total.  plain: equal chunks (see FEW_ROWS).  part:
 // chunk_list_part_words(nblocks) words.  split (may be null; plain only): the
-// chunks once more, those of at most SMALL_CHUNK particles (nchunks[1] of them)
-// from the end of its split_cap entries, the others from the start.
+// chunks once more, those of at most SMALL_CHUNK particles (nchunks[1] of them, 0
+// if they are few) from the end of its split_cap entries, the others from the start.
 constexpr int SMALL_CHUNK = 128, SPLIT_COUNT_BITS = 11;
 size_t chunk_list_part_words(int64_t nblocks);
 void chunk_list(const uint32_t* bocc, const uint32_t* bstart, const uint32_t* bend, const int* block_scene,

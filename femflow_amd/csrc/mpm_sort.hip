@@ -241,6 +241,14 @@ constexpr uint32_t GROUP_ABOVE = 18 * 64;
 // another fixed-point scale now and then moves a light node's velocity gradient
 // by 1e-3 (262,144 particles in 5,400 cells: no difference in time).
 constexpr uint32_t FEW_ROWS = 384;
+// Small chunks go to the launch of their own (split) from this many on, one round
+// of four-wave workgroups (three per compute unit): fewer find room beside the
+// others, and a second pass over the few takes longer than they do there.  Us per
+// substep of engines at 16 particles per cell, all apart / none: 8 scenes of
+// 16,384 (231 small of 619 chunks) 46 / 36, 16 of 32,768 (16 of 1,483) 76 / 61; at
+// 1 per cell, all chunks small, 8 scenes of 4,096 (959) 29 / 37, 8 of 32,768 (5,743)
+// 69 / 107.  (Before there was a second launch: 43, 69, 55, 124.)
+constexpr uint32_t APART_FROM = 768;
 
 // Of a block (or their sums over a tile): rows, chunks with rows grouped, rows
 // in dense blocks.  A block's pairs that would be less than 3/4 full stay
@@ -283,11 +291,12 @@ __global__ __launch_bounds__(SCAN_THREADS) void block_chunks_kernel(
     int4* __restrict__ chunks, uint32_t* __restrict__ bfirst, uint32_t* __restrict__ bcount,
     uint32_t* __restrict__ nchunks, int plain, int4* __restrict__ split, uint32_t split_cap) {
   __shared__ uint32_t sh[SCAN_THREADS];
-  uint32_t rows_before = 0, chunks_before = 0, small_before = 0, rows = 0, dense = 0;
+  uint32_t rows_before = 0, chunks_before = 0, small_before = 0, rows = 0, dense = 0, small = 0;
   for (uint32_t q = threadIdx.x; q < gridDim.x; q += SCAN_THREADS) {
     const uint4 v = part[q];
     rows += v.x;
     dense += v.z;
+    small += v.w;
     if (q < blockIdx.x) {
       rows_before += v.x;
       chunks_before += v.y;
@@ -301,15 +310,17 @@ __global__ __launch_bounds__(SCAN_THREADS) void block_chunks_kernel(
   const bool single = !plain && (rows_all <= FEW_ROWS || 2u * dense_all < rows_all);
   block_exclusive_scan(single ? rows_before : chunks_before, sh, &before);
   const int64_t b = (int64_t)blockIdx.x * SCAN_THREADS + threadIdx.x;
-  const BlockRows r = b < nblocks ? block_rows(bocc, bstart, bend, b, per_chunk, plain) : BlockRows{0u, 0u, 0u, 0u};
+  BlockRows r = b < nblocks ? block_rows(bocc, bstart, bend, b, per_chunk, plain) : BlockRows{0u, 0u, 0u, 0u};
   const uint32_t c = single ? r.rows : r.chunks;
   uint32_t tot;
   const uint32_t run = block_exclusive_scan(c, sh, &tot) + before;
   uint32_t small_run = 0;
   if (split) {
-    uint32_t small_all;
-    block_exclusive_scan(small_before, sh, &small_all);
-    small_run = block_exclusive_scan(r.small, sh, &tot) + small_all;
+    uint32_t small_all, first;
+    block_exclusive_scan(small, sh, &small_all);
+    if (small_all < APART_FROM) r.small = small_before = 0u;
+    block_exclusive_scan(small_before, sh, &first);
+    small_run = block_exclusive_scan(r.small, sh, &tot) + first;
   }
   if (b < nblocks) {
     bfirst[b] = run;
