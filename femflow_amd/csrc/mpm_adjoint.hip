@@ -80,10 +80,10 @@ __device__ __forceinline__ void bspline_d(float fx, float w[3], float dw[3]) {
 // particle were most of the rest (68 us per substep -> 24).
 // Row-major cell order gives a workgroup a strip of cells, which wraps where a
 // row of the body ends: boxes are larger than those of the phase P2G's blocks.
-// The arena's LDS is spare (registers hold two workgroups per compute unit):
-// 576 / 1,024 / 2,048 nodes, before the particles drift, at 8 per cell: 4,096 on
-// 64^3 20 / 19 / 20 us, 131,072 on 64^3 45 / 29 / 30, 885,000 on 128^3 283 / 150 /
-// 159 (with FP32 sums of 1,024 nodes by runs of lanes 41, 54, 243).
+// 576 / 1,024 / 2,048 nodes, with registers for two workgroups per compute unit, at
+// 8 per cell: 4,096 on 64^3 20 / 19 / 20 us, 131,072 on 64^3 45 / 29 / 30, 885,000
+// on 128^3 283 / 150 / 159 (with FP32 sums of 1,024 nodes by runs of lanes 41, 54,
+// 243).  Registers (167) and LDS now hold three: 20, 29, 116.
 constexpr int ADJ_ARENA = 1024;
 __global__ __launch_bounds__(CELLSUM_THREADS) __attribute__((amdgpu_waves_per_eu(2))) void adj_g2p_kernel(AdjArgs a) {
   using Sum = CellSum<float, 3, 3, ADJ_ARENA>;
@@ -171,6 +171,10 @@ __global__ __launch_bounds__(CELLSUM_THREADS) __attribute__((amdgpu_waves_per_eu
   // x' = x + dt v'
 #pragma unroll
   for (int d = 0; d < 3; ++d) vt[d] = vo[d] + a.dt * xo[d];
+  auto add = [&](const int* b, int c, float v) {
+    atomicAdd(a.gbar + 4 * (((int64_t)b[0] * r1 + b[1]) * r1 + b[2]) + c, v);
+  };
+  bool summed = valid;
   // the table entry of the scatter: row d is (q, A) with q + A (i, j, k) =
   // vt[d] + c4 Ct[d] (n - fx)
   if (valid) {
@@ -189,6 +193,12 @@ __global__ __launch_bounds__(CELLSUM_THREADS) __attribute__((amdgpu_waves_per_eu
     for (int d = 0; d < 3; ++d)
 #pragma unroll
       for (int c = 0; c < 3; ++c) e[3 * Sum::ROW + 3 * d + c] = w[d][c];
+    if (!Sum::finite(e)) {
+      summed = false;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) e[d * Sum::ROW] = vt[d];
+      Sum::scatter_one(e, base, fx, add);
+    }
     // C' depends on fx through (n - fx):  dC'_ab/dfx_c = -c4 v'_a delta_bc
     float gx[3];
 #pragma unroll
@@ -215,11 +225,8 @@ __global__ __launch_bounds__(CELLSUM_THREADS) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
     for (int e9 = 0; e9 < 9; ++e9) a.Fb[9 * p + e9] = Fbar[e9];
   }
-  auto add = [&](const int* b, int c, float v) {
-    atomicAdd(a.gbar + 4 * (((int64_t)b[0] * r1 + b[1]) * r1 + b[2]) + c, v);
-  };
-  Sum::prepare(sh, base, valid);
-  Sum::sum_groups(sh, base, valid, add);
+  Sum::prepare(sh, base, summed);
+  Sum::sum_groups(sh, base, summed, add);
   Sum::flush(sh, add);
 }
 

@@ -46,6 +46,42 @@ template <typename T, int DIM, int NCH, int ARENA = 576> struct CellSum {
     int box[2 * DIM];  // low corner, extent (0: the box does not fit the arena)
   };
 
+  // Whether all linear terms of a table entry are finite.  sum_groups must not see
+  // others: q + A n is A (n - fx) multiplied out, where an infinite A gives NaN
+  // for an infinity.
+  static __device__ __forceinline__ bool finite(const T* e) {
+    T zero = T(0);
+#pragma unroll
+    for (int r = 0; r < NCH * ROW; ++r) zero += e[r] * T(0);
+    return zero == T(0);
+  }
+
+  // One particle's terms to its nodes, for an entry whose q is the value at fx
+  // (without A fx taken off).  Rolled: it is rarely run.
+  template <typename Add>
+  static __device__ __forceinline__ void scatter_one(const T* e, const int (&base)[DIM], const T (&fx)[DIM], Add add) {
+#pragma unroll 1
+    for (int node = 0; node < NODES; ++node) {
+      int o[DIM], b[DIM], rest = node;
+      T w = T(1);
+#pragma unroll
+      for (int d = DIM - 1; d >= 0; --d) {
+        o[d] = rest % 3;
+        rest /= 3;
+        b[d] = base[d] + o[d];
+      }
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) w *= e[NCH * ROW + 3 * d + o[d]];
+#pragma unroll 1
+      for (int c = 0; c < NCH; ++c) {
+        T ad = T(0);
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) ad += e[c * ROW + 1 + d] * (T(o[d]) - fx[d]);
+        add(b, c, w * (e[c * ROW] + ad));
+      }
+    }
+  }
+
   // Bounding box of the workgroup's stencils (valid particles) and the
   // cleared arena.  Every thread of the workgroup calls it; ends in a
   // barrier, so the table may be written before it and read after it.

@@ -300,7 +300,14 @@ __global__ __launch_bounds__(CELLSUM_THREADS) void phase_p2g_sorted_kernel(Phase
   T fx[DIM];
   const bool located = locate<T, DIM>(a.x + p * DIM, a.inv_dx, a.res, base, fx);
   if (inrange && !located && a.oob) atomicAdd(a.oob, 1ull);
-  const bool valid = inrange && located;
+  bool valid = inrange && located;
+  const int64_t r1 = a.res + 1;
+  auto add = [&](const int* b, int c, T v) {
+    int64_t node = (int64_t)b[0] * r1 + b[1];
+    if constexpr (DIM == 3) node = node * r1 + b[2];
+    if (c < DIM) atomicAdd(a.grid_v + DIM * node + c, v);
+    else atomicAdd(a.grid_m + node, v);
+  };
   if (valid) {
     int kind;
     T h, tc, ts;
@@ -336,14 +343,13 @@ __global__ __launch_bounds__(CELLSUM_THREADS) void phase_p2g_sorted_kernel(Phase
 #pragma unroll
       for (int c = 0; c < 3; ++c) e[(DIM + 1) * Sum::ROW + 3 * d + c] = w[c];
     }
+    if (!Sum::finite(e)) {
+      valid = false;
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) e[d * Sum::ROW] = m * a.v[DIM * p + d];
+      Sum::scatter_one(e, base, fx, add);
+    }
   }
-  const int64_t r1 = a.res + 1;
-  auto add = [&](const int* b, int c, T v) {
-    int64_t node = (int64_t)b[0] * r1 + b[1];
-    if constexpr (DIM == 3) node = node * r1 + b[2];
-    if (c < DIM) atomicAdd(a.grid_v + DIM * node + c, v);
-    else atomicAdd(a.grid_m + node, v);
-  };
   Sum::prepare(sh, base, valid);
   Sum::sum_groups(sh, base, valid, add);
   Sum::flush(sh, add);
