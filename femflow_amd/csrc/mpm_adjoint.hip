@@ -175,19 +175,19 @@ __global__ __launch_bounds__(CELLSUM_THREADS) __attribute__((amdgpu_waves_per_eu
     atomicAdd(a.gbar + 4 * (((int64_t)b[0] * r1 + b[1]) * r1 + b[2]) + c, v);
   };
   bool summed = valid;
-  // the table entry of the scatter: row d is (q, A) with q + A (i, j, k) =
-  // vt[d] + c4 Ct[d] (n - fx)
+  // the table entry of the scatter: row d is (q, A) with q + A (n - 1) = vt[d] +
+  // c4 Ct[d] (n - fx)
   if (valid) {
     float* e = sh.table + threadIdx.x * Sum::ENTRY;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      float off = 0.f;
+      float mid = 0.f;
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         e[d * Sum::ROW + 1 + c] = c4 * Ct[3 * d + c];
-        off += c4 * Ct[3 * d + c] * fx[c];
+        mid += c4 * Ct[3 * d + c] * (1.f - fx[c]);
       }
-      e[d * Sum::ROW] = vt[d] - off;
+      e[d * Sum::ROW] = vt[d] + mid;
     }
 #pragma unroll
     for (int d = 0; d < 3; ++d)

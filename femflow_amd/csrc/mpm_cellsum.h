@@ -13,7 +13,10 @@
 // are served behind it), which is what a per-particle scatter is bound by.
 //
 // Value of channel c at stencil node (i, j[, k]) of a particle:
-//   w_i w_j [w_k] (q[c] + A[c][0] i + A[c][1] j [+ A[c][2] k]).
+//   w_i w_j [w_k] (q[c] + A[c][0] (i - 1) + A[c][1] (j - 1) [+ A[c][2] (k - 1)]),
+// q being the value at the middle node: expanded there, the terms are no larger
+// than those of A (n - fx) and round no more (about node 0 the offset A fx and
+// what it takes back are up to three times as large).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -47,8 +50,8 @@ template <typename T, int DIM, int NCH, int ARENA = 576> struct CellSum {
   };
 
   // Whether all linear terms of a table entry are finite.  sum_groups must not see
-  // others: q + A n is A (n - fx) multiplied out, where an infinite A gives NaN
-  // for an infinity.
+  // others: q + A (n - 1) is A (n - fx) multiplied out, where an infinite A gives
+  // NaN for an infinity.
   static __device__ __forceinline__ bool finite(const T* e) {
     T zero = T(0);
 #pragma unroll
@@ -152,7 +155,7 @@ template <typename T, int DIM, int NCH, int ARENA = 576> struct CellSum {
     const int i = DIM == 3 ? node / 9 : node / 3, j = DIM == 3 ? (node / 3) % 3 : node % 3, k = node % 3;
     const int c0 = DIM == 3 ? 2 * sub : o / NODES;
     const bool on0 = lane < 2 * OUT && c0 < NCH, on1 = DIM == 3 && lane < OUT * 2 && c0 + 1 < NCH;
-    const T fi = (T)i, fj = (T)j, fk = (T)k;
+    const T fi = (T)(i - 1), fj = (T)(j - 1), fk = (T)(k - 1);
     const int r0 = (on0 ? c0 : 0) * ROW, r1 = (on1 ? c0 + 1 : 0) * ROW;
     const int wi = NCH * ROW + i, wj = NCH * ROW + 3 + j, wk = NCH * ROW + (DIM == 3 ? 6 + k : 0);
     const bool arena = sh.box[DIM] > 0;

@@ -324,14 +324,14 @@ __global__ __launch_bounds__(CELLSUM_THREADS) void phase_p2g_sorted_kernel(Phase
     T* e = sh.table + threadIdx.x * Sum::ENTRY;
 #pragma unroll
     for (int d = 0; d < DIM; ++d) {
-      T off = T(0);  // A (ijk - fx) dx = A dx ijk - A dx fx
+      T mid = T(0);  // A (n - fx) dx at the middle node
 #pragma unroll
       for (int c = 0; c < DIM; ++c) {
         const T ad = A[DIM * d + c] * a.dx;
         e[d * Sum::ROW + 1 + c] = ad;
-        off += ad * fx[c];
+        mid += ad * (T(1) - fx[c]);
       }
-      e[d * Sum::ROW] = m * a.v[DIM * p + d] - off;
+      e[d * Sum::ROW] = m * a.v[DIM * p + d] + mid;
     }
     e[DIM * Sum::ROW] = m;
 #pragma unroll
