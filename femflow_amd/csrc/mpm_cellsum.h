@@ -1,6 +1,6 @@
 // Particle-to-node sums without one atomic per particle and node.
 //
-// A workgroup takes CELLSUM_THREADS consecutive particles of a cell-ordered
+// A workgroup takes THREADS consecutive particles of a cell-ordered
 // list.  Each thread writes its particle's B-spline weights and linear terms
 // to an LDS table; each wave then walks the groups of equal stencil bases
 // among its 64 particles with one lane per (node, channel) output (3D: 54
@@ -34,7 +34,7 @@ constexpr int CELLSUM_THREADS = 256;
 // FP32 particles, sort included, 80 -> 65 us at 2 per cell and 83 -> 64 at 16, with
 // an arena of 1,024 FP32 nodes before).  576 leaves room for two workgroups of the
 // phase P2G (FP64, 3D) per compute unit, whose particles come in blocks of cells.
-template <typename T, int DIM, int NCH, int ARENA = 576> struct CellSum {
+template <typename T, int DIM, int NCH, int ARENA = 576, int THREADS = CELLSUM_THREADS> struct CellSum {
   static constexpr int NODES = DIM == 3 ? 27 : 9;
   static constexpr int ROW = DIM == 3 ? 4 : 3;  // q, A[0..DIM-1] of a channel
   // per-particle table entry: NCH rows, then DIM x 3 weights, padded to 16
@@ -43,9 +43,9 @@ template <typename T, int DIM, int NCH, int ARENA = 576> struct CellSum {
   static constexpr int ENTRY = (NCH * ROW + 3 * DIM + PAD - 1) / PAD * PAD;
   typedef T Row3 __attribute__((ext_vector_type(4), aligned(16)));
   struct alignas(16) Shared {
-    T table[CELLSUM_THREADS * ENTRY];
+    T table[THREADS * ENTRY];
     double arena[ARENA * NCH];
-    int box_w[CELLSUM_THREADS / 64][2 * DIM];
+    int box_w[THREADS / 64][2 * DIM];
     int box[2 * DIM];  // low corner, extent (0: the box does not fit the arena)
   };
 
@@ -112,7 +112,7 @@ template <typename T, int DIM, int NCH, int ARENA = 576> struct CellSum {
 #pragma unroll
       for (int d = 0; d < DIM; ++d) {
         int a = INT_MAX, b = INT_MIN;
-        for (int w = 0; w < CELLSUM_THREADS / 64; ++w) {
+        for (int w = 0; w < THREADS / 64; ++w) {
           a = min(a, sh.box_w[w][d]);
           b = max(b, sh.box_w[w][DIM + d]);
         }
@@ -129,7 +129,7 @@ template <typename T, int DIM, int NCH, int ARENA = 576> struct CellSum {
     }
     __syncthreads();
     const int n = volume(sh) * NCH;
-    for (int e = t; e < n; e += CELLSUM_THREADS) sh.arena[e] = 0.0;
+    for (int e = t; e < n; e += THREADS) sh.arena[e] = 0.0;
     __syncthreads();
   }
 
@@ -215,7 +215,7 @@ template <typename T, int DIM, int NCH, int ARENA = 576> struct CellSum {
   template <typename Add> static __device__ __forceinline__ void flush(Shared& sh, Add add) {
     __syncthreads();
     const int n = volume(sh) * NCH;
-    for (int e = threadIdx.x; e < n; e += CELLSUM_THREADS) {
+    for (int e = threadIdx.x; e < n; e += THREADS) {
       const T v = (T)sh.arena[e];
       if (v != T(0)) {
         const int c = e % NCH;

@@ -84,13 +84,75 @@ __device__ __forceinline__ bool locate(const T* xp, T inv_dx, int res, int base[
   return ok;
 }
 
-// P2G of few particles (or without scratch memory) in any order: a workgroup
-// takes THREADS of them and sums into an LDS arena over their stencils'
-// bounding box, which goes to memory once.  What bounds it: up to a few
-// thousand particles the chain of loads, stress and LDS adds of one workgroup,
-// then the arenas' flushes (each workgroup's box is that of the whole body
-// when the order is arbitrary).  Layers of the box that the arena cannot hold
-// go to memory particle by particle.
+// Adds channel c (momentum, then mass) at node b to the grids.
+template <typename T, int DIM>
+__device__ __forceinline__ void add_to_grid(const PhaseArgs<T>& a, const int* b, int c, T v) {
+  const int64_t r1 = a.res + 1;
+  int64_t node = (int64_t)b[0] * r1 + b[1];
+  if constexpr (DIM == 3) node = node * r1 + b[2];
+  if (c < DIM) atomicAdd(a.grid_v + DIM * node + c, v);
+  else atomicAdd(a.grid_m + node, v);
+}
+
+// The cell-sum table entry e of particle p; false, with its terms already added
+// to the grids, if they are not all finite.
+template <typename Sum, typename T, int DIM>
+__device__ __forceinline__ bool write_entry(const PhaseArgs<T>& a, int64_t p, const int (&base)[DIM],
+                                            const T (&fx)[DIM], T* e) {
+  int kind;
+  T h, tc, ts;
+  material_of(a, p, kind, h, tc, ts);
+  T m, mu0, lam0, mu, lam;
+  constants_of(a, p, m, mu0, lam0);
+  lame<T>(kind, h, mu0, lam0, a.Jp[p], mu, lam);
+  const bool textbook = a.quirks == MPM_QUIRKS_TEXTBOOK;
+  T A[DIM * DIM];
+  if constexpr (DIM == 3)
+    affine3<T>(a.F + 9 * p, a.C + 9 * p, m, mu, lam, kind, a.inv_dx, a.dt, a.vol, textbook, A);
+  else
+    affine2<T>(a.F + 4 * p, a.C + 4 * p, m, mu, lam, kind, a.inv_dx, a.dt, a.vol, textbook, A);
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) {
+    T mid = T(0);  // A (n - fx) dx at the middle node
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) {
+      const T ad = A[DIM * d + c] * a.dx;
+      e[d * Sum::ROW + 1 + c] = ad;
+      mid += ad * (T(1) - fx[c]);
+    }
+    e[d * Sum::ROW] = m * a.v[DIM * p + d] + mid;
+  }
+  e[DIM * Sum::ROW] = m;
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) e[DIM * Sum::ROW + 1 + c] = T(0);
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) {
+    T w[3];
+    bspline(fx[d], w);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) e[(DIM + 1) * Sum::ROW + 3 * d + c] = w[c];
+  }
+  if (Sum::finite(e)) return true;
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) e[d * Sum::ROW] = m * a.v[DIM * p + d];
+  Sum::scatter_one(e, base, fx, [&](const int* b, int c, T v) { add_to_grid<T, DIM>(a, b, c, v); });
+  return false;
+}
+
+// P2G of few particles (or without scratch memory) in the order in which they
+// come.  A workgroup takes THREADS of them, finds the bounding box of their
+// stencils, and
+// - where neighbouring lanes share cells (cell order, BOX_RUN particles per run and
+//   more) or the box has few adds per node, takes the sums of mpm_cellsum.h: in the
+//   one case a cell's particles would add to the same LDS words one after the other,
+//   in the other an arena would be cleared and read for nothing, and one particle's
+//   nodes side by side make better atomics than one lane per particle;
+// - else adds particle by particle into an LDS arena over the box, which goes to
+//   memory once; layers of the box that the arena cannot hold go to memory particle
+//   by particle.
+// What bounds it: up to a few thousand particles the chain of loads, stress and
+// LDS adds of one workgroup, then the arenas' flushes (each workgroup's box is
+// that of the whole body when the order is arbitrary).
 // Small workgroups spread few particles over more compute units: 2,048 3D
 // particles at 256 / 512 / 1,024 threads 17 / 26 / 46 us at 16 per cell and 23
 // / 30 / 47 at 2; in 2D, with a third of the adds, 512 is the best from 8,192
@@ -98,16 +160,34 @@ __device__ __forceinline__ bool locate(const T* xp, T inv_dx, int res, int base[
 // The arena is FP64 for FP32 particles too: LDS adds of floats run at a third
 // of a lane per cycle here, those of doubles at about five (8,192 2D FP32
 // particles 41 us with an FP32 arena, 9 with this one).
-// Per-particle device atomics, which this replaces: 8,192 2D FP64 particles at
-// 16 per cell 46 us (8.7 here), 2,048 3D 78 us (17).
+// Per-particle device atomics with sums over runs of lanes, which this replaces /
+// always the arena / this, in us: arbitrary order, 8,192 2D FP64 at 16 per cell 30 /
+// 7 / 7, 2,048 3D FP64 at 16 55 / 18 / 18, 2,048 3D at 0.05 50 / 57 / 24, 8,192 2D at
+// 0.25 15 / 29 / 21, 131,072 3D FP32 at 2 897 / 901 / 304; row-major cell order, 3D
+// FP32, 885,000 at 2 / 16 per cell 573, 242 / 331, 484 / 319, 201, 131,072 at 16 57 /
+// 65 / 34; 500,000 2D FP32 at 2 / 16 48, 24 / 38, 66 / 39, 36 (one workgroup per
+// compute unit: the loads of dense cells in 2D are what the arena's LDS costs).
 template <int DIM> constexpr int BOX_THREADS_OF = DIM == 3 ? 256 : 512;
+// Particles per run of lanes from which the sums are as fast as the arena: in us
+// (arena / sums), 3D FP32 131,072 at 2 / 4 / 8 per cell 70, 57, 54 / 61, 42, 49 and
+// 4,000 FP64 at 2 / 8 22, 25 / 23, 19; 2D FP32 80,000 at 2 / 4 / 8 10, 11, 14 / 16, 16, 11.
+template <int DIM> constexpr int BOX_RUN_OF = DIM == 3 ? 3 : 6;
 constexpr int BOX_WORDS = (144 << 10) / (int)sizeof(double);
 
 template <typename T, int DIM>
 __global__ __launch_bounds__(BOX_THREADS_OF<DIM>) void phase_p2g_box_kernel(PhaseArgs<T> a) {
   constexpr int NCH = DIM + 1, THREADS = BOX_THREADS_OF<DIM>, WAVES = THREADS / 64;
-  __shared__ double arena[BOX_WORDS];
-  __shared__ int box_w[WAVES][2 * DIM];
+  // the arena, or the table and arena of the cell sums
+  using Entry = CellSum<T, DIM, NCH>;
+  constexpr int TABLE = (int)sizeof(T) * THREADS * Entry::ENTRY;
+  using Sum = CellSum<T, DIM, NCH, ((int)sizeof(double) * BOX_WORDS - TABLE) / ((int)sizeof(double) * NCH), THREADS>;
+  union BoxShared {
+    double arena[BOX_WORDS];
+    typename Sum::Shared sum;
+  };
+  __shared__ __align__(16) BoxShared sh;
+  double* const arena = sh.arena;
+  __shared__ int box_w[WAVES][2 * DIM], count_w[WAVES], runs_w[WAVES];
   const int t = threadIdx.x;
   const int64_t p0 = (int64_t)blockIdx.x * THREADS + t;
   const bool inrange = p0 < a.n;
@@ -117,6 +197,18 @@ __global__ __launch_bounds__(BOX_THREADS_OF<DIM>) void phase_p2g_box_kernel(Phas
   const bool located = locate<T, DIM>(a.x + p * DIM, a.inv_dx, a.res, base, fx);
   if (inrange && !located && a.oob) atomicAdd(a.oob, 1ull);
   const bool valid = inrange && located;
+  {
+    // runs of neighbouring lanes in one cell
+    bool first = (t & 63) == 0;
+    const unsigned long long in = __ballot(valid);
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) first = __shfl_up(base[d], 1) != base[d] || first;
+    const unsigned long long heads = __ballot(valid && (first || !((in >> ((t & 63) - 1)) & 1ull)));
+    if ((t & 63) == 0) {
+      count_w[t >> 6] = __popcll(in);
+      runs_w[t >> 6] = __popcll(heads);
+    }
+  }
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
     int lo = valid ? base[d] : INT_MAX, hi = valid ? base[d] : INT_MIN;
@@ -144,6 +236,24 @@ __global__ __launch_bounds__(BOX_THREADS_OF<DIM>) void phase_p2g_box_kernel(Phas
     low[d] = lo;
     ext[d] = lo <= hi ? hi - lo + 3 : 0;
     vol *= ext[d];
+  }
+  int count = 0, runs = 0;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    count += count_w[w];
+    runs += runs_w[w];
+  }
+  // (sparse: 0.4 adds per node; 16,384 2D FP64 at 0.3 / 0.5 25 / 27 us as sums, 35 /
+  // 27 with the arena)
+  const bool merge = runs * BOX_RUN_OF<DIM> <= count, sparse = (int64_t)count * Entry::NODES * 5 < 2 * vol;
+  if (2 * count > THREADS && (merge || sparse)) {  // (the same in every wave)
+    const bool summed =
+        valid && write_entry<Sum, T, DIM>(a, p, base, fx, sh.sum.table + t * Sum::ENTRY);
+    auto add = [&](const int* b, int c, T v) { add_to_grid<T, DIM>(a, b, c, v); };
+    Sum::prepare(sh.sum, base, summed);
+    Sum::sum_groups(sh.sum, base, summed, add);
+    Sum::flush(sh.sum, add);
+    return;
   }
   // the layers of the first axis that the arena holds
   const int64_t layer = ext[0] ? vol / ext[0] * NCH : 1;
@@ -301,55 +411,8 @@ __global__ __launch_bounds__(CELLSUM_THREADS) void phase_p2g_sorted_kernel(Phase
   const bool located = locate<T, DIM>(a.x + p * DIM, a.inv_dx, a.res, base, fx);
   if (inrange && !located && a.oob) atomicAdd(a.oob, 1ull);
   bool valid = inrange && located;
-  const int64_t r1 = a.res + 1;
-  auto add = [&](const int* b, int c, T v) {
-    int64_t node = (int64_t)b[0] * r1 + b[1];
-    if constexpr (DIM == 3) node = node * r1 + b[2];
-    if (c < DIM) atomicAdd(a.grid_v + DIM * node + c, v);
-    else atomicAdd(a.grid_m + node, v);
-  };
-  if (valid) {
-    int kind;
-    T h, tc, ts;
-    material_of(a, p, kind, h, tc, ts);
-    T m, mu0, lam0, mu, lam;
-    constants_of(a, p, m, mu0, lam0);
-    lame<T>(kind, h, mu0, lam0, a.Jp[p], mu, lam);
-    const bool textbook = a.quirks == MPM_QUIRKS_TEXTBOOK;
-    T A[DIM * DIM];
-    if constexpr (DIM == 3)
-      affine3<T>(a.F + 9 * p, a.C + 9 * p, m, mu, lam, kind, a.inv_dx, a.dt, a.vol, textbook, A);
-    else
-      affine2<T>(a.F + 4 * p, a.C + 4 * p, m, mu, lam, kind, a.inv_dx, a.dt, a.vol, textbook, A);
-    T* e = sh.table + threadIdx.x * Sum::ENTRY;
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-      T mid = T(0);  // A (n - fx) dx at the middle node
-#pragma unroll
-      for (int c = 0; c < DIM; ++c) {
-        const T ad = A[DIM * d + c] * a.dx;
-        e[d * Sum::ROW + 1 + c] = ad;
-        mid += ad * (T(1) - fx[c]);
-      }
-      e[d * Sum::ROW] = m * a.v[DIM * p + d] + mid;
-    }
-    e[DIM * Sum::ROW] = m;
-#pragma unroll
-    for (int c = 0; c < DIM; ++c) e[DIM * Sum::ROW + 1 + c] = T(0);
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-      T w[3];
-      bspline(fx[d], w);
-#pragma unroll
-      for (int c = 0; c < 3; ++c) e[(DIM + 1) * Sum::ROW + 3 * d + c] = w[c];
-    }
-    if (!Sum::finite(e)) {
-      valid = false;
-#pragma unroll
-      for (int d = 0; d < DIM; ++d) e[d * Sum::ROW] = m * a.v[DIM * p + d];
-      Sum::scatter_one(e, base, fx, add);
-    }
-  }
+  if (valid) valid = write_entry<Sum, T, DIM>(a, p, base, fx, sh.table + threadIdx.x * Sum::ENTRY);
+  auto add = [&](const int* b, int c, T v) { add_to_grid<T, DIM>(a, b, c, v); };
   Sum::prepare(sh, base, valid);
   Sum::sum_groups(sh, base, valid, add);
   Sum::flush(sh, add);
@@ -636,6 +699,9 @@ static inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t -
 //           131,072: 772 / 72, 779 / 70
 //   2D FP64  16,384: 27 / 41, 10 / 34    32,768: 64 / 41, 15 / 35
 //           131,072: 198 / 50, 144 / 49
+// Below one per cell the sort finds nothing to merge (0.25 per cell, box / sorted,
+// in calls back to back: 3D 4,096 24 / 53, 131,072 279 / 294; 2D 24,576 30 / 54, 65,536
+// 59 / 85), but the host cannot tell such a cloud from a body in a corner of its grid.
 static int64_t p2g_sort_from(int dim) { return dim == 3 ? 4096 : 24576; }
 
 // Cells of the key space, or 0 when the sorted form does not apply.
