@@ -450,8 +450,10 @@ MPM_DEV void affine2(const T* F, const T* C, T mass, T mu, T lam, int kind, T in
   const T x = F[0] + F[3], y = F[2] - F[1];
   const T denom = tsqrt(x * x + y * y) + (textbook ? T(0) : T(1e-10));
   const T sc = T(1) / denom;
-  const T c = x * sc, s = y * sc;
-  const T r[4] = {c, -s, s, c};
+  // F - R, R = sc ((x, -y), (y, x)), by FMA: the difference is small, so that
+  // a rounded x sc is most of the stress's error (left to the compiler, one kernel
+  // did and another did not)
+  const T f_r[4] = {fma(-x, sc, F[0]), fma(y, sc, F[1]), fma(-y, sc, F[2]), fma(-x, sc, F[3])};
   const T scale = -(dt * vol) * (T(4) * inv_dx * inv_dx);
   const T vt = lam * (J - T(1)) * J;
   const bool diag_only = textbook || kind == MPM_WATER;
@@ -460,7 +462,7 @@ MPM_DEV void affine2(const T* F, const T* C, T mass, T mu, T lam, int kind, T in
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      T pf = m2 * (F[2 * i] - r[2 * i]) * F[2 * j] + m2 * (F[2 * i + 1] - r[2 * i + 1]) * F[2 * j + 1];
+      T pf = m2 * f_r[2 * i] * F[2 * j] + m2 * f_r[2 * i + 1] * F[2 * j + 1];
       pf += (diag_only && i != j) ? T(0) : vt;
       A[2 * i + j] = scale * pf + mass * C[2 * i + j];
     }
