@@ -328,9 +328,9 @@ def config1_bench(dev, cpu=True):
 
 
 def binning_bench(x, res, reps=7):
-    """The standalone binning entry point (mpm_bin: cell keys and their stable
-    LSD radix sort) on the headline positions; median of `reps` calls, each
-    including the entry point's own workspace allocation."""
+    """The standalone binning entry point (bin_particles: cell keys and their
+    stable LSD radix sort) on the headline positions; median of `reps` calls,
+    each with its outputs and scratch memory from torch's caching allocator."""
     import torch
 
     from femflow_amd.engine import bin_particles
@@ -345,8 +345,8 @@ def binning_bench(x, res, reps=7):
         times.append(time.perf_counter() - t0)
     ms = sorted(times)[len(times) // 2] * 1e3
     n = int(x.shape[0])
-    return {"workload": f"mpm_bin on the {n} headline positions, {res}^3 grid, blocked keys, stable sort; "
-                        "wall time per call including its workspace allocation",
+    return {"workload": f"bin_particles on the {n} headline positions, {res}^3 grid, blocked keys, stable sort; "
+                        "wall time per call, outputs and scratch memory from torch's allocator",
             "ms": ms, "value": n / (ms / 1e3), "unit": "particles/s"}
 
 
