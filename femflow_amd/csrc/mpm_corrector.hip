@@ -497,7 +497,7 @@ int Engine::corrector_sample(uint16_t* X, uint32_t* nodes, float* vel, int64_t m
   {
     EngineArgs a0 = a;
     a0.perm = pending_perm;  // this P2G moves the particles into binned order
-    a0.rec = in_records ? rec_mem[0] : nullptr;
+    a0.rec = in_records ? d_rec : nullptr;
     in_records = false;
     pending_perm = nullptr;
     launch_transfer(0, s, a0);

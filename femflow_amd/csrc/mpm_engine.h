@@ -110,12 +110,19 @@ struct Engine {
   std::vector<void*> allocs;
   EngineState st[2] = {};
   int cur = 0;
-  // The uploaded particles are still records (in st[0]'s memory except its x
-  // and attr, which hold them as ever, for the rebin's keys); the first rebin
-  // moves them into st[1].  tiled() does so without one, for calls that read the
-  // state before.
+  // The uploaded particles are still records (in d_rec; st[0] has only their x and
+  // attr, for the rebin's keys); the first rebin moves them into st[1].  tiled()
+  // unpacks them into st[0] instead, for calls that read the state before, and
+  // for callers that capture.
   bool in_records = false;
-  float4* rec_mem[2] = {};  // the same memory as st[0], st[1] without x and attr
+  // 128 bytes per particle, of an upload or on a large download's way out.  Memory
+  // of its own: a graph of the caller's may read either state copy at any time.
+  float4* d_rec = nullptr;
+  // something of this engine went into a graph of the caller's.  Its replays start
+  // from the state that was there, so from then on (and within the capture) uploads
+  // end in st[0] as tiles, and downloads leave d_rec, which holds the last upload,
+  // alone.
+  bool captured = false;
   SceneDev* d_scenes = nullptr;
   MatParams* d_mats = nullptr;
   int* d_block_scene = nullptr;
@@ -165,6 +172,7 @@ struct Engine {
   int upload(const mpm_particles* p, const int32_t* scene_ids);
   int download(mpm_particles* p);
   void tiled();
+  bool capturing();  // whether the caller's stream is (noted in `captured`)
   // rebin; also starts the segment of len substeps (counters, sums index;
   // keep_speeds: not the speed counts, for a segment that is no part of a run)
   void enqueue_bin(hipStream_t s, int len, int with_sums, bool keep_speeds = false);

@@ -1806,24 +1806,24 @@ int Engine::init(int64_t n_max_, int nscenes, const mpm_scene* sc, int nmat_, co
   }
   HIPCHK(hipMemcpy(d_mats, hm.data(), sizeof(MatParams) * nmat, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(d_block_scene, bscene.data(), sizeof(int) * blocks, hipMemcpyHostToDevice));
-  // particle state (two copies for reordering)
+  // particle state (two copies for reordering) and records, in one allocation
+  constexpr int STATE_WORDS = 30;
+  float* words = nullptr;
+  if ((rc = alloc((void**)&words, sizeof(float) * (2 * STATE_WORDS + REC_WORDS) * n))) return rc;
+  d_rec = reinterpret_cast<float4*>(words + 2 * STATE_WORDS * n);  // (n is a multiple of 64)
   for (int b = 0; b < 2; ++b) {
     EngineState& s = st[b];
-    // 104 bytes per particle beside x and attr, which a rebin's keys read;
-    // the same memory holds 128-byte records of an upload or a download
-    float* rest = nullptr;
-    if ((rc = alloc((void**)&s.x, 12 * n)) || (rc = alloc((void**)&s.attr, 4 * n)) ||
-        (rc = alloc((void**)&rest, 4 * REC_WORDS * n)))
-      return rc;
-    rec_mem[b] = reinterpret_cast<float4*>(rest);
-    s.v = rest;
-    s.F = rest + 3 * n;
-    s.C = rest + 12 * n;
-    s.Jp = rest + 21 * n;
-    s.mass = rest + 22 * n;
-    s.mu0 = rest + 23 * n;
-    s.lam0 = rest + 24 * n;
-    s.order = reinterpret_cast<uint32_t*>(rest + 25 * n);
+    float* w = words + b * STATE_WORDS * n;
+    s.x = w;
+    s.v = w + 3 * n;
+    s.F = w + 6 * n;
+    s.C = w + 15 * n;
+    s.Jp = w + 24 * n;
+    s.mass = w + 25 * n;
+    s.mu0 = w + 26 * n;
+    s.lam0 = w + 27 * n;
+    s.attr = reinterpret_cast<uint32_t*>(w + 28 * n);
+    s.order = reinterpret_cast<uint32_t*>(w + 29 * n);
   }
   // grids
   if ((rc = alloc((void**)&d_acc, sizeof(float4) * 64 * blocks))) return rc;
@@ -1956,16 +1956,27 @@ int Engine::upload(const mpm_particles* p, const int32_t* scene_ids) {
                        p->mat_scalar,      (int)scenes_host.size()};
     speeds_at = SPEEDS_UPLOAD;
     cadence = 0;
-    hipLaunchKernelGGL(upload_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[0], rec_mem[0], n, u);
+    hipLaunchKernelGGL(upload_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[0], d_rec, n, u);
   }
+  if (capturing() || captured) tiled();
   HIPCHK(hipGetLastError());
   return MPM_OK;
 }
 
+bool Engine::capturing() {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(user_stream, &status) != hipSuccess) {
+    (void)hipGetLastError();  // (what uses the stream next reports it)
+    return true;
+  }
+  if (status != hipStreamCaptureStatusNone) captured = true;
+  return status != hipStreamCaptureStatusNone;
+}
+
 void Engine::tiled() {
   if (!in_records) return;
-  hipLaunchKernelGGL(unpack_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[1], rec_mem[0], n);
-  cur = 1;
+  capturing();  // (if so, the replays read d_rec)
+  hipLaunchKernelGGL(unpack_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[0], d_rec, n);
   in_records = false;
 }
 
@@ -1975,13 +1986,13 @@ int Engine::download(mpm_particles* p) {
     return MPM_ERR_ARG;
   }
   tiled();
-  if (n > 0 && n < TWO_PASS_DOWNLOAD) {
+  const bool two_pass = n >= TWO_PASS_DOWNLOAD && !capturing() && !captured;
+  if (n > 0 && !two_pass) {
     hipLaunchKernelGGL(download_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[cur], n,
                        (float*)p->x, (float*)p->v, (float*)p->F, (float*)p->C, (float*)p->Jp);
-  } else if (n > 0) {  // through the other state copy, which holds nothing between runs
-    float4* rec = rec_mem[cur ^ 1];
-    hipLaunchKernelGGL(pack_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[cur], n, rec);
-    hipLaunchKernelGGL(split_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, rec, n, (float*)p->x,
+  } else if (n > 0) {
+    hipLaunchKernelGGL(pack_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, st[cur], n, d_rec);
+    hipLaunchKernelGGL(split_kernel, dim3(nblk(n, 256)), dim3(256), 0, own_stream, d_rec, n, (float*)p->x,
                        (float*)p->v, (float*)p->F, (float*)p->C, (float*)p->Jp);
   }
   HIPCHK(hipGetLastError());
@@ -2167,7 +2178,7 @@ void Engine::enqueue_segment(int k0, int len, bool bin, hipStream_t s, double* s
   if (k0 == 0) {
     EngineArgs a0 = args(sums, max_steps, 0);
     a0.perm = bin ? pending_perm : nullptr;
-    a0.rec = in_records ? rec_mem[0] : nullptr;  // a segment after an upload rebins
+    a0.rec = in_records ? d_rec : nullptr;  // a segment after an upload rebins
     pending_perm = nullptr;
     launch_transfer(cont ? 3 : 0, s, a0, sep);
     if (corr_on) launch_cellf(s, args(sums, max_steps, 0));
@@ -2243,11 +2254,10 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
   // run then keeps the cadence that it had.
   bool probe =
       speeds_at != SPEEDS_NONE && n > 0 && nsteps > MIN_CADENCE && sort_every > MIN_CADENCE && !sums;
-  if (probe) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    HIPCHK(hipStreamIsCapturing(user_stream, &cap));
-    probe = cap == hipStreamCaptureStatusNone;
-  }
+  // (a caller that captures has the engine's own graphs off, or asks for frames or states)
+  const bool graphed = use_graph && !timing && n > 0 && !frames && !sink;
+  const bool in_capture = (probe || !graphed) && capturing();
+  if (in_capture) probe = false;
   uint32_t* const sent = h_speeds + SPEED_CLASSES;
   if (probe && speeds_pending) {
     speeds_pending = !__atomic_load_n(sent, __ATOMIC_ACQUIRE);
@@ -2264,6 +2274,7 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
   if (speeds_at != SPEEDS_NONE) speeds_at = n > 0 ? SPEEDS_RUN : SPEEDS_NONE;
   HIPCHK(hipEventRecord(ev_in, user_stream));
   HIPCHK(hipStreamWaitEvent(own_stream, ev_in, 0));
+  if (in_capture) tiled();
   if (sums) {
     hipLaunchKernelGGL(fill_f64_kernel, dim3(nblk((int64_t)nsteps * 8, 256)), dim3(256), 0, own_stream,
                        sums, (int64_t)nsteps * 8, 0.0);
@@ -2298,7 +2309,6 @@ int Engine::run(int nsteps, double* sums, float* frames, const StateSink* sink) 
     if (len > nsteps - done) len = nsteps - done;
     const bool cont = n > 0 && done > 0;
     const bool fin = n <= 0 || done + len == nsteps;
-    const bool graphed = use_graph && !timing && n > 0 && !frames && !sink;
     if (graphed) {
       const int parity = cur;
       const GraphKey key{n, len, parity, bin ? 1 : 0, (uintptr_t)sums, sums ? nsteps : 0, cont ? 1 : 0,
