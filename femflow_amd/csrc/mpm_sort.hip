@@ -207,32 +207,37 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
 
 // ------------------------------------------------------- chunk list ----
 // Chunk list of the new binning, numbered over blocks.  A transfer workgroup
-// works through a chunk in rows of CHUNK_ROW particles, one per thread, so a
-// block's particles are cut into R = ceil(count / CHUNK_ROW) rows of nearly
-// equal size first (chunks of 333 would take two rows each for the work of
-// 1.3).  Either every row is a chunk, or the rows of a block are grouped into
-// chunks of up to `chunk` particles: a row by itself finishes sooner and
-// leaves a shorter tail; a pair loads and stages one arena for both and
-// spreads a wave's lanes over twice as many cells, which is what counts where
-// a cell holds dozens of particles (the lanes that share one add to the same
-// words).  One choice for the whole list: chunks of one and of two rows side
-// by side were the slowest (2^20 particles 5,464 us, see below).  Two launches
-// over tiles of SCAN_THREADS blocks, one block per thread (coalesced reads,
-// a few hundred tiles for a 128^3 grid): per-tile counts, then each tile adds
-// the counts of the tiles before it, scans its own blocks and writes their
-// chunks, first chunk and chunk count.
+// works through a chunk in steps of CHUNK_ROW particles, one per thread, and
+// loads, clears and stages an arena for it: a chunk costs about 1.4 steps beside
+// its own.  Three ways to cut a block, one for the whole list:
+// - plain: ceil(count / chunk) equal chunks, the fewest (but 333 particles take
+//   two steps for the work of 1.3);
+// - single: rows of nearly equal size, ceil(count / CHUNK_ROW) of them, each a
+//   chunk: the fewest steps and the shortest tail, at most twice the chunks;
+// - grouped: those rows in chunks of up to `chunk` particles; pairs that would be
+//   less than 3/4 full stay single (260 particles: 130 + 130, not 256 + 4).
+// Two launches over tiles of SCAN_THREADS blocks, one block per thread
+// (coalesced reads, a few hundred tiles for a 128^3 grid): per-tile sums, then
+// each tile adds those of the tiles before it, scans its own blocks and writes
+// their chunks, first chunk and chunk count.
 constexpr uint32_t CHUNK_ROW = 256;
-// Rows are grouped where most of them are in blocks of more than 18 particles
-// per cell.  48 substeps, all rows single / grouped, in us: 100,003 particles
-// at 17 per cell 1,500 / 1,723; 400,000 at 17 2,839 / 2,978; 524,288 at 10
-// 3,425 / 3,908; 262,144 at 21 2,210 / 2,118; 2^20 at 21 5,581 / 5,164;
-// 131,072 at 62 1,744 / 1,638.
+// A block is dense above this (18 particles per cell).
 constexpr uint32_t GROUP_ABOVE = 18 * 64;
-// And single up to this many rows in all, one and a half per compute unit of
-// an MI355X: fewer, larger chunks would leave units without one (16,384
-// particles at 8 per cell 1,035 / 1,230).
-// Engines of many scenes (plain) cut a block into ceil(count / chunk) equal
-// chunks, without regard to rows: their tens of thousands of chunks come from
+// The rule, for engines of one scene without the corrector.  R rows in all, T steps
+// of the plain list, 768 chunks running at once on an MI355X (three per compute
+// unit); us per substep, plain / single / grouped, one elastic body:
+// - R <= 384: single; fewer, larger chunks would leave units without one.  20,000
+//   particles at 8 per cell 21.2 / 17.6 / 21.1.
+// - most rows in dense blocks: grouped up to R = 2,100 (200,000 at 64 per cell 34.9 /
+//   38.4 / 30.5, at 20 30.2 / 30.8 / 29.3), where its fewer steps leave a shorter
+//   tail; beyond, plain (2^20 in three bodies at 20 75.0 / 83.5 / 79.4, 1,600,000 at
+//   32 95.7 / 114.7 / 99.9, at 64 93.5 / 115.7 / 91.6).
+// - else up to one round of chunks, R <= 768, single (100,000 at 12 25.5 / 21.2 / 24.9),
+//   and up to 2,100 where it saves a tenth of the steps, 10 T >= 11 R (300,000 in
+//   three bodies at 18, T = 1.16 R, 39.2 / 34.9 / 37.4; but 200,000 at 14, 1.04 R, 27.0
+//   / 29.9 / 29.7); beyond, plain: the chunks' arenas are what counts (800,000 at 6
+//   and 16 66.0 / 80.4 / 75.9, 60.0 / 65.4 / 60.2; 4,000,000 at 8 291 / 335 / 323).
+// Engines of many scenes are plain: their tens of thousands of chunks come from
 // contended ticket queues, and single rows cost more there (64 scenes, 24
 // substeps with upload and download: 16,112 single, 14,827 rows grouped,
 // 15,160 plain; grouping moves the fixed-point scale of scenes with a fraction
@@ -240,7 +245,7 @@ constexpr uint32_t GROUP_ABOVE = 18 * 64;
 // the corrector are plain too: its features and activations round to BF16, so
 // another fixed-point scale now and then moves a light node's velocity gradient
 // by 1e-3 (262,144 particles in 5,400 cells: no difference in time).
-constexpr uint32_t FEW_ROWS = 384;
+constexpr uint32_t FEW_ROWS = 384, ONE_ROUND = 768, FEW_ROUNDS = 2100;
 // Small chunks go to the launch of their own (split) from this many on, one round
 // of four-wave workgroups (three per compute unit): fewer find room beside the
 // others, and a second pass over the few takes longer than they do there.  Us per
@@ -250,77 +255,97 @@ constexpr uint32_t FEW_ROWS = 384;
 // 69 / 107.  (Before there was a second launch: 43, 69, 55, 124.)
 constexpr uint32_t APART_FROM = 768;
 
-// Of a block (or their sums over a tile): rows, chunks with rows grouped, rows
-// in dense blocks.  A block's pairs that would be less than 3/4 full stay
-// single (260 particles: 130 + 130, not 256 + 4).
-struct BlockRows {
-  uint32_t rows, chunks, dense, small;
-};
-__device__ __forceinline__ BlockRows block_rows(const uint32_t* __restrict__ bocc, const uint32_t* __restrict__ bstart,
-                                                const uint32_t* __restrict__ bend, int64_t b, uint32_t per_chunk,
-                                                int plain) {
-  if (!bocc[b]) return {0u, 0u, 0u, 0u};
+// Of a block, or their sums: rows, chunks with rows grouped, plain chunks, plain
+// chunks of at most SMALL_CHUNK, steps of the plain chunks, rows in dense blocks.
+enum { CUT_ROWS, CUT_GROUPED, CUT_PLAIN, CUT_SMALL, CUT_STEPS, CUT_DENSE, CUTS };
+typedef uint32_t BlockCuts[CUTS];
+__device__ __forceinline__ void block_cuts(const uint32_t* __restrict__ bocc, const uint32_t* __restrict__ bstart,
+                                           const uint32_t* __restrict__ bend, int64_t b, int64_t nblocks,
+                                           uint32_t per_chunk, BlockCuts& r) {
+#pragma unroll
+  for (int i = 0; i < CUTS; ++i) r[i] = 0u;
+  if (b >= nblocks || !bocc[b]) return;
   const uint32_t cnt = bend[b] - bstart[b], rows = (cnt + CHUNK_ROW - 1u) / CHUNK_ROW;
-  if (plain) {
-    const uint32_t c = (cnt + per_chunk * CHUNK_ROW - 1u) / (per_chunk * CHUNK_ROW);
-    return {c, c, 0u, cnt <= (uint32_t)SMALL_CHUNK ? 1u : 0u};  // (a small block is one chunk)
-  }
-  const bool group = 4u * cnt >= 3u * CHUNK_ROW * rows;
-  return {rows, group ? (rows + per_chunk - 1u) / per_chunk : rows, cnt > GROUP_ABOVE ? rows : 0u, 0u};
+  const uint32_t plain = (rows + per_chunk - 1u) / per_chunk;
+  const bool group = 4ull * cnt >= 3ull * CHUNK_ROW * rows;
+  r[CUT_ROWS] = rows;
+  r[CUT_GROUPED] = group ? plain : rows;
+  r[CUT_PLAIN] = plain;
+  r[CUT_SMALL] = cnt <= (uint32_t)SMALL_CHUNK ? 1u : 0u;  // (a small block is one chunk)
+  r[CUT_STEPS] = plain * (((cnt + plain - 1u) / plain + CHUNK_ROW - 1u) / CHUNK_ROW);
+  r[CUT_DENSE] = cnt > GROUP_ABOVE ? rows : 0u;
 }
+
+// Sums over the 256 threads of a workgroup, to every thread.
+template <int K>
+__device__ __forceinline__ void block_sums(uint32_t (&v)[K], uint32_t (*sh)[K]) {
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v[i] += __shfl_xor(v[i], o);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][i] = v[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < K; ++i) v[i] = (sh[0][i] + sh[1][i]) + (sh[2][i] + sh[3][i]);
+}
+
+constexpr int PART_WORDS = 8;  // per tile: its BlockCuts
 
 __global__ __launch_bounds__(SCAN_THREADS) void block_tile_kernel(const uint32_t* __restrict__ bocc,
                                                                   const uint32_t* __restrict__ bstart,
                                                                   const uint32_t* __restrict__ bend,
                                                                   int64_t nblocks, uint32_t per_chunk,
-                                                                  uint4* __restrict__ part, int plain) {
-  __shared__ uint32_t sh[SCAN_THREADS];
-  const int64_t b = (int64_t)blockIdx.x * SCAN_THREADS + threadIdx.x;
-  const BlockRows r = b < nblocks ? block_rows(bocc, bstart, bend, b, per_chunk, plain) : BlockRows{0u, 0u, 0u, 0u};
-  uint32_t rows, chunks, dense, small;
-  block_exclusive_scan(r.rows, sh, &rows);
-  block_exclusive_scan(r.chunks, sh, &chunks);
-  block_exclusive_scan(r.dense, sh, &dense);
-  block_exclusive_scan(r.small, sh, &small);
-  if (threadIdx.x == 0) part[blockIdx.x] = make_uint4(rows, chunks, dense, small);
+                                                                  uint32_t* __restrict__ part) {
+  __shared__ uint32_t sh[SCAN_THREADS / 64][CUTS];
+  BlockCuts r;
+  block_cuts(bocc, bstart, bend, (int64_t)blockIdx.x * SCAN_THREADS + threadIdx.x, nblocks, per_chunk, r);
+  block_sums<CUTS>(r, sh);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int i = 0; i < CUTS; ++i) part[(size_t)blockIdx.x * PART_WORDS + i] = r[i];
+  }
 }
 
 __global__ __launch_bounds__(SCAN_THREADS) void block_chunks_kernel(
     const uint32_t* __restrict__ bocc, const uint32_t* __restrict__ bstart, const uint32_t* __restrict__ bend,
-    const int* __restrict__ block_scene, int64_t nblocks, uint32_t per_chunk, const uint4* __restrict__ part,
+    const int* __restrict__ block_scene, int64_t nblocks, uint32_t per_chunk, const uint32_t* __restrict__ part,
     int4* __restrict__ chunks, uint32_t* __restrict__ bfirst, uint32_t* __restrict__ bcount,
     uint32_t* __restrict__ nchunks, int plain, int4* __restrict__ split, uint32_t split_cap) {
-  __shared__ uint32_t sh[SCAN_THREADS];
-  uint32_t rows_before = 0, chunks_before = 0, small_before = 0, rows = 0, dense = 0, small = 0;
+  __shared__ uint32_t sh[SCAN_THREADS], sums_s[SCAN_THREADS / 64][2 * CUTS];
+  uint32_t sums[2 * CUTS];  // over all tiles, over those before this one
+#pragma unroll
+  for (int i = 0; i < 2 * CUTS; ++i) sums[i] = 0u;
   for (uint32_t q = threadIdx.x; q < gridDim.x; q += SCAN_THREADS) {
-    const uint4 v = part[q];
-    rows += v.x;
-    dense += v.z;
-    small += v.w;
-    if (q < blockIdx.x) {
-      rows_before += v.x;
-      chunks_before += v.y;
-      small_before += v.w;
+    const uint4 lo = reinterpret_cast<const uint4*>(part)[2 * q], hi = reinterpret_cast<const uint4*>(part)[2 * q + 1];
+    const BlockCuts v = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y};
+#pragma unroll
+    for (int i = 0; i < CUTS; ++i) {
+      sums[i] += v[i];
+      sums[CUTS + i] += q < blockIdx.x ? v[i] : 0u;
     }
   }
-  uint32_t rows_all, dense_all, before;
-  block_exclusive_scan(rows, sh, &rows_all);
-  block_exclusive_scan(dense, sh, &dense_all);
-  // the same in every workgroup
-  const bool single = !plain && (rows_all <= FEW_ROWS || 2u * dense_all < rows_all);
-  block_exclusive_scan(single ? rows_before : chunks_before, sh, &before);
+  block_sums<2 * CUTS>(sums, sums_s);
   const int64_t b = (int64_t)blockIdx.x * SCAN_THREADS + threadIdx.x;
-  BlockRows r = b < nblocks ? block_rows(bocc, bstart, bend, b, per_chunk, plain) : BlockRows{0u, 0u, 0u, 0u};
-  const uint32_t c = single ? r.rows : r.chunks;
+  BlockCuts r;
+  block_cuts(bocc, bstart, bend, b, nblocks, per_chunk, r);
+  // the cut (the same in every workgroup)
+  const uint32_t R = sums[CUT_ROWS];
+  const bool dense = 2u * sums[CUT_DENSE] >= R, few = R <= FEW_ROUNDS;
+  const bool single = !plain && (R <= FEW_ROWS || (!dense && (R <= ONE_ROUND || (few && 10ull * sums[CUT_STEPS] >= 11ull * R))));
+  const bool grouped = !plain && !single && dense && few;
+  const int cut = single ? CUT_ROWS : (grouped ? CUT_GROUPED : CUT_PLAIN);
+  const uint32_t c = single ? r[CUT_ROWS] : (grouped ? r[CUT_GROUPED] : r[CUT_PLAIN]);
+  const uint32_t before = cut == CUT_ROWS ? sums[CUTS + CUT_ROWS]
+                                          : (cut == CUT_GROUPED ? sums[CUTS + CUT_GROUPED] : sums[CUTS + CUT_PLAIN]);
+  const uint32_t pieces = single || grouped ? r[CUT_ROWS] : r[CUT_PLAIN];  // equal parts that chunks are made of
   uint32_t tot;
   const uint32_t run = block_exclusive_scan(c, sh, &tot) + before;
-  uint32_t small_run = 0;
-  if (split) {
-    uint32_t small_all, first;
-    block_exclusive_scan(small, sh, &small_all);
-    if (small_all < APART_FROM) r.small = small_before = 0u;
-    block_exclusive_scan(small_before, sh, &first);
-    small_run = block_exclusive_scan(r.small, sh, &tot) + first;
+  uint32_t small = 0, small_run = 0;
+  if (split) {  // (plain)
+    const bool apart = sums[CUT_SMALL] >= APART_FROM;
+    small = apart ? r[CUT_SMALL] : 0u;
+    small_run = block_exclusive_scan(small, sh, &tot) + (apart ? sums[CUTS + CUT_SMALL] : 0u);
   }
   if (b < nblocks) {
     bfirst[b] = run;
@@ -330,19 +355,19 @@ __global__ __launch_bounds__(SCAN_THREADS) void block_chunks_kernel(
       const int sc = block_scene[b];
       uint32_t s0 = 0, s1;
       for (uint32_t j = 0; j < c; ++j, s0 = s1) {
-        // its rows end at r1 (64 bits: rows^2 leaves 32 from 2^24 particles in one block on)
-        const uint32_t r1 = (uint32_t)((uint64_t)r.rows * (j + 1u) / c);
-        s1 = (uint32_t)((uint64_t)cnt * r1 / r.rows);
+        // its pieces end at r1 (64 bits: rows^2 leaves 32 from 2^24 particles in one block on)
+        const uint32_t r1 = (uint32_t)((uint64_t)pieces * (j + 1u) / c);
+        s1 = (uint32_t)((uint64_t)cnt * r1 / pieces);
         chunks[run + j] = make_int4((int)(p0 + s0), (int)(s1 - s0), (int)b, sc);
         if (split)
-          split[r.small ? split_cap - 1u - small_run : run + j - small_run] =
+          split[small ? split_cap - 1u - small_run : run + j - small_run] =
               make_int4((int)(p0 + s0), (int)((s1 - s0) | ((uint32_t)sc << SPLIT_COUNT_BITS)), (int)b, (int)(run + j));
       }
     }
   }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == SCAN_THREADS - 1) {
     nchunks[0] = run + c;
-    nchunks[1] = small_run + r.small;
+    nchunks[1] = small_run + small;
   }
 }
 
@@ -448,7 +473,7 @@ size_t radix_workspace_bytes(int64_t n) {
   return sizeof(uint32_t) * (2 * (size_t)(n > 0 ? n : 0) + 2 * radix_hist_words(n) + RS_MAX_BINS);
 }
 
-size_t chunk_list_part_words(int64_t nblocks) { return 4 * ((size_t)cdiv(nblocks, SCAN_THREADS) + 1); }
+size_t chunk_list_part_words(int64_t nblocks) { return PART_WORDS * ((size_t)cdiv(nblocks, SCAN_THREADS) + 1); }
 
 void chunk_list(const uint32_t* bocc, const uint32_t* bstart, const uint32_t* bend, const int* block_scene,
                 int64_t nblocks, int chunk, uint32_t* part, int4* chunks, uint32_t* bfirst, uint32_t* bcount,
@@ -456,11 +481,11 @@ void chunk_list(const uint32_t* bocc, const uint32_t* bstart, const uint32_t* be
   if (nblocks <= 0) return;
   const unsigned tiles = (unsigned)cdiv(nblocks, SCAN_THREADS);
   const uint32_t per_chunk = (uint32_t)chunk / CHUNK_ROW;
-  uint4* part4 = reinterpret_cast<uint4*>(part);
   hipLaunchKernelGGL(block_tile_kernel, dim3(tiles), dim3(SCAN_THREADS), 0, st, bocc, bstart, bend, nblocks,
-                     per_chunk, part4, plain ? 1 : 0);
+                     per_chunk, part);
   hipLaunchKernelGGL(block_chunks_kernel, dim3(tiles), dim3(SCAN_THREADS), 0, st, bocc, bstart, bend,
-                     block_scene, nblocks, per_chunk, part4, chunks, bfirst, bcount, nchunks, plain ? 1 : 0, split, (uint32_t)split_cap);
+                     block_scene, nblocks, per_chunk, part, chunks, bfirst, bcount, nchunks, plain ? 1 : 0, split,
+                     (uint32_t)split_cap);
 }
 
 uint32_t* radix_first_hist(void* ws, int64_t n) { return (uint32_t*)ws + 2 * n; }
