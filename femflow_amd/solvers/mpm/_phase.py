@@ -120,9 +120,8 @@ class OutOfGrid:
     """Counts the particles whose stencil leaves the grid, ahead of a phase's
     own launches, so that the host can wait for the count while they run."""
 
-    def __init__(self, sp, prm):
+    def __init__(self, sp, prm, p):
         count = torch.zeros(1, dtype=torch.int64, device=sp.device)
-        p = sp.struct()
         _lib.check(_lib.load().mpm_count_oob(stream_ptr(sp.device), ct.byref(prm), ct.byref(p), count.data_ptr()),
                    "count_oob")
         self.host = torch.empty(1, dtype=torch.int64, pin_memory=True)
@@ -142,12 +141,12 @@ def _workspace(sp, prm):
     return work, None if work is None else work.data_ptr(), nbytes.value
 
 
-def launch_p2g(sp, prm, kind_override, hardening, grid_velocity, grid_mass, materials=None):
+def launch_p2g(sp, prm, p, kind_override, hardening, grid_velocity, grid_mass, materials=None):
+    """p: sp.struct(), built once for the launches of a call (2 us of host time)."""
     L = _lib.load()
     gv = Staged(grid_velocity, sp.dtype, sp.device)
     gm = Staged(grid_mass, sp.dtype, sp.device)
     mats, nmat = materials_array(materials)
-    p = sp.struct()
     work, ptr, nbytes = _workspace(sp, prm)
     _lib.check(L.mpm_p2g_ws(stream_ptr(sp.device), ct.byref(prm), ct.byref(p), int(kind_override),
                             float(hardening), mats, nmat, gv.ptr, gm.ptr, None, ptr, nbytes), "p2g")
@@ -158,8 +157,9 @@ def launch_p2g(sp, prm, kind_override, hardening, grid_velocity, grid_mass, mate
 def run_p2g(sp, prm, kind_override, hardening, grid_velocity, grid_mass, materials=None):
     """P2G; the number of particles off the grid."""
     _lib.require_gpu()
-    out = OutOfGrid(sp, prm)
-    launch_p2g(sp, prm, kind_override, hardening, grid_velocity, grid_mass, materials)
+    p = sp.struct()
+    out = OutOfGrid(sp, prm, p)
+    launch_p2g(sp, prm, p, kind_override, hardening, grid_velocity, grid_mass, materials)
     return out.wait()
 
 
@@ -210,12 +210,10 @@ def run_collide_planes(points, normals, res, dx, grid_velocity, quirks):
     gv.commit()
 
 
-def launch_g2p(sp, prm, kind_override, grid_velocity, theta_c=THETA_C, theta_s=THETA_S, materials=None):
-    _lib.require_gpu()
+def launch_g2p(sp, prm, p, kind_override, grid_velocity, theta_c=THETA_C, theta_s=THETA_S, materials=None):
     L = _lib.load()
     gv = Staged(grid_velocity, sp.dtype, sp.device, writable=False)
     mats, nmat = materials_array(materials)
-    p = sp.struct()
     _lib.check(L.mpm_g2p(stream_ptr(sp.device), ct.byref(prm), ct.byref(p), int(kind_override),
                          float(theta_c), float(theta_s), mats, nmat, gv.ptr, None), "g2p")
 
@@ -223,6 +221,7 @@ def launch_g2p(sp, prm, kind_override, grid_velocity, theta_c=THETA_C, theta_s=T
 def run_g2p(sp, prm, kind_override, grid_velocity, theta_c=THETA_C, theta_s=THETA_S, materials=None):
     """G2P; the number of particles off the grid."""
     _lib.require_gpu()
-    out = OutOfGrid(sp, prm)
-    launch_g2p(sp, prm, kind_override, grid_velocity, theta_c, theta_s, materials)
+    p = sp.struct()
+    out = OutOfGrid(sp, prm, p)
+    launch_g2p(sp, prm, p, kind_override, grid_velocity, theta_c, theta_s, materials)
     return out.wait()

@@ -66,13 +66,14 @@ def solve_mls_mpm_3d(res: int, inv_dx: float, hardening: float, dx: float, dt: f
         prm = _phase.make_params(3, res, inv_dx, dx, dt, volume, gravity, boundary=bc, bound=int(bound),
                                  quirks=q)
         _lib.require_gpu()
-        out = _phase.OutOfGrid(sp, prm)  # P2G and G2P find the particles at the same places
-        _phase.launch_p2g(sp, prm, _lib.MPM_ELASTIC, hardening, gv, gm)
+        p = sp.struct()
+        out = _phase.OutOfGrid(sp, prm, p)  # P2G and G2P find the particles at the same places
+        _phase.launch_p2g(sp, prm, p, _lib.MPM_ELASTIC, hardening, gv, gm)
         _phase.run_grid_op(prm, gv, gm)
         n_oob = out.wait()
         if n_oob:
             raise RuntimeError(f"{n_oob} particle(s) outside the grid")
-        _phase.launch_g2p(sp, prm, _lib.MPM_ELASTIC, gv)
+        _phase.launch_g2p(sp, prm, p, _lib.MPM_ELASTIC, gv)
         sp.commit()
         return
     if abs(inv_dx * dx - 1.0) > 1e-9 or abs(inv_dx - res) > 1e-9 * res:
